@@ -889,11 +889,10 @@ int giem2g_unet_forward_dev(void* net, const float* x_dev, float* y_dev, int B, 
   return guard([&] {
     UNet* n = NET(net);
     unet_reserve(*n, B, nx, ny, nz, keep_for_backward != 0);
-    unet_load_input(*n, x_dev, n->stream);
-    unet_forward(*n, n->stream);
-    if (y_dev)
-      G2G_HIP(hipMemcpyAsync(y_dev, n->out, sizeof(float) * 6 * (size_t)B * nx * ny * nz,
-                             hipMemcpyDeviceToDevice, n->stream));
+    // without a backward to follow the first layer reads x itself (vector loads: 16-byte aligned)
+    const bool direct = !n->training && ((uintptr_t)x_dev & 15) == 0;
+    if (!direct) unet_load_input(*n, x_dev, n->stream);
+    unet_forward(*n, n->stream, direct ? x_dev : nullptr, y_dev);
     G2G_HIP(hipStreamSynchronize(n->stream));
   });
 }

@@ -11,8 +11,8 @@
 //   out[co][p] = bias[co] + sum_k W[co][k] X[k][p],  k = tap*Cin + ci,
 // A = weights (16 output channels x 32 k), B = input (32 k x 16 voxels).
 // Lane l of a wave holds A row l%16 / B column l%16 and the 8 consecutive
-// k = 8*(l/16) .. 8*(l/16)+7, which is one 16-byte load of 8 channels of one
-// tap (Cin is a multiple of 8); the FP32 result of lane l is rows
+// k = 8*(l/16) .. 8*(l/16)+7, which is one 16-byte read of 8 channels of one
+// tap (Cin is a multiple of 8) from the tile's copy in LDS; the FP32 result of lane l is rows
 // 4*(l/16) .. 4*(l/16)+3 of column l%16 -- four consecutive output channels
 // of one voxel, stored as one 8-byte bf16 write.  The data gradient is the
 // same kernel run on the transposed, tap-flipped weights; the weight
@@ -57,103 +57,261 @@ struct ConvArgs {
   int ldy;
   int64_t ybstride;
   int nx, ny, nz;
+  // input layer: the caller's FP32 volume instead of s1.p (or null)
+  const float* xf;
+  // the 1x1 output layer applied to this layer's result (16 channels): its
+  // weight fragment, bias and FP32 result of cout2 channels (or null)
+  const bf16* w2;
+  const float* bias2;
+  float* y2;
+  int cout2;
 };
 
-// One wave: 16 output channels x 64 voxels (4 MFMA columns); 4 waves per block.
-__global__ __launch_bounds__(UB) void k_conv(ConvArgs a) {
+// bias, ReLU and store of four consecutive output channels of one voxel
+__device__ inline void conv_store(const ConvArgs& a, f32x4 c, int co0, int64_t p, int bat) {
+  if (co0 >= a.cout) return;
+  float o[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    o[q] = c[q] + ((a.bias && co0 + q < a.cout) ? a.bias[co0 + q] : 0.f);
+    if (a.relu) o[q] = fmaxf(o[q], 0.f);
+  }
+  if (a.ybf) {
+    const bf16x4 b = {(bf16)o[0], (bf16)o[1], (bf16)o[2], (bf16)o[3]};
+    *reinterpret_cast<bf16x4*>(a.ybf + bat * a.ybstride + p * a.ldy + co0) = b;
+  } else {
+    float* y = a.yf + bat * a.ybstride + p * a.ldy + co0;
+    if ((a.ldy & 3) == 0 && co0 + 3 < a.cout) {
+      *reinterpret_cast<f32x4*>(y) = f32x4{o[0], o[1], o[2], o[3]};
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (co0 + q < a.cout) y[q] = o[q];
+    }
+  }
+}
+
+// A convolution tile of (1 << lx, 1 << ly, 1 << lz) voxels: tile counts, the
+// voxels with the rim, the plane stride of the LDS copy, and multipliers for
+// division by the rim's row and plane sizes (exact for v < 2048); the same
+// for an upsampled source's rim at half resolution.  Matrix column group
+// n = sum of s[k] over the set bits k of (wave, g): the groups of one wave
+// share the parities of their voxels' coordinates.
+struct ConvBox {
+  int hx, hy, hvox, hv;
+  unsigned mx, mxy;
+};
+struct ConvTile {
+  int lx, ly, lz, ntx, nty, nt;
+  ConvBox f, h;
+  int sg[2], sw[2];
+};
+
+// 1x1 convolutions (27-tap ones: k_conv3 below).  One wave: 16 output
+// channels x 64 voxels (4 MFMA columns), one k-step; HBM bound.
+__global__ __launch_bounds__(UB) void k_conv1x1(ConvArgs a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, kq = lane >> 4;
   const int nvox = a.nx * a.ny * a.nz;
   const int pbase = (blockIdx.x * 4 + wave) * 64;
   const int cb = blockIdx.y, bat = blockIdx.z;
   const bf16* x1 = a.s1.p + bat * a.s1.bstride;
-  const bf16* x2 = a.s2.p ? a.s2.p + bat * a.s2.bstride : a.s1.p;
-  int vx0, vy0, vz0, vx1, vy1, vz1, vx2, vy2, vz2, vx3, vy3, vz3;
-#define G2G_VXYZ(s)                                        \
-  {                                                        \
-    int p_ = pbase + (s) * 16 + col;                       \
-    if (p_ >= nvox) p_ = -1;                               \
-    int q_ = p_ < 0 ? 0 : p_;                              \
-    vx##s = q_ % a.nx;                                     \
-    q_ /= a.nx;                                            \
-    vy##s = q_ % a.ny;                                     \
-    vz##s = p_ < 0 ? -1000 : q_ / a.ny;                    \
+  const bf16x8 af = *reinterpret_cast<const bf16x8*>(a.w + ((int64_t)cb * 64 + lane) * 8);
+  const int k0 = kq * 8;
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const int p = pbase + s * 16 + col;
+    bf16x8 bfr = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (k0 < a.cin && p < nvox) bfr = *reinterpret_cast<const bf16x8*>(x1 + (int64_t)p * a.cin + k0);
+    f32x4 c = {0, 0, 0, 0};
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr, c, 0, 0, 0);
+    if (p < nvox) conv_store(a, c, cb * 16 + kq * 4, (int64_t)p, bat);
   }
-  G2G_VXYZ(0) G2G_VXYZ(1) G2G_VXYZ(2) G2G_VXYZ(3)
-#undef G2G_VXYZ
-  f32x4 c0 = {0, 0, 0, 0}, c1 = c0, c2 = c0, c3 = c0;
-  const bf16* wrow = a.w + (int64_t)(cb * 16 + col) * a.kp;
-  const int nks = a.kp / 32;
-  const int nxh = a.nx >> 1, nyh = a.ny >> 1;
-  for (int ks = 0; ks < nks; ks++) {
-    const int k0 = ks * 32 + kq * 8;
-    const bf16x8 af = *reinterpret_cast<const bf16x8*>(wrow + k0);
-    const int tap = k0 / a.cin;
-    const int ci = k0 - tap * a.cin;
-    const bool tv = tap < a.ntap;
-    int dx = 0, dy = 0, dz = 0;
-    if (a.ntap == 27) {
-      dz = tap / 9 - 1;
-      dy = (tap / 3) % 3 - 1;
-      dx = tap % 3 - 1;
+}
+
+// 3x3x3 convolution, CIN input channels, CT x 16 output channels, a tile of
+// 64 G voxels (4 waves of 16 G voxels x all output channels).
+// The tile with its one-voxel rim is copied to LDS once, zero outside the
+// volume, concatenated and upsampled on the way, in planes of 8 channels
+// ([chunk][voxel], 16 bytes each): the 16 lanes of a matrix column then read
+// 16 neighbouring voxels without bank conflicts, and a tap is an offset added
+// to the lane's own voxel (a 4-byte table entry per k-step and lane quarter)
+// instead of the three bounds checks, the address and the global gather that
+// each fragment took when every wave read its input from memory: that kernel
+// ran at 0.10-0.17 of the matrix rate with the vector unit busy on addresses.
+// Every fragment read from LDS feeds the CT output tiles.  LDS bandwidth
+// bounds it (16 bytes a lane per CT products).  Measured at 256x256x32, all
+// layers of one forward pass: 1508 -> 555 us (251 GFLOP, 0.17 -> 0.45
+// PFLOP/s; 48 -> 16 channels 0.60 PFLOP/s); the whole pass 1541 -> 595 us
+// with the input conversion and the 1x1 output layer done on the way.  The sums run over k in the same order and instruction
+// as before, so the results are the same bit for bit.
+// Weights: fragment order [co tile][k-step][lane][8], one contiguous 1 KB
+// load per k-step and tile.
+constexpr int conv_g(int cin) { return cin >= 64 ? 2 : 4; }
+
+// An upsampled source (its first UPC channels) is kept in LDS at half
+// resolution: a quarter to an eighth of the bytes, so that three to five
+// blocks share a CU instead of one or two (48 channels 270 -> 143 us, 96
+// channels 173 -> 81 us).  Its offset of a tap depends on
+// the parity of the voxel's coordinates (eight table entries per k-step).
+// FP32 input rounded to bf16 on the way
+__device__ inline bf16x8 to_bf16x8(const float* x) {
+  const f32x4 a = *reinterpret_cast<const f32x4*>(x), b = *reinterpret_cast<const f32x4*>(x + 4);
+  return bf16x8{(bf16)a[0], (bf16)a[1], (bf16)a[2], (bf16)a[3], (bf16)b[0], (bf16)b[1], (bf16)b[2], (bf16)b[3]};
+}
+
+// Copies the tile's box at (X0, Y0, Z0) of a source to planes of 8 channels, zero outside the volume
+template <int NCH, typename T>
+__device__ inline void conv_stage(bf16x8* xs, const ConvBox& b, const T* x, int X0, int Y0, int Z0, int nx, int ny,
+                                  int nz, int tid) {
+  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 4
+  for (int e = tid; e < b.hvox * NCH; e += UB) {
+    const int v = e / NCH, ch = e - v * NCH;
+    const int vz = (int)(((unsigned)v * b.mxy) >> 20), vr = v - vz * b.hx * b.hy;
+    const int vy = (int)(((unsigned)vr * b.mx) >> 20), vx = vr - vy * b.hx;
+    const int X = X0 + vx, Y = Y0 + vy, Z = Z0 + vz;
+    const bool in = X >= 0 && X < nx && Y >= 0 && Y < ny && Z >= 0 && Z < nz;
+    // the load is unconditional, from a clamped voxel, so that several are in flight
+    const int Xc = min(max(X, 0), nx - 1), Yc = min(max(Y, 0), ny - 1), Zc = min(max(Z, 0), nz - 1);
+    const T* xp = x + (((int64_t)Zc * ny + Yc) * nx + Xc) * (NCH * 8) + ch * 8;
+    bf16x8 val;
+    if constexpr (sizeof(T) == 4) val = to_bf16x8(xp);
+    else val = *reinterpret_cast<const bf16x8*>(xp);
+    xs[ch * b.hv + v] = in ? val : zero;
+  }
+}
+
+template <int CIN, int CT, int UPC>
+__global__ __launch_bounds__(UB) void k_conv3(ConvArgs a, ConvTile t) {
+  constexpr int G = conv_g(CIN), NKS = (27 * CIN + 31) / 32, NU = UPC / 8, NF = CIN / 8 - NU;
+  constexpr int NPAR = UPC ? 8 : 1;
+  constexpr bool TAIL = (27 * CIN) % 32 != 0;
+  extern __shared__ unsigned char conv_sm[];
+  bf16x8* xs = reinterpret_cast<bf16x8*>(conv_sm);  // half-resolution planes, then the full ones
+  const int full0 = NU * t.h.hv;
+  // offset of the k-step's chunk and tap for lane quarter kq and voxel
+  // parity; bit 15: of an upsampled source; 0xffff: past the last tap
+  unsigned short* tab = reinterpret_cast<unsigned short*>(conv_sm + sizeof(bf16x8) * (full0 + NF * t.f.hv));
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 15, kq = lane >> 4;
+  // consecutive workgroups go round-robin to the eight XCDs: each XCD gets a
+  // run of neighbouring tiles, whose rims meet in its L2
+  int tile;
+  {
+    const int n = gridDim.x, q = n >> 3, r = n & 7, x = blockIdx.x & 7, i = blockIdx.x >> 3;
+    tile = x * q + (x < r ? x : r) + i;
+  }
+  const int bat = tile / t.nt;
+  tile -= bat * t.nt;
+  const int tz0 = tile / (t.ntx * t.nty), ty0 = (tile / t.ntx) % t.nty, tx0 = tile % t.ntx;
+  const int x0 = tx0 << t.lx, y0 = ty0 << t.ly, z0 = tz0 << t.lz;
+  for (int i = tid; i < NKS * 4 * NPAR; i += UB) {
+    const int par = i % NPAR, e = i / NPAR, k0 = (e >> 2) * 32 + (e & 3) * 8, tap = k0 / CIN, ch = (k0 - tap * CIN) >> 3;
+    const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
+    int off = 0xffff;
+    if (tap < 27) {
+      if (ch < NU)  // voxel 2a + p with tap d reads half voxel a + (p + d + 1) / 2 of the rim
+        off = 0x8000 | (ch * t.h.hv + ((((par >> 2) + dz + 1) >> 1) * t.h.hy + ((((par >> 1) & 1) + dy + 1) >> 1)) * t.h.hx +
+                        (((par & 1) + dx + 1) >> 1));
+      else
+        off = full0 + (ch - NU) * t.f.hv + (dz * t.f.hy + dy) * t.f.hx + dx;
     }
-    const bool first = ci < a.s1.C;
-    const bf16* sp = x1;
-    int C = a.s1.C, cc = ci, up = a.s1.up;
-    if (!first) {
-      sp = x2;
-      C = a.s2.C;
-      cc = ci - a.s1.C;
-      up = a.s2.up;
+    tab[i] = (unsigned short)off;
+  }
+  if constexpr (UPC > 0) {
+    conv_stage<NU>(xs, t.h, a.s1.p + bat * a.s1.bstride, (x0 >> 1) - 1, (y0 >> 1) - 1, (z0 >> 1) - 1, a.nx >> 1,
+                   a.ny >> 1, a.nz >> 1, tid);
+    conv_stage<NF>(xs + full0, t.f, a.s2.p + bat * a.s2.bstride, x0 - 1, y0 - 1, z0 - 1, a.nx, a.ny, a.nz, tid);
+  } else {
+    if (CIN == 8 && a.xf)
+      conv_stage<NF>(xs, t.f, a.xf + bat * a.s1.bstride, x0 - 1, y0 - 1, z0 - 1, a.nx, a.ny, a.nz, tid);
+    else
+      conv_stage<NF>(xs, t.f, a.s1.p + bat * a.s1.bstride, x0 - 1, y0 - 1, z0 - 1, a.nx, a.ny, a.nz, tid);
+  }
+  __syncthreads();
+  int base[G], baseh[G], vx[G], vy[G], vz[G];
+#pragma unroll
+  for (int g = 0; g < G; g++) {
+    const int n = (g & 1) * t.sg[0] + (g >> 1) * t.sg[1] + (wave & 1) * t.sw[0] + (wave >> 1) * t.sw[1];
+    const int v = n * 16 + col;
+    vx[g] = v & ((1 << t.lx) - 1);
+    vy[g] = (v >> t.lx) & ((1 << t.ly) - 1);
+    vz[g] = v >> (t.lx + t.ly);
+    base[g] = (vz[g] * t.f.hy + vy[g]) * t.f.hx + vx[g];
+    baseh[g] = ((vz[g] >> 1) * t.h.hy + (vy[g] >> 1)) * t.h.hx + (vx[g] >> 1);
+  }
+  const int par = UPC ? (vx[0] & 1) + 2 * (vy[0] & 1) + 4 * (vz[0] & 1) : 0;  // the same for every g
+  f32x4 acc[CT][G];
+#pragma unroll
+  for (int c = 0; c < CT; c++)
+#pragma unroll
+    for (int g = 0; g < G; g++) acc[c][g] = f32x4{0, 0, 0, 0};
+  const bf16x8* wf = reinterpret_cast<const bf16x8*>(a.w) + lane;
+  constexpr int NFULL = TAIL ? NKS - 1 : NKS;
+#pragma unroll 3
+  for (int ks = 0; ks < NFULL; ks++) {
+    const int off = tab[(ks * 4 + kq) * NPAR + par], o = off & 0x7fff;
+    const bool up = UPC > 0 && (off & 0x8000);
+    bf16x8 af[CT];
+#pragma unroll
+    for (int c = 0; c < CT; c++) af[c] = wf[(c * NKS + ks) * 64];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      const bf16x8 b = xs[(up ? baseh[g] : base[g]) + o];
+#pragma unroll
+      for (int c = 0; c < CT; c++) acc[c][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[c], b, acc[c][g], 0, 0, 0);
     }
-#define G2G_BFRAG(s)                                                                    \
-  {                                                                                     \
-    bf16x8 bfr = {0, 0, 0, 0, 0, 0, 0, 0};                                              \
-    const int X = vx##s + dx, Y = vy##s + dy, Z = vz##s + dz;                           \
-    if (tv && X >= 0 && X < a.nx && Y >= 0 && Y < a.ny && Z >= 0 && Z < a.nz) {         \
-      int64_t q;                                                                        \
-      if (up) q = ((int64_t)(Z >> 1) * nyh + (Y >> 1)) * nxh + (X >> 1);               \
-      else q = ((int64_t)Z * a.ny + Y) * a.nx + X;                                      \
-      bfr = *reinterpret_cast<const bf16x8*>(sp + q * C + cc);                          \
-    }                                                                                   \
-    c##s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr, c##s, 0, 0, 0);             \
   }
-    G2G_BFRAG(0) G2G_BFRAG(1) G2G_BFRAG(2) G2G_BFRAG(3)
-#undef G2G_BFRAG
+  if constexpr (TAIL) {  // k past the 27th tap: zero input
+    const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int off = tab[(NFULL * 4 + kq) * NPAR + par];
+    const bool past = off == 0xffff, up = UPC > 0 && !past && (off & 0x8000);
+    const int o = past ? 0 : off & 0x7fff;
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      const bf16x8 v = xs[(up ? baseh[g] : base[g]) + o];
+      const bf16x8 b = past ? zero : v;
+#pragma unroll
+      for (int c = 0; c < CT; c++)
+        acc[c][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[(c * NKS + NFULL) * 64], b, acc[c][g], 0, 0, 0);
+    }
   }
-  const int co0 = cb * 16 + kq * 4;
-  float b0 = 0, b1 = 0, b2 = 0, b3 = 0;
-  if (a.bias) {
-    if (co0 < a.cout) b0 = a.bias[co0];
-    if (co0 + 1 < a.cout) b1 = a.bias[co0 + 1];
-    if (co0 + 2 < a.cout) b2 = a.bias[co0 + 2];
-    if (co0 + 3 < a.cout) b3 = a.bias[co0 + 3];
+#pragma unroll
+  for (int g = 0; g < G; g++) {
+    const int X = x0 + vx[g], Y = y0 + vy[g], Z = z0 + vz[g];
+    const bool in = X < a.nx && Y < a.ny && Z < a.nz;
+    const int64_t p = ((int64_t)Z * a.ny + Y) * a.nx + X;
+    if (in && (a.ybf || a.yf)) {
+#pragma unroll
+      for (int c = 0; c < CT; c++) conv_store(a, acc[c][g], c * 16 + kq * 4, p, bat);
+    }
+    if constexpr (CIN == 16 && CT == 1) {
+      if (a.w2) {
+        // the 1x1 layer's operand: lane quarter kq < 2 takes channels 8 kq ..
+        // 8 kq + 7 of its voxel from quarters 2 kq and 2 kq + 1
+        bf16x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const float v = acc[0][g][q] + (a.bias ? a.bias[kq * 4 + q] : 0.f);
+          o[q] = (bf16)(a.relu ? fmaxf(v, 0.f) : v);
+        }
+        const int2 w = __builtin_bit_cast(int2, o);
+        const int l0 = (col + 32 * kq) & 63, l1 = (l0 + 16) & 63;
+        const int4 u = {__shfl(w.x, l0), __shfl(w.y, l0), __shfl(w.x, l1), __shfl(w.y, l1)};
+        const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+        const bf16x8 b = kq < 2 ? __builtin_bit_cast(bf16x8, u) : zero;
+        f32x4 r = {0, 0, 0, 0};
+        r = __builtin_amdgcn_mfma_f32_16x16x32_bf16(reinterpret_cast<const bf16x8*>(a.w2)[lane], b, r, 0, 0, 0);
+        if (in) {
+          float* y = a.y2 + ((int64_t)bat * a.nx * a.ny * a.nz + p) * a.cout2;
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            if (kq * 4 + q < a.cout2) y[kq * 4 + q] = r[q] + a.bias2[kq * 4 + q];
+        }
+      }
+    }
   }
-#define G2G_EPI(s)                                                                   \
-  {                                                                                  \
-    const int p = pbase + (s) * 16 + col;                                            \
-    if (p < nvox && co0 < a.cout) {                                                  \
-      float o0 = c##s[0] + b0, o1 = c##s[1] + b1, o2 = c##s[2] + b2, o3 = c##s[3] + b3; \
-      if (a.relu) {                                                                  \
-        o0 = fmaxf(o0, 0.f);                                                         \
-        o1 = fmaxf(o1, 0.f);                                                         \
-        o2 = fmaxf(o2, 0.f);                                                         \
-        o3 = fmaxf(o3, 0.f);                                                         \
-      }                                                                              \
-      if (a.ybf) {                                                                   \
-        bf16x4 o = {(bf16)o0, (bf16)o1, (bf16)o2, (bf16)o3};                         \
-        *reinterpret_cast<bf16x4*>(a.ybf + bat * a.ybstride + (int64_t)p * a.ldy + co0) = o; \
-      } else {                                                                       \
-        float* y = a.yf + bat * a.ybstride + (int64_t)p * a.ldy + co0;               \
-        y[0] = o0;                                                                   \
-        if (co0 + 1 < a.cout) y[1] = o1;                                             \
-        if (co0 + 2 < a.cout) y[2] = o2;                                             \
-        if (co0 + 3 < a.cout) y[3] = o3;                                             \
-      }                                                                              \
-    }                                                                                \
-  }
-  G2G_EPI(0) G2G_EPI(1) G2G_EPI(2) G2G_EPI(3)
-#undef G2G_EPI
 }
 
 // Weight gradient dW[co][t][ci] += sum_p dZ[p][co] X[p+off(t)][ci] and
@@ -254,20 +412,30 @@ __global__ __launch_bounds__(UB) void k_dw(DwArgs a) {
 }
 
 // forward weights w[co][tap*cin+ci] and transposed weights
-// wt[ci][tap'*coutT+co] = W[co][ntap-1-tap'][ci] (bf16, zero padded)
+// wt[ci][tap'*coutT+co] = W[co][ntap-1-tap'][ci] (bf16, zero padded), both in
+// fragment order: element j of lane l in k-step s of output tile c, at
+// ((c*nks + s)*64 + l)*8 + j, is row 16c + l%16, column 32s + 8(l/16) + j
+__device__ inline void frag_rc(int64_t i, int kp, int* row, int* k) {
+  const int j = (int)(i & 7), l = (int)(i >> 3) & 63, nks = kp / 32;
+  const int cs = (int)(i >> 9), s = cs % nks, c = cs / nks;
+  *row = c * 16 + (l & 15);
+  *k = s * 32 + (l >> 4) * 8 + j;
+}
 __global__ void k_wprep(const float* __restrict__ W, int cout, int cin, int ntap, bf16* w, int coutP,
                         int kp, bf16* wt, int cinP, int coutT, int kpT) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t n1 = (int64_t)coutP * kp, n2 = (int64_t)cinP * kpT;
   if (i < n1) {
-    const int co = (int)(i / kp), k = (int)(i % kp);
+    int co, k;
+    frag_rc(i, kp, &co, &k);
     const int t = k / cin, ci = k % cin;
     float v = 0.f;
     if (co < cout && t < ntap) v = W[((int64_t)co * ntap + t) * cin + ci];
     w[i] = (bf16)v;
   } else if (i < n1 + n2) {
     const int64_t j = i - n1;
-    const int ci = (int)(j / kpT), k = (int)(j % kpT);
+    int ci, k;
+    frag_rc(j, kpT, &ci, &k);
     const int tp = k / coutT, co = k % coutT;
     float v = 0.f;
     if (ci < cin && tp < ntap && co < cout) v = W[((int64_t)co * ntap + (ntap - 1 - tp)) * cin + ci];
@@ -357,9 +525,18 @@ __global__ void k_pool_back_add(const float* __restrict__ dc, float* __restrict_
   df[i] += 0.125f * dc[(bat * (nf / 8) + q) * C + c];
 }
 
-__global__ void k_f32_to_bf16(const float* __restrict__ a, bf16* __restrict__ b, int64_t n) {
+// n voxels of 8 channels; VEC: a is 16-byte aligned
+template <bool VEC> __global__ void k_f32_to_bf16(const float* __restrict__ a, bf16* __restrict__ b, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = (bf16)a[i];
+  if (i >= n) return;
+  bf16x8 o;
+  if constexpr (VEC) {
+    o = to_bf16x8(a + i * 8);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; k++) o[k] = (bf16)a[i * 8 + k];
+  }
+  *reinterpret_cast<bf16x8*>(b + i * 8) = o;
 }
 
 // MSE: loss += sum (o-t)^2 / n; dout[p][0..7] = 2 (o-t)/n (channels 6, 7 zero)
@@ -628,11 +805,82 @@ static Src src(const bf16* p, int C, int up, int64_t bstride) {
   return r;
 }
 
+static ConvBox conv_box(int hx, int hy, int hz) {
+  ConvBox b;
+  b.hx = hx;
+  b.hy = hy;
+  b.hvox = hx * hy * hz;
+  b.hv = b.hvox | 1;  // planes start on different banks
+  b.mx = ((1u << 20) + hx - 1) / hx;
+  b.mxy = ((1u << 20) + hx * hy - 1) / (hx * hy);
+  return b;
+}
+
+// Tile of 64 G voxels: 16 long in x, or 8 or 4 where that covers the volume
+// with fewer tiles
+static ConvTile conv_tile(int G, int nx, int ny, int nz) {
+  // log2 sides, then the group strides of bits (g0, g1, w0, w1)
+  static const int shapes[2][3][7] = {{{4, 2, 1, 2, 0, 1, 4}, {3, 2, 2, 1, 0, 2, 4}, {2, 3, 2, 1, 0, 2, 4}},
+                                      {{4, 2, 2, 2, 8, 1, 4}, {3, 3, 2, 1, 2, 4, 8}, {2, 3, 3, 1, 4, 2, 8}}};
+  ConvTile best{};
+  int64_t least = -1;
+  for (auto& sh : shapes[G == 4]) {
+    ConvTile t;
+    t.lx = sh[0];
+    t.ly = sh[1];
+    t.lz = sh[2];
+    auto up = [](int n, int l) { return (n + (1 << l) - 1) >> l; };
+    t.ntx = up(nx, t.lx);
+    t.nty = up(ny, t.ly);
+    t.nt = t.ntx * t.nty * up(nz, t.lz);
+    t.f = conv_box((1 << t.lx) + 2, (1 << t.ly) + 2, (1 << t.lz) + 2);
+    t.h = conv_box((1 << t.lx) / 2 + 2, (1 << t.ly) / 2 + 2, (1 << t.lz) / 2 + 2);
+    t.sg[0] = sh[3];
+    t.sg[1] = sh[4];
+    t.sw[0] = sh[5];
+    t.sw[1] = sh[6];
+    if (least < 0 || t.nt < least) {
+      least = t.nt;
+      best = t;
+    }
+  }
+  return best;
+}
+
+template <int CIN, int CT, int UPC> static void conv3_go(const ConvArgs& a, int B, hipStream_t s) {
+  G2G_CHECK(UPC ? a.s1.up == 1 && a.s1.C == UPC && a.s2.up == 0 && a.s2.C == CIN - UPC : a.s1.up == 0 && a.s2.C == 0, -1,
+            "convolution sources do not match the layer");
+  const ConvTile t = conv_tile(conv_g(CIN), a.nx, a.ny, a.nz);
+  constexpr int NKS = (27 * CIN + 31) / 32, NU = UPC / 8;
+  const size_t lds = (size_t)16 * (NU * t.h.hv + (CIN / 8 - NU) * t.f.hv) + sizeof(short) * NKS * 4 * (UPC ? 8 : 1);
+  if (lds > 65536)
+    G2G_HIP(hipFuncSetAttribute((const void*)k_conv3<CIN, CT, UPC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
+  hipLaunchKernelGGL((k_conv3<CIN, CT, UPC>), dim3((unsigned)(t.nt * B)), dim3(UB), lds, s, a, t);
+}
+
+// the network's widths (forward, and the data gradient's transposed ones)
+static void conv_launch(const ConvArgs& a, int coutP, int B, hipStream_t s) {
+  const int64_t nvox = (int64_t)a.nx * a.ny * a.nz;
+  if (a.ntap == 1) {
+    G2G_CHECK(a.kp == 32 && a.s2.C == 0 && a.s1.up == 0, -1, "1x1 convolution of more than 32 channels");
+    hipLaunchKernelGGL(k_conv1x1, dim3(nblk(nvox, 256), coutP / 16, B), dim3(UB), 0, s, a);
+    return;
+  }
+  const int ct = coutP / 16;
+#define G2G_CONV(ci, c, u) \
+  if (a.cin == ci && ct == c) return conv3_go<ci, c, u>(a, B, s);
+  G2G_CONV(8, 1, 0) G2G_CONV(16, 1, 0) G2G_CONV(16, 2, 0) G2G_CONV(16, 3, 0) G2G_CONV(32, 1, 0) G2G_CONV(32, 2, 0)
+  G2G_CONV(32, 4, 0) G2G_CONV(32, 6, 0) G2G_CONV(48, 1, 32) G2G_CONV(64, 2, 0) G2G_CONV(64, 4, 0) G2G_CONV(96, 2, 64)
+#undef G2G_CONV
+  G2G_CHECK(false, -1, "no convolution kernel for this layer width");
+}
+
 // y = conv(x) at level dims (nx, ny, nz), batch B
-static void conv_fwd(UNet& n, int li, Src s1, Src s2, int nx, int ny, int nz, bf16* ybf, float* yf,
-                     int ldy, hipStream_t s) {
+static void conv_fwd(UNet& n, int li, Src s1, Src s2, int nx, int ny, int nz, bf16* ybf, hipStream_t s,
+                     const float* xf = nullptr, float* y2 = nullptr) {
   const UNetLayer& l = n.L[li];
-  ConvArgs a;
+  ConvArgs a{};
   a.s1 = s1;
   a.s2 = s2;
   a.w = n.w + l.woff;
@@ -643,22 +891,30 @@ static void conv_fwd(UNet& n, int li, Src s1, Src s2, int nx, int ny, int nz, bf
   a.cout = l.cout;
   a.relu = l.relu;
   a.ybf = ybf;
-  a.yf = yf;
-  a.ldy = ldy;
-  a.ybstride = (int64_t)nx * ny * nz * ldy;
+  a.ldy = l.cout;
+  a.ybstride = (int64_t)nx * ny * nz * l.cout;
+  a.xf = xf;
+  if (y2) {
+    const UNetLayer& o = n.L[10];
+    G2G_CHECK(l.cin == 16 && l.cout == 16 && o.cin == 16 && o.ntap == 1 && o.kp == 32 && o.coutP == 16, -1,
+              "the output layer does not follow a 16-channel layer");
+    a.w2 = n.w + o.woff;
+    a.bias2 = n.params + o.poff + (int64_t)o.cout * o.cin;
+    a.y2 = y2;
+    a.cout2 = o.cout;
+  }
   a.nx = nx;
   a.ny = ny;
   a.nz = nz;
   G2G_CHECK(s1.C + s2.C == l.cin, -1, "U-Net layer input width mismatch");
-  const int64_t nvox = (int64_t)nx * ny * nz;
-  hipLaunchKernelGGL(k_conv, dim3(nblk(nvox, 256), l.coutP / 16, n.B), dim3(UB), 0, s, a);
+  conv_launch(a, l.coutP, n.B, s);
 }
 
 // data gradient: dx[p][ci] (FP32, row length cin) from dzb[p][coutT] (bf16)
 static void conv_dx(UNet& n, int li, const bf16* dzb, int nx, int ny, int nz, float* dx, hipStream_t s) {
   const UNetLayer& l = n.L[li];
   const int64_t nvox = (int64_t)nx * ny * nz;
-  ConvArgs a;
+  ConvArgs a{};
   a.s1 = src(dzb, l.coutT, 0, nvox * l.coutT);
   a.s2 = src(nullptr, 0, 0, 0);
   a.w = n.wt + l.wtoff;
@@ -675,7 +931,7 @@ static void conv_dx(UNet& n, int li, const bf16* dzb, int nx, int ny, int nz, fl
   a.nx = nx;
   a.ny = ny;
   a.nz = nz;
-  hipLaunchKernelGGL(k_conv, dim3(nblk(nvox, 256), l.cinP / 16, n.B), dim3(UB), 0, s, a);
+  conv_launch(a, l.cinP, n.B, s);
 }
 
 static void conv_dw(UNet& n, int li, const float* dzf, int ldz, Src s1, Src s2, int nx, int ny, int nz,
@@ -704,12 +960,15 @@ static void conv_dw(UNet& n, int li, const float* dzf, int ldz, Src s1, Src s2, 
   hipLaunchKernelGGL(k_dw, dim3((unsigned)((nch + a.chunks - 1) / a.chunks), l.ntap, n.B), dim3(UB), lds, s, a);
 }
 
+static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
 void unet_load_input(UNet& n, const float* x, hipStream_t s) {
-  const int64_t cnt = (int64_t)n.B * n.nx * n.ny * n.nz * 8;
-  hipLaunchKernelGGL(k_f32_to_bf16, dim3(nblk(cnt)), dim3(UB), 0, s, x, n.in, cnt);
+  const int64_t cnt = (int64_t)n.B * n.nx * n.ny * n.nz;
+  if (aligned16(x)) hipLaunchKernelGGL(k_f32_to_bf16<true>, dim3(nblk(cnt)), dim3(UB), 0, s, x, n.in, cnt);
+  else hipLaunchKernelGGL(k_f32_to_bf16<false>, dim3(nblk(cnt)), dim3(UB), 0, s, x, n.in, cnt);
 }
 
-void unet_forward(UNet& n, hipStream_t s) {
+void unet_forward(UNet& n, hipStream_t s, const float* x, float* y) {
   G2G_CHECK(n.ws != nullptr, -4, "U-Net workspace not reserved");
   unet_prepare_weights(n, s);
   const int X0 = n.nx, Y0 = n.ny, Z0 = n.nz, X1 = X0 / 2, Y1 = Y0 / 2, Z1 = Z0 / 2, X2 = X1 / 2,
@@ -717,21 +976,23 @@ void unet_forward(UNet& n, hipStream_t s) {
   const int64_t v0 = (int64_t)X0 * Y0 * Z0, v1 = v0 / 8, v2 = v0 / 64;
   const Src none = src(nullptr, 0, 0, 0);
   bf16** A = n.act;
-  conv_fwd(n, 0, src(n.in, 8, 0, v0 * 8), none, X0, Y0, Z0, A[0], nullptr, 16, s);
-  conv_fwd(n, 1, src(A[0], 16, 0, v0 * 16), none, X0, Y0, Z0, A[1], nullptr, 16, s);
+  conv_fwd(n, 0, src(n.in, 8, 0, v0 * 8), none, X0, Y0, Z0, A[0], s, x);
+  conv_fwd(n, 1, src(A[0], 16, 0, v0 * 16), none, X0, Y0, Z0, A[1], s);
   hipLaunchKernelGGL(k_pool, dim3(nblk((int64_t)n.B * v1 * 2)), dim3(UB), 0, s, A[1], n.p1, 16, X0, Y0, Z0,
                      (int64_t)n.B);
-  conv_fwd(n, 2, src(n.p1, 16, 0, v1 * 16), none, X1, Y1, Z1, A[2], nullptr, 32, s);
-  conv_fwd(n, 3, src(A[2], 32, 0, v1 * 32), none, X1, Y1, Z1, A[3], nullptr, 32, s);
+  conv_fwd(n, 2, src(n.p1, 16, 0, v1 * 16), none, X1, Y1, Z1, A[2], s);
+  conv_fwd(n, 3, src(A[2], 32, 0, v1 * 32), none, X1, Y1, Z1, A[3], s);
   hipLaunchKernelGGL(k_pool, dim3(nblk((int64_t)n.B * v2 * 4)), dim3(UB), 0, s, A[3], n.p2, 32, X1, Y1, Z1,
                      (int64_t)n.B);
-  conv_fwd(n, 4, src(n.p2, 32, 0, v2 * 32), none, X2, Y2, Z2, A[4], nullptr, 64, s);
-  conv_fwd(n, 5, src(A[4], 64, 0, v2 * 64), none, X2, Y2, Z2, A[5], nullptr, 64, s);
-  conv_fwd(n, 6, src(A[5], 64, 1, v2 * 64), src(A[3], 32, 0, v1 * 32), X1, Y1, Z1, A[6], nullptr, 32, s);
-  conv_fwd(n, 7, src(A[6], 32, 0, v1 * 32), none, X1, Y1, Z1, A[7], nullptr, 32, s);
-  conv_fwd(n, 8, src(A[7], 32, 1, v1 * 32), src(A[1], 16, 0, v0 * 16), X0, Y0, Z0, A[8], nullptr, 16, s);
-  conv_fwd(n, 9, src(A[8], 16, 0, v0 * 16), none, X0, Y0, Z0, A[9], nullptr, 16, s);
-  conv_fwd(n, 10, src(A[9], 16, 0, v0 * 16), none, X0, Y0, Z0, nullptr, n.out, 6, s);
+  conv_fwd(n, 4, src(n.p2, 32, 0, v2 * 32), none, X2, Y2, Z2, A[4], s);
+  conv_fwd(n, 5, src(A[4], 64, 0, v2 * 64), none, X2, Y2, Z2, A[5], s);
+  conv_fwd(n, 6, src(A[5], 64, 1, v2 * 64), src(A[3], 32, 0, v1 * 32), X1, Y1, Z1, A[6], s);
+  conv_fwd(n, 7, src(A[6], 32, 0, v1 * 32), none, X1, Y1, Z1, A[7], s);
+  conv_fwd(n, 8, src(A[7], 32, 1, v1 * 32), src(A[1], 16, 0, v0 * 16), X0, Y0, Z0, A[8], s);
+  // the 1x1 output layer runs on the last layer's registers; its bf16 input
+  // is stored only for a backward pass
+  conv_fwd(n, 9, src(A[8], 16, 0, v0 * 16), none, X0, Y0, Z0, n.training ? A[9] : nullptr, s, nullptr,
+           y ? y : n.out);
   G2G_HIP(hipGetLastError());
 }
 

@@ -46,8 +46,10 @@ void unet_init(UNet& n, int seed_unused);
 void unet_free(UNet& n);
 void unet_reserve(UNet& n, int B, int nx, int ny, int nz, bool training);
 void unet_prepare_weights(UNet& n, hipStream_t s);
-// forward of the batch already packed in n.in; output FP32 [B][vox][6] in n.out
-void unet_forward(UNet& n, hipStream_t s);
+// forward of the batch packed in n.in, or, when x is not null (16-byte aligned,
+// no backward to follow), of the FP32 [B][vox][8] volume x; output FP32
+// [B][vox][6] in y, or n.out when y is null
+void unet_forward(UNet& n, hipStream_t s, const float* x = nullptr, float* y = nullptr);
 // gradient of sum(dy*out) for the last forward; dy FP32 [B][vox][8] in n.dout
 void unet_backward(UNet& n, hipStream_t s);
 // copy an FP32 [B][vox][8] input into n.in (bf16)

@@ -139,3 +139,33 @@ def test_learned_modes_converge_with_untrained_net(mode, prec):
     op.set_learned(None)
     op.close()
     net.close()
+
+
+@pytest.mark.parametrize("B,Z,Y,X", [(1, 4, 4, 20), (2, 4, 12, 36), (1, 12, 20, 4), (1, 20, 36, 8)])
+def test_unet_tiles_with_remainders(B, Z, Y, X):
+    """Volumes that no tile shape (16x4x4, 8x8x4, 4x8x8 and their halves)
+    divides, at every level: the output against the oracle with the same
+    roundings (the 2e-2 bar above) and, bit for bit, the pass that reads the
+    FP32 input itself against the one that keeps activations, and an input
+    that is not 16-byte aligned against an aligned one."""
+    torch = _torch()
+    from giem2g_amd import learned
+    from oracle import unet_ref as U
+    print("case", B, Z, Y, X, flush=True)
+    rng = np.random.default_rng(B * 100 + Z + Y + X)
+    p = _params(11)
+    x = rng.standard_normal((B, Z, Y, X, 8)).astype(np.float32)
+    xt = torch.from_numpy(x).cuda()
+    off = torch.empty(xt.numel() + 1, dtype=torch.float32, device="cuda")[1:].view(xt.shape)
+    off.copy_(xt)
+    assert off.data_ptr() % 16 and off.is_contiguous()
+    net = learned.UNet(params=p)
+    y = net.forward(xt)
+    assert torch.equal(net.forward(off), y)
+    assert torch.equal(net.forward(xt, keep=True), y)
+    assert torch.equal(net.forward(off, keep=True), y)
+    y = y.cpu().numpy().astype(np.float64)
+    for b in range(B):
+        o, _ = U.forward(p.astype(np.float64), x[b].astype(np.float64), round_bf16=True)
+        assert rel(y[b], o) < 2e-2
+    net.close()
