@@ -16,7 +16,7 @@
 // 4*(l/16) .. 4*(l/16)+3 of column l%16 -- four consecutive output channels
 // of one voxel, stored as one 8-byte bf16 write.  The data gradient is the
 // same kernel run on the transposed, tap-flipped weights; the weight
-// gradient accumulates in FP32 through LDS tiles.  No reference counterpart:
+// gradient (k_dw) takes exact products and FP32 sums.  No reference counterpart:
 // GFGMRES/seq_fgmres.F90:142-152 preconditions with an inner GMRES.
 #include <cmath>
 #include <complex>
@@ -314,101 +314,216 @@ __global__ __launch_bounds__(UB) void k_conv3(ConvArgs a, ConvTile t) {
   }
 }
 
-// Weight gradient dW[co][t][ci] += sum_p dZ[p][co] X[p+off(t)][ci] and
-// db[co] += sum_p dZ[p][co], FP32.  Block: one tap, a run of 64-voxel
-// chunks; thread: a 4x4 (co, ci) register tile.
+// Weight gradient dW[co][t][ci] = sum_p dZ[p][co] X[p+off(t)][ci] and db[co] =
+// sum_p dZ[p][co] on v_mfma_f32_16x16x32_bf16: 16 co x 16 ci tiles, 32 voxels
+// (two x rows of 16) per instruction.  X is bf16; dZ is FP32 and enters as
+// three bf16 numbers of 8 bits each (h + m + l = dZ exactly), so every product
+// is exact and the sums are FP32, as in the FP32 vector kernel this replaces.
+// A tile of 16 x 4 x 2 voxels is transposed into LDS once, [ci][row][x] and
+// [part][co][row][x], 8 voxels per 16-byte read; the x taps of a row are its
+// 16-byte chunk shifted by one element into or out of the neighbouring dwords,
+// the y and z taps other rows.  Wave (dz, ci tile) accumulates its 9 taps x
+// NCO tiles in registers over all tiles of the block; each block writes its
+// sums to a slot of its own, which k_dw_reduce adds in a fixed order (the
+// sums no longer depend on the order of atomics).  The parts m and l have
+// accumulators of their own, which keeps their roundings out of the large
+// sums.  Strides of an odd number of 16-byte units spread the 16 channels of a
+// read over the banks.  The transposition and the LDS reads bound it (matrix
+// cores about a fifth busy).  Measured at 8 x 64x64x16, all layers: 7910 us on
+// the FP32 vector unit with atomics -> 560 us; error of the sums against FP64
+// 4.4e-7 -> 0.6e-7.
 struct DwArgs {
   const float* dz;
-  int ldz, cout, cout4;
+  int ldz, cout;
   Src s1, s2;
   int cin, ntap;
-  float *dW, *db;
-  int nx, ny, nz;
-  int64_t dzbstride;
-  int chunks;
+  float* part;
+  int64_t pstride;  // cout*ntap*cin + cout
+  int nx, ny, nz, ntx, nty, nt, ntot;
 };
+constexpr int DW_XROW = 24;                 // 16 voxels, then (-, x = -1), (x = 16, -) of a row
+constexpr int DW_XST = 24 * DW_XROW + 8;    // 24 rows (6 y, 4 z) of a channel
+constexpr int DW_ZST = 8 * 16 + 8;          // 8 rows (4 y, 2 z) of a channel
 
-constexpr int DWV = 64;
-
-__global__ __launch_bounds__(UB) void k_dw(DwArgs a) {
-  extern __shared__ float sm[];
-  float* sdz = sm;                    // [DWV][cout4]
-  float* sx = sm + DWV * a.cout4;     // [DWV][cin]
-  const int t = blockIdx.y, bat = blockIdx.z;
-  const int nvox = a.nx * a.ny * a.nz;
-  int dx = 0, dy = 0, dz = 0;
-  if (a.ntap == 27) {
-    dz = t / 9 - 1;
-    dy = (t / 3) % 3 - 1;
-    dx = t % 3 - 1;
-  }
-  const int nci4 = a.cin / 4;
-  const int tiles = (a.cout4 / 4) * nci4;
-  const int tile = threadIdx.x;
-  const int co = (tile / nci4) * 4, ci = (tile % nci4) * 4;
-  float acc[16];
-#pragma unroll
-  for (int q = 0; q < 16; q++) acc[q] = 0.f;
-  float bacc = 0.f;
-  const float* dzb = a.dz + bat * a.dzbstride;
-  const bf16* x1 = a.s1.p + bat * a.s1.bstride;
-  const bf16* x2 = a.s2.p ? a.s2.p + bat * a.s2.bstride : a.s1.p;
+template <int NCO, int NCI, bool ONE>
+__global__ __launch_bounds__(192 * NCI) void k_dw(DwArgs a) {
+  constexpr int NT = 192 * NCI, NCH = 2 * NCI;
+  extern __shared__ __align__(16) unsigned char dw_sm[];
+  bf16* xs = reinterpret_cast<bf16*>(dw_sm);
+  bf16* zs = xs + NCI * 16 * DW_XST;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 15, kq = lane >> 4, half = kq & 1;
+  const int dzi = ONE ? 1 : wave % 3, cit = ONE ? 0 : wave / 3;
+  const int c0 = blockIdx.y * NCI * 16, o0 = blockIdx.z * NCO * 16;
   const int nxh = a.nx >> 1, nyh = a.ny >> 1;
-  for (int ch = 0; ch < a.chunks; ch++) {
-    const int p0 = (blockIdx.x * a.chunks + ch) * DWV;
-    if (p0 >= nvox) break;
-    for (int e = threadIdx.x; e < DWV * a.cout4; e += UB) {
-      const int v = e / a.cout4, c = e - v * a.cout4;
-      const int p = p0 + v;
-      sdz[e] = (p < nvox && c < a.cout) ? dzb[(int64_t)p * a.ldz + c] : 0.f;
+  const bool bias = ONE || (dzi == 1 && cit == 0 && blockIdx.y == 0);
+  constexpr int NTAP = ONE ? 1 : 9;
+  f32x4 acc[2][NTAP][NCO], bacc[2][NCO];  // [0]: the leading part h, [1]: m and l
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+#pragma unroll
+    for (int t = 0; t < NCO; t++) {
+      bacc[h][t] = f32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int k = 0; k < NTAP; k++) acc[h][k][t] = f32x4{0, 0, 0, 0};
     }
-    for (int e = threadIdx.x; e < DWV * a.cin; e += UB) {
-      const int v = e / a.cin, c = e - v * a.cin;
-      const int p = p0 + v;
-      float val = 0.f;
-      if (p < nvox) {
-        const int x = p % a.nx, y = (p / a.nx) % a.ny, z = p / (a.nx * a.ny);
-        const int X = x + dx, Y = y + dy, Z = z + dz;
-        if (X >= 0 && X < a.nx && Y >= 0 && Y < a.ny && Z >= 0 && Z < a.nz) {
-          const bf16* sp = x1;
-          int C = a.s1.C, cc = c, up = a.s1.up;
-          if (c >= a.s1.C) {
-            sp = x2;
-            C = a.s2.C;
-            cc = c - a.s1.C;
-            up = a.s2.up;
-          }
-          int64_t q;
-          if (up) q = ((int64_t)(Z >> 1) * nyh + (Y >> 1)) * nxh + (X >> 1);
-          else q = ((int64_t)Z * a.ny + Y) * a.nx + X;
-          val = (float)sp[q * C + cc];
+  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  const bf16 one1 = (bf16)1.f;
+  const bf16x8 ones = {one1, one1, one1, one1, one1, one1, one1, one1};
+  const int first = (int)((int64_t)a.ntot * blockIdx.x / gridDim.x);
+  const int last = (int)((int64_t)a.ntot * (blockIdx.x + 1) / gridDim.x);
+  for (int tile = first; tile < last; tile++) {
+    const int bat = tile / a.nt, tt = tile - bat * a.nt;
+    const int z0 = tt / (a.ntx * a.nty) * 2, y0 = (tt / a.ntx) % a.nty * 4, x0 = tt % a.ntx * 16;
+    // one voxel's 8 channels of chunk c (zero outside the volume); the load is
+    // unconditional, from a clamped voxel
+    auto ldx = [&](int c, int X, int Y, int Z) -> bf16x8 {
+      const int ci = c0 + c * 8;
+      const bool in = ci < a.cin && X >= 0 && X < a.nx && Y >= 0 && Y < a.ny && Z >= 0 && Z < a.nz;
+      const int Xc = min(max(X, 0), a.nx - 1), Yc = min(max(Y, 0), a.ny - 1), Zc = min(max(Z, 0), a.nz - 1);
+      const int cc = ci < a.cin ? ci : 0;
+      const bool f = cc < a.s1.C;
+      const Src& sr = f ? a.s1 : a.s2;
+      const int64_t q = sr.up ? ((int64_t)(Zc >> 1) * nyh + (Yc >> 1)) * nxh + (Xc >> 1)
+                              : ((int64_t)Zc * a.ny + Yc) * a.nx + Xc;
+      const bf16x8 v =
+          *reinterpret_cast<const bf16x8*>(sr.p + bat * sr.bstride + q * sr.C + (f ? cc : cc - a.s1.C));
+      return in ? v : zero;
+    };
+    for (int e = tid; e < 48 * NCH; e += NT) {
+      const int c = e % NCH, r = e / NCH, h8 = (r & 1) * 8, row = r >> 1, hy = row % 6, hz = row / 6;
+      bf16x8 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[j] = ldx(c, x0 + h8 + j, y0 + hy - 1, z0 + hz - 1);
+      bf16* dst = xs + c * 8 * DW_XST + row * DW_XROW + h8;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const bf16x8 o = {v[0][k], v[1][k], v[2][k], v[3][k], v[4][k], v[5][k], v[6][k], v[7][k]};
+        *reinterpret_cast<bf16x8*>(dst + k * DW_XST) = o;
+      }
+    }
+    if constexpr (!ONE) {
+      for (int e = tid; e < 48 * NCH; e += NT) {
+        const int c = e % NCH, r = e / NCH, side = r & 1, row = r >> 1, hy = row % 6, hz = row / 6;
+        const bf16x8 v = ldx(c, side ? x0 + 16 : x0 - 1, y0 + hy - 1, z0 + hz - 1);
+        bf16* dst = xs + c * 8 * DW_XST + row * DW_XROW + 17 + side;
+#pragma unroll
+        for (int k = 0; k < 8; k++) dst[k * DW_XST] = v[k];
+      }
+    }
+    for (int e = tid; e < 64 * NCO; e += NT) {
+      const int q = e % (4 * NCO), r = e / (4 * NCO), h8 = (r & 1) * 8, row = r >> 1, co = o0 + q * 4;
+      const int Y = y0 + (row & 3), Z = z0 + (row >> 2);
+      const bool in = co < a.ldz && Y < a.ny && Z < a.nz;
+      const float* src = a.dz + (((int64_t)bat * a.nz + min(Z, a.nz - 1)) * a.ny + min(Y, a.ny - 1)) * a.nx * a.ldz +
+                         (co < a.ldz ? co : 0);
+      f32x4 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int X = x0 + h8 + j;
+        const f32x4 g = *reinterpret_cast<const f32x4*>(src + (int64_t)min(X, a.nx - 1) * a.ldz);
+        v[j] = in && X < a.nx ? g : f32x4{0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        bf16x8 p0, p1, p2;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          // h, m: the leading 8 bits of v and of the rest (truncated, so that
+          // both rests are exact); an infinity or NaN goes into h alone
+          const float x = v[j][i];
+          const unsigned u = __float_as_uint(x);
+          const bool fin = (u & 0x7f800000u) != 0x7f800000u;
+          const float h = __uint_as_float(u & 0xffff0000u);
+          const float r1 = fin ? x - h : 0.f;
+          const float m = __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+          p0[j] = (bf16)(fin ? h : x);
+          p1[j] = (bf16)m;
+          p2[j] = (bf16)(r1 - m);
+        }
+        bf16* dst = zs + (q * 4 + i) * DW_ZST + row * 16 + h8;
+        *reinterpret_cast<bf16x8*>(dst) = p0;
+        *reinterpret_cast<bf16x8*>(dst + NCO * 16 * DW_ZST) = p1;
+        *reinterpret_cast<bf16x8*>(dst + 2 * NCO * 16 * DW_ZST) = p2;
+      }
+    }
+    __syncthreads();
+    for (int s = ONE ? wave : 0; s < 4; s += ONE ? 3 : 1) {
+      const int z = s >> 1, y = (s & 1) * 2 + (kq >> 1);
+      bf16x8 af[3][NCO];
+#pragma unroll
+      for (int p = 0; p < 3; p++)
+#pragma unroll
+        for (int t = 0; t < NCO; t++)
+          af[p][t] = *reinterpret_cast<const bf16x8*>(zs + ((p * NCO + t) * 16 + col) * DW_ZST + (z * 4 + y) * 16 + half * 8);
+#pragma unroll
+      for (int dy = ONE ? 1 : 0; dy < (ONE ? 2 : 3); dy++) {
+        const bf16* row = xs + (cit * 16 + col) * DW_XST + ((z + dzi) * 6 + y + dy) * DW_XROW;
+        const bf16x8 bc = *reinterpret_cast<const bf16x8*>(row + half * 8);
+        if constexpr (ONE) {
+#pragma unroll
+          for (int t = 0; t < NCO; t++)
+#pragma unroll
+            for (int p = 2; p >= 0; p--) acc[p > 0][0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][t], bc, acc[p > 0][0][t], 0, 0, 0);
+        } else {
+          const unsigned prev = *reinterpret_cast<const unsigned*>(row + (half ? 6 : 16));
+          const unsigned next = *reinterpret_cast<const unsigned*>(row + (half ? 18 : 8));
+          const uint4 c = __builtin_bit_cast(uint4, bc);
+          const unsigned m0 = __builtin_amdgcn_alignbit(c.x, prev, 16), m1 = __builtin_amdgcn_alignbit(c.y, c.x, 16),
+                         m2 = __builtin_amdgcn_alignbit(c.z, c.y, 16), m3 = __builtin_amdgcn_alignbit(c.w, c.z, 16),
+                         m4 = __builtin_amdgcn_alignbit(next, c.w, 16);
+          const bf16x8 bx[3] = {__builtin_bit_cast(bf16x8, uint4{m0, m1, m2, m3}), bc,
+                                __builtin_bit_cast(bf16x8, uint4{m1, m2, m3, m4})};
+#pragma unroll
+          for (int p = 2; p >= 0; p--)
+#pragma unroll
+            for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+              for (int t = 0; t < NCO; t++)
+                acc[p > 0][dy * 3 + dx][t] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][t], bx[dx], acc[p > 0][dy * 3 + dx][t], 0, 0, 0);
         }
       }
-      sx[e] = val;
-    }
-    __syncthreads();
-    if (tile < tiles) {
-      for (int v = 0; v < DWV; v++) {
-        const f32x4 g = *reinterpret_cast<const f32x4*>(sdz + v * a.cout4 + co);
-        const f32x4 xv = *reinterpret_cast<const f32x4*>(sx + v * a.cin + ci);
+      if (bias) {
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int t = 0; t < NCO; t++)
 #pragma unroll
-          for (int j = 0; j < 4; j++) acc[i * 4 + j] += g[i] * xv[j];
+          for (int p = 2; p >= 0; p--)
+            bacc[p > 0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][t], ones, bacc[p > 0][t], 0, 0, 0);
       }
     }
-    if (t == 0 && threadIdx.x < a.cout)
-      for (int v = 0; v < DWV; v++) bacc += sdz[v * a.cout4 + threadIdx.x];
     __syncthreads();
   }
-  if (tile < tiles) {
+  // lane (col, kq) holds input channel col and output channels 4 kq + q of each tile
+  float* part = a.part + (ONE ? (int64_t)blockIdx.x * 3 + wave : (int64_t)blockIdx.x) * a.pstride;
+  const int ci = c0 + cit * 16 + col;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+  for (int t = 0; t < NCO; t++)
 #pragma unroll
-      for (int j = 0; j < 4; j++)
-        if (co + i < a.cout) atomicAdd(a.dW + ((int64_t)(co + i) * a.ntap + t) * a.cin + ci + j, acc[i * 4 + j]);
+    for (int q = 0; q < 4; q++) {
+      const int co = o0 + t * 16 + kq * 4 + q;
+      if (co >= a.cout) continue;
+      if (ci < a.cin) {
+#pragma unroll
+        for (int k = 0; k < NTAP; k++) part[((int64_t)co * a.ntap + (ONE ? 0 : dzi * 9 + k)) * a.cin + ci] = acc[0][k][t][q] + acc[1][k][t][q];
+      }
+      if (bias && col == 0) part[(int64_t)a.cout * a.ntap * a.cin + co] = bacc[0][t][q] + bacc[1][t][q];
+    }
+}
+
+// g[i] = sum over the np slots of part[slot][i], in a fixed order, in double
+__global__ __launch_bounds__(UB) void k_dw_reduce(const float* __restrict__ part, int np, int64_t n, float* __restrict__ g) {
+  __shared__ double red[UB];
+  const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+  double s = 0;
+  if (i < n) {
+#pragma unroll 8
+    for (int k = threadIdx.x >> 6; k < np; k += UB / 64) s += (double)part[k * n + i];
   }
-  if (t == 0 && threadIdx.x < a.cout) atomicAdd(a.db + threadIdx.x, bacc);
+  red[threadIdx.x] = s;
+  __syncthreads();
+  if (threadIdx.x < 64 && i < n)
+    g[i] = (float)((red[threadIdx.x] + red[threadIdx.x + 64]) + (red[threadIdx.x + 128] + red[threadIdx.x + 192]));
 }
 
 // forward weights w[co][tap*cin+ci] and transposed weights
@@ -736,6 +851,31 @@ void unet_free(UNet& n) {
   n = UNet();
 }
 
+// tiles of the weight gradient at a level
+static int dw_tiles(int B, int nx, int ny, int nz) { return B * ((nx + 15) / 16) * ((ny + 3) / 4) * ((nz + 1) / 2); }
+
+// Slots of a layer's weight gradient (one per block), one tile or more each, at
+// least 64: as many as 32 MB of partial sums hold for up to 16 output channels
+// (three 64-thread waves a block: 60 -> 47 us a layer against 16 MB), 16 MB
+// for wider ones (42 us against 49 with 32 MB: the sums' traffic)
+static int dw_slots(const UNetLayer& l, int tiles) {
+  const int64_t per = (int64_t)l.cout * l.ntap * l.cin + l.cout;
+  return (int)std::min<int64_t>(tiles, std::min<int64_t>(1024, std::max<int64_t>(64, (int64_t(l.cout <= 16 ? 8 : 4) << 20) / per)));
+}
+
+// floats of the partial sums of every layer of a training step
+static int64_t dw_part_size(const UNet& n, int B, int nx, int ny, int nz) {
+  int64_t most = 0;
+  static const int level[11] = {0, 0, 1, 1, 2, 2, 1, 1, 0, 0, 0};
+  for (int i = 0; i < 11; i++) {
+    const UNetLayer& l = n.L[i];
+    const int64_t per = (int64_t)l.cout * l.ntap * l.cin + l.cout;
+    const int t = dw_tiles(B, nx >> level[i], ny >> level[i], nz >> level[i]);
+    most = std::max<int64_t>(most, per * dw_slots(l, t) * (l.ntap == 1 ? 3 : 1));
+  }
+  return most;
+}
+
 void unet_reserve(UNet& n, int B, int nx, int ny, int nz, bool training) {
   G2G_CHECK(nx % 4 == 0 && ny % 4 == 0 && nz % 4 == 0 && nx > 0 && ny > 0 && nz > 0, -2,
             "U-Net volume dimensions must be positive multiples of 4");
@@ -769,8 +909,9 @@ void unet_reserve(UNet& n, int B, int nx, int ny, int nz, bool training) {
     add((void**)&n.de2, 4 * n1 * 32);
     add((void**)&n.dzf, 4 * n0 * 16);
     add((void**)&n.dzb, 2 * n0 * 16);
+    add((void**)&n.dwp, 4 * dw_part_size(n, B, nx, ny, nz));
   } else {
-    n.dout = n.f48 = n.fa = n.fb = n.de1 = n.de2 = n.dzf = nullptr;
+    n.dout = n.f48 = n.fa = n.fb = n.de1 = n.de2 = n.dzf = n.dwp = nullptr;
     n.dzb = nullptr;
   }
   void* base = nullptr;
@@ -934,6 +1075,14 @@ static void conv_dx(UNet& n, int li, const bf16* dzb, int nx, int ny, int nz, fl
   conv_launch(a, l.cinP, n.B, s);
 }
 
+template <int NCO, int NCI, bool ONE> static void dw_go(const DwArgs& a, int slots, int gy, int gz, hipStream_t s) {
+  const size_t lds = sizeof(bf16) * (NCI * 16 * DW_XST + 3 * NCO * 16 * DW_ZST);
+  if (lds > 65536)
+    G2G_HIP(hipFuncSetAttribute((const void*)k_dw<NCO, NCI, ONE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
+  hipLaunchKernelGGL((k_dw<NCO, NCI, ONE>), dim3(slots, gy, gz), dim3(192 * NCI), lds, s, a);
+}
+
 static void conv_dw(UNet& n, int li, const float* dzf, int ldz, Src s1, Src s2, int nx, int ny, int nz,
                     hipStream_t s) {
   const UNetLayer& l = n.L[li];
@@ -941,23 +1090,34 @@ static void conv_dw(UNet& n, int li, const float* dzf, int ldz, Src s1, Src s2, 
   a.dz = dzf;
   a.ldz = ldz;
   a.cout = l.cout;
-  a.cout4 = (int)up_to(l.cout, 4);
   a.s1 = s1;
-  a.s2 = s2;
+  a.s2 = s2.p ? s2 : s1;
   a.cin = l.cin;
   a.ntap = l.ntap;
-  a.dW = n.grads + l.poff;
-  a.db = n.grads + l.poff + (int64_t)l.cout * l.ntap * l.cin;
+  a.part = n.dwp;
+  a.pstride = (int64_t)l.cout * l.ntap * l.cin + l.cout;
   a.nx = nx;
   a.ny = ny;
   a.nz = nz;
-  const int64_t nvox = (int64_t)nx * ny * nz;
-  a.dzbstride = nvox * ldz;
-  const int64_t nch = (nvox + DWV - 1) / DWV;
-  a.chunks = (int)std::max<int64_t>(1, std::min<int64_t>(32, nch / 64));
-  const size_t lds = sizeof(float) * DWV * (a.cout4 + l.cin);
-  G2G_CHECK((a.cout4 / 4) * (l.cin / 4) <= UB, -1, "weight-gradient tile count exceeds the block");
-  hipLaunchKernelGGL(k_dw, dim3((unsigned)((nch + a.chunks - 1) / a.chunks), l.ntap, n.B), dim3(UB), lds, s, a);
+  a.ntx = (nx + 15) / 16;
+  a.nty = (ny + 3) / 4;
+  a.ntot = dw_tiles(n.B, nx, ny, nz);
+  a.nt = a.ntot / n.B;
+  const int slots = dw_slots(l, a.ntot);
+  G2G_CHECK(ldz % 4 == 0 && l.cin % 8 == 0 && s1.C + s2.C == l.cin, -1, "weight gradient: layer widths");
+  // tiles of 16 channels: one by one or two by two in a block; wider layers
+  // take blocks side by side (48 input channels: 135 us as three blocks, 166
+  // us as one of nine waves, which left a third of the CUs idle)
+  const int no = (l.cout + 15) / 16, ni = (l.cin + 15) / 16;
+  if (l.ntap == 1) {
+    G2G_CHECK(no == 1 && ni == 1, -1, "weight gradient: 1x1 layer of more than 16 channels");
+    dw_go<1, 1, true>(a, slots, 1, 1, s);
+  } else if (no == 1) dw_go<1, 1, false>(a, slots, ni, 1, s);
+  else if (no % 2 == 0 && ni == 1) dw_go<2, 1, false>(a, slots, 1, no / 2, s);
+  else if (no % 2 == 0 && ni % 2 == 0) dw_go<2, 2, false>(a, slots, ni / 2, no / 2, s);
+  else G2G_CHECK(false, -1, "no weight-gradient kernel for this layer width");
+  hipLaunchKernelGGL(k_dw_reduce, dim3(nblk(a.pstride, 64)), dim3(UB), 0, s, n.dwp, slots * (l.ntap == 1 ? 3 : 1),
+                     a.pstride, n.grads + l.poff);
 }
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -1015,7 +1175,6 @@ void unet_backward(UNet& n, hipStream_t s) {
   const int64_t B = n.B;
   const Src none = src(nullptr, 0, 0, 0);
   bf16** A = n.act;
-  G2G_HIP(hipMemsetAsync(n.grads, 0, sizeof(float) * n.nparams, s));
   layer_back(n, 10, n.dout, 8, nullptr, src(A[9], 16, 0, v0 * 16), none, X0, Y0, Z0, n.fa, s);
   layer_back(n, 9, n.fa, 16, A[9], src(A[8], 16, 0, v0 * 16), none, X0, Y0, Z0, n.fa, s);
   layer_back(n, 8, n.fa, 16, A[8], src(A[7], 32, 1, v1 * 32), src(A[1], 16, 0, v0 * 16), X0, Y0, Z0, n.f48,

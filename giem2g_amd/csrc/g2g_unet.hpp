@@ -36,7 +36,7 @@ struct UNet {
   bf16 *in = nullptr, *act[11] = {}, *p1 = nullptr, *p2 = nullptr;
   float* out = nullptr;
   float *dout = nullptr, *f48 = nullptr, *fa = nullptr, *fb = nullptr, *de1 = nullptr,
-        *de2 = nullptr, *dzf = nullptr;
+        *de2 = nullptr, *dzf = nullptr, *dwp = nullptr;
   bf16* dzb = nullptr;
   double* dscal = nullptr;  // loss accumulator / residual scale
 };

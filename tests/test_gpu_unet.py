@@ -169,3 +169,54 @@ def test_unet_tiles_with_remainders(B, Z, Y, X):
         o, _ = U.forward(p.astype(np.float64), x[b].astype(np.float64), round_bf16=True)
         assert rel(y[b], o) < 2e-2
     net.close()
+
+
+@pytest.mark.parametrize("B,Z,Y,X", [(1, 4, 4, 4), (2, 12, 20, 36), (1, 8, 12, 64), (3, 4, 28, 16)])
+def test_weight_gradient_sums(B, Z, Y, X):
+    """Weight and bias gradients of the last two layers against FP64 sums of
+    the same products, where they are known exactly: a network that hands
+    channels 0-7 through (identity taps), so that both layers' input is
+    relu(x) and the output gradient reaches them unmixed.  The products are
+    exact and the sums FP32, over 32 voxels at a time: within
+    (voxels / 32 + 64) 2^-24 of the sum of the terms' magnitudes."""
+    torch = _torch()
+    from giem2g_amd import learned
+    print("case", B, Z, Y, X, flush=True)
+    parts, offs, off = [], [], 0
+    for li, (ci, co, t) in enumerate(learned.ARCH):
+        W = np.zeros((co, t, ci), np.float32)
+        for c in range(6 if li == 10 else 8):
+            if li in (0, 1, 9, 10):
+                W[c, t // 2, c] = 1
+            elif li == 8:
+                W[c, t // 2, 32 + c] = 1
+        parts += [W.ravel(), np.zeros(co, np.float32)]
+        offs.append(off)
+        off += co * t * ci + co
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(X)
+    x = torch.randn((B, Z, Y, X, 8), generator=gen, device="cuda").to(torch.bfloat16).float()
+    dy = torch.randn((B, Z, Y, X, 6), generator=gen, device="cuda")
+    net = learned.UNet(params=np.concatenate(parts))
+    net.forward(x, keep=True)
+    g = net.backward(dy)
+    assert np.array_equal(net.backward(dy), g)  # fixed order of the sums
+    g = g.astype(np.float64)
+    a, d = torch.relu(x).double().cpu().numpy(), dy.double().cpu().numpy()
+    n = B * Z * Y * X
+    bar = (n / 32 + 64) * 2.0 ** -24
+    A, D = a.reshape(n, 8), d.reshape(n, 6)
+    w10 = g[offs[10]:offs[10] + 96].reshape(6, 16)[:, :8]
+    assert np.all(np.abs(w10 - D.T @ A) <= bar * (np.abs(D).T @ A))
+    assert np.all(np.abs(g[offs[10] + 96:] - D.sum(0)) <= bar * np.abs(D).sum(0))
+    d9 = dy.to(torch.bfloat16).double().cpu().numpy() * (a[..., :6] > 0)
+    D9 = d9.reshape(n, 6)
+    p = np.pad(a, ((0, 0), (1, 1), (1, 1), (1, 1), (0, 0)))
+    w9 = g[offs[9]:offs[9] + 16 * 27 * 16].reshape(16, 27, 16)
+    for t in range(27):
+        dz, ty, tx = t // 9, (t // 3) % 3, t % 3
+        q = p[:, dz:dz + Z, ty:ty + Y, tx:tx + X].reshape(n, 8)
+        assert np.all(np.abs(w9[:6, t, :8] - D9.T @ q) <= bar * (np.abs(D9).T @ q)), t
+    b9 = g[offs[9] + 16 * 27 * 16:offs[10]]
+    assert np.all(np.abs(b9[:6] - D9.sum(0)) <= bar * np.abs(D9).sum(0)) and not np.any(b9[6:])
+    net.close()
