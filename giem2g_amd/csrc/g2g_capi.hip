@@ -170,9 +170,12 @@ void set_background(Operator& op, int Nl, const double* csigb, const double* thi
   if (op.have_sigma) op_set_sigma(op, op.csiga);
 }
 
+// stage 0: the real-space tensor, 1: its spectrum, -1: both (the real-space
+// tensor is then not seen, so a grid with the x-y mirror sums half of it)
 void build_tensor(Operator& op, int stage) {
+  const bool half = stage < 0 && op.Nx == op.Ny && op.dx == op.dy;
   if (stage <= 0) {
-    op_build_tensor(op);
+    op_build_tensor(op, half);
     op.have_tensor = false;
     op.have_g32 = false;
     op.tensor_own = true;
@@ -182,7 +185,7 @@ void build_tensor(Operator& op, int stage) {
     G2G_HIP(hipEventCreate(&a));
     G2G_HIP(hipEventCreate(&b));
     G2G_HIP(hipEventRecord(a, op.stream));
-    op_tensor_fft(op, op.d64.G);
+    op_tensor_fft(op, op.d64.G, half);
     G2G_HIP(hipEventRecord(b, op.stream));
     G2G_HIP(hipEventSynchronize(b));
     float ms = 0;

@@ -309,8 +309,11 @@ void op_set_geometry(Operator& op, double dx, double dy, const double* z);
 void op_apply_adjoint(Operator& op, const zd* vin, zd* vout, hipStream_t s);
 void op_make_g32(Operator& op);
 // tensor build (g2g_tensor.hip)
-void op_build_tensor(Operator& op);
-void op_tensor_fft(Operator& op, zd* G);
+// half (a square grid with dx = dy, nobody reads the real-space tensor): only
+// the components and offsets from which op_tensor_fft(half) makes the whole
+// spectrum by the x-y mirror
+void op_build_tensor(Operator& op, bool half);
+void op_tensor_fft(Operator& op, zd* G, bool half);
 void op_free_tensor_scratch(Operator& op);
 // receiver continuation
 void rc_init(RcOperator& rc, Operator& op, int Nr, const double* xs, const double* ys,

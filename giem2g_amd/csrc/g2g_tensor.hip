@@ -18,8 +18,7 @@
 //                    tables a,b,c (packed symmetric) and d (full) of
 //                    Calc_Double_Integral_U;
 //   3. k_wgemm     : G(offset, entry) = sum_K w(offset,K) * table(K, entry),
-//                    one lane per (offset, z, z') output -- an FP64
-//                    (NxNy x 501) x (501 x Nz^2) product per component;
+//                    FP64 (NxNy x taps) x (taps x Nz^2) matrix products;
 //   4. k_tfft_y/x  : symmetric extension with per-component signs, 2-D FFT,
 //                    Nyquist cancellation, in place.
 #include "g2g_fft.hpp"
@@ -136,8 +135,17 @@ __device__ inline double block_max(double v, double* red) {
   return r;
 }
 
-// One block per offset b = lx + Nx*ly.  Output wts[c][K][b] (IE order).
-__global__ __launch_bounds__(256) void k_weights(double* __restrict__ wts,
+// Window of taps [x, y) outside which every weight of an offset is zero:
+// every thread reports its taps that are on
+__device__ inline void tap_window(int* kw, int K, bool on) {
+  if (!on) return;
+  atomicMin(&kw[0], K);
+  atomicMax(&kw[1], K + 1);
+}
+
+// One block per offset b = lx + Nx*ly.  Output wts[c][K][b] (IE order) and
+// the offset's window of taps win[b].
+__global__ __launch_bounds__(256) void k_weights(double* __restrict__ wts, int2* __restrict__ win,
                                                  const zd* __restrict__ f1,
                                                  const zd* __restrict__ twg,
                                                  const double* __restrict__ lms, WParams P) {
@@ -211,6 +219,9 @@ __global__ __launch_bounds__(256) void k_weights(double* __restrict__ wts,
   }
   W0[IE_D0] = colmax(IE_D0);
   const int64_t M = (int64_t)P.Nx * P.Ny;
+  __shared__ int kw[2];
+  if (threadIdx.x < 2) kw[threadIdx.x] = threadIdx.x == 0 ? NTAPS : 0;
+  __syncthreads();
   for (int K = threadIdx.x; K < NTAPS; K += 256) {
     double w[6];
     for (int c = 0; c < 6; c++) w[c] = wt[c][K];
@@ -237,7 +248,10 @@ __global__ __launch_bounds__(256) void k_weights(double* __restrict__ wts,
     o[IE_DY] = w[IE_DY] * lm;
     o[IE_D0] = w[IE_D0] * lm;
     for (int c = 0; c < 6; c++) wts[((int64_t)c * NTAPS + K) * M + b] = on ? o[c] : 0.0;
+    tap_window(kw, K, on);
   }
+  __syncthreads();
+  if (threadIdx.x == 0) win[b] = make_int2(kw[0], kw[1]);
 }
 
 // ------------------------------------------------------ lambda tables ---
@@ -484,57 +498,157 @@ __global__ __launch_bounds__(64) void k_lambda(zd* __restrict__ tabs,
 }
 
 // --------------------------------------------------------- weighted sum ---
-// C[b][off + e] = scale * sum_seg sum_K A_seg[K][b] * B_seg[K][e]
-// (A real, B complex).  Tile 64 offsets x 32 entries, K-chunks of 16.
-struct GemmSeg {
-  const double* A;   // [K][M]
-  const zd* B;  // [K][ldb], entry e at B[K*ldb + e]
+// C[o][coff + e] = scale * sum_seg sum_K A_seg[K][o] * B_seg[K][e] for every
+// offset o and entry e (A real weights, B complex tables): FP64 matrix
+// products (offsets x taps) (taps x 2 entries) on v_mfma_f64_16x16x4, all
+// jobs (tensor components) of a build in one launch.  Bound by the FP64
+// matrix rate.  Three things keep it below the (offsets x 501 x entries) of
+// the plain sum:
+//   - the taps: a block sums the window in which one of its offsets has a
+//     weight (the 1e-12 mask of the weights leaves 210 to 370 of 501 taps);
+//   - the x-y mirror (TRI): on a square grid with dx = dy the block at
+//     (ly,lx) is that at (lx,ly) with x and y exchanged, so offsets lx >= ly
+//     are summed and stored in both places (coff2: the exchanged component);
+//   - a tile is 128 offsets x 32 complex entries, double-buffered in LDS by
+//     chunks of 8 taps, so that the loads of a chunk run beside the matrix
+//     products of the one before.
+// Measured (128x128x32): six launches on the vector unit, every tap and offset,
+// 4830 us (35 TFLOP/s) -> 980 us (46 TFLOP/s of the sums that are left); with
+// two receivers, thirty launches 5930 us (27 TFLOP/s) -> 1400 us (59 TFLOP/s).
+struct WJob {
+  int coff, coff2, Ne, nseg;  // coff or coff2 < 0: not stored there
+  const double *A0, *A1;  // [K][lda]
+  const zd *B0, *B1;      // [K][ldb], entry e at B[K*ldb + e]
 };
-__global__ __launch_bounds__(256) void k_wgemm(zd* __restrict__ C, int64_t M, int64_t BS,
-                                               int coff, int Ne, int64_t ldb, GemmSeg s0,
-                                               GemmSeg s1, int nseg, double scale) {
-  constexpr int TM = 64, TN = 32, TK = 16;
-  __shared__ double As[TK][TM];
-  __shared__ zd Bs[TK][TN + 1];
-  const int m0 = blockIdx.x * TM, n0 = blockIdx.y * TN;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;  // 16 x 16
-  zd acc[4][2];
-  for (int a = 0; a < 4; a++)
-    for (int c = 0; c < 2; c++) acc[a][c] = mkz(0, 0);
-  for (int sgi = 0; sgi < nseg; sgi++) {
-    const GemmSeg sg = sgi == 0 ? s0 : s1;
-    for (int k0 = 0; k0 < NTAPS; k0 += TK) {
+struct WJobs {
+  int n;
+  WJob j[15];
+};
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// (at least three waves per SIMD asked for: below two the compiler keeps the
+// accumulators in the second register file and copies them every chunk)
+template <bool TRI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_wgemm(zd* __restrict__ C, int64_t rows, int64_t lda, int64_t BS, int64_t ldb,
+                                               const int2* __restrict__ win, int Nx, double scale, WJobs jobs) {
+  constexpr int TM = 128, TE = 32, TK = 8, LA = TM + 16, LB = 2 * TE + 16;
+  __shared__ double As[2][TK][LA];
+  __shared__ __align__(16) double Bs[2][TK][LB];
+  __shared__ int64_t mo[TM], mt[TM];
+  __shared__ int kw[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, kq = lane >> 4;
+  // job and entry tile of this block
+  int jt = blockIdx.y, ji = 0;
+  while (jt >= (jobs.j[ji].Ne + TE - 1) / TE) {
+    jt -= (jobs.j[ji].Ne + TE - 1) / TE;
+    ji++;
+  }
+  const WJob job = jobs.j[ji];
+  const int n0 = jt * TE;
+  if (tid < 2) kw[tid] = tid == 0 ? NTAPS : 0;
+  __syncthreads();
+  if (tid < TM) {
+    const int64_t t = (int64_t)blockIdx.x * TM + tid;
+    int64_t o = -1, ot = -1;
+    if (t < rows) {
+      if constexpr (TRI) {
+        // rows ly = r (lx = r .. Nx-1) and ly = Nx-1-r together have Nx+1 offsets
+        const int r = (int)(t / (Nx + 1)), c = (int)(t - (int64_t)r * (Nx + 1));
+        const int ly = c < Nx - r ? r : Nx - 1 - r, lx = c < Nx - r ? r + c : c - 1;
+        o = lx + (int64_t)Nx * ly;
+        if (lx != ly) ot = ly + (int64_t)Nx * lx;
+      } else {
+        o = t;
+      }
+      const int2 w = win[o];
+      atomicMin(&kw[0], w.x);
+      atomicMax(&kw[1], w.y);
+    }
+    mo[tid] = o;
+    mt[tid] = ot;
+  }
+  __syncthreads();
+  const int klo = kw[0], khi = kw[1];
+  const int nch = khi > klo ? (khi - klo + TK - 1) / TK : 0, nct = nch * job.nseg;
+  // loads: offset tid % 128 of taps tid / 128 + 2 i; entry tid % 32 of tap tid / 32
+  const int am = tid & (TM - 1), ak = tid >> 7, bn = tid & (TE - 1), bk = tid >> 5;
+  // (rows and entries past the end read the first ones and are not stored;
+  // taps past the window count as zero weights.  No branch: with one per load
+  // or chunk the compiler moved the accumulators between register files in
+  // every chunk, 1180 us against 980)
+  const int64_t ao = mo[am] < 0 ? 0 : mo[am];
+  const int bo = n0 + bn < job.Ne ? n0 + bn : n0;
+  double ra[4];
+  zd rb;
+  auto load = [&](int c) {
+    const bool second = c >= nch;
+    const int k0 = klo + (second ? c - nch : c) * TK;
+    const double* A = second ? job.A1 : job.A0;
+    const zd* B = second ? job.B1 : job.B0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int K = k0 + ak + 2 * i;
+      const double v = A[(int64_t)min(K, NTAPS - 1) * lda + ao];
+      ra[i] = K < khi ? v : 0.0;
+    }
+    rb = B[(int64_t)min(k0 + bk, NTAPS - 1) * ldb + bo];
+  };
+  auto stash = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) As[buf][ak + 2 * i][am] = ra[i];
+    *reinterpret_cast<zd*>(&Bs[buf][bk][2 * bn]) = rb;
+  };
+  f64x4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc[i][j] = f64x4{0, 0, 0, 0};
+  if (nct > 0) {
+    load(0);
+    stash(0);
+    __syncthreads();
+    for (int c = 0; c < nct; c++) {
+      const int buf = c & 1;
+      load(min(c + 1, nct - 1));
+#pragma unroll
+      for (int s = 0; s < TK / 4; s++) {
+        double a[2], b[4];
+#pragma unroll
+        for (int i = 0; i < 2; i++) a[i] = As[buf][s * 4 + kq][wave * 32 + i * 16 + col];
+#pragma unroll
+        for (int j = 0; j < 4; j++) b[j] = Bs[buf][s * 4 + kq][j * 16 + col];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+      }
+      stash(buf ^ 1);
       __syncthreads();
-      for (int i = threadIdx.x; i < TK * TM; i += 256) {
-        const int kk = i / TM, mm = i - kk * TM;
-        const int K = k0 + kk;
-        As[kk][mm] = (K < NTAPS && m0 + mm < M) ? sg.A[(int64_t)K * M + m0 + mm] : 0.0;
-      }
-      for (int i = threadIdx.x; i < TK * TN; i += 256) {
-        const int kk = i / TN, nn = i - kk * TN;
-        const int K = k0 + kk;
-        Bs[kk][nn] = (K < NTAPS && n0 + nn < Ne) ? sg.B[(int64_t)K * ldb + n0 + nn] : mkz(0, 0);
-      }
-      __syncthreads();
-#pragma unroll 4
-      for (int kk = 0; kk < TK; kk++) {
-        double a[4];
-        for (int r = 0; r < 4; r++) a[r] = As[kk][ty + 16 * r];
-        zd bv[2] = {Bs[kk][tx], Bs[kk][tx + 16]};
-        for (int r = 0; r < 4; r++)
-          for (int c = 0; c < 2; c++) {
-            acc[r][c].x = fma(a[r], bv[c].x, acc[r][c].x);
-            acc[r][c].y = fma(a[r], bv[c].y, acc[r][c].y);
-          }
-      }
     }
   }
-  for (int r = 0; r < 4; r++)
-    for (int c = 0; c < 2; c++) {
-      const int64_t m = m0 + ty + 16 * r;
-      const int n = n0 + tx + 16 * c;
-      if (m < M && n < Ne) C[m * BS + coff + n] = acc[r][c] * scale;
+  // lane (col, kq) holds real column 16 j + col of offsets 16 i + kq + 4 q
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int r = wave * 32 + i * 16 + kq + 4 * q;
+      if (mo[r] < 0) continue;
+      double* d0 = !TRI || job.coff >= 0 ? reinterpret_cast<double*>(C + mo[r] * BS + job.coff + n0) + col : nullptr;
+      double* d1 =
+          TRI && job.coff2 >= 0 && mt[r] >= 0 ? reinterpret_cast<double*>(C + mt[r] * BS + job.coff2 + n0) + col : nullptr;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        if (n0 + j * 8 + (col >> 1) >= job.Ne) continue;
+        const double v = acc[i][j][q] * scale;
+        if (!TRI || d0) d0[j * 16] = v;
+        if (TRI && d1) d1[j * 16] = v;
+      }
     }
+}
+static dim3 wgemm_grid(int64_t rows, const WJobs& w) {
+  unsigned nt = 0;
+  for (int i = 0; i < w.n; i++) nt += (unsigned)((w.j[i].Ne + 31) / 32);
+  return dim3((unsigned)((rows + 127) / 128), nt);
 }
 
 // ------------------------------------------------------------ tensor FFT ---
@@ -551,7 +665,12 @@ template <int L> constexpr int ne_for() { return L <= 64 ? 32 : (L <= 128 ? 16 :
 
 // AXIS 0: transform along y for a fixed lx (blockIdx.x); AXIS 1: along x for fixed ky.
 // L is the buffer capacity; with RT the transform length is plan.L <= L.
-template <int L, int AXIS, bool RT = false>
+// MIR (the half tensor of op_build_tensor): yy and yz are xx and xz with the
+// axes exchanged, so only xx, xy, zz and xz are read and transformed, and the
+// second pass stores xx and xz of (kx,ky) also as yy and yz of (ky,kx): 0.72
+// of the bytes.  HBM bound (128x128x32: 1180 -> 790 us for the two passes,
+// 4.0 TB/s).
+template <int L, int AXIS, bool RT, bool MIR>
 __global__ __launch_bounds__(256) void k_tfft(zd* __restrict__ G, const zd* __restrict__ twg,
                                               int Nx, int Ny, int Nz, int64_t BS, FftPlan plan) {
   constexpr int NE = ne_for<L>(), LS = L + 1;
@@ -561,16 +680,18 @@ __global__ __launch_bounds__(256) void k_tfft(zd* __restrict__ G, const zd* __re
   const int N = Lr / 2;  // Ny (AXIS 0) or Nx (AXIS 1)
   const int fixed = blockIdx.x;
   const int64_t e0 = (int64_t)blockIdx.y * NE;
+  const int64_t P = (int64_t)Nz * (Nz + 1) / 2, NN = (int64_t)Nz * Nz, ne = MIR ? 3 * P + NN : BS;
   for (int i = threadIdx.x; i < Lr; i += 256) tw[i] = twg[i];
   auto gidx = [&](int l) -> int64_t {
     return AXIS == 0 ? ((int64_t)fixed + (int64_t)Nx * l) * BS : ((int64_t)l + (int64_t)Nx * fixed) * BS;
   };
+  auto entry = [&](int64_t e) -> int64_t { return MIR && e >= 2 * P ? e + P : e; };
   for (int i = threadIdx.x; i < NE * N; i += 256) {
     const int l = i / NE, s = i - l * NE;
-    const int64_t e = e0 + s;
     zd g = mkz(0, 0);
     double sx = 1, sy = 1;
-    if (e < BS) {
+    if (e0 + s < ne) {
+      const int64_t e = entry(e0 + s);
       g = G[gidx(l) + e];
       entry_signs(Nz, e, &sx, &sy);
     }
@@ -583,11 +704,16 @@ __global__ __launch_bounds__(256) void k_tfft(zd* __restrict__ G, const zd* __re
   lds_fft_any<zd, L, NE, LS, 256, -1, RT>(buf, tw, plan);
   for (int i = threadIdx.x; i < NE * N; i += 256) {
     const int k = i / NE, s = i - k * NE;
-    const int64_t e = e0 + s;
-    if (e < BS) {
+    if (e0 + s < ne) {
+      const int64_t e = entry(e0 + s);
       const zd t = buf[s * LS + N];
       const double sg = (k & 1) ? -1.0 : 1.0;
-      G[gidx(k) + e] = buf[s * LS + k] - t * sg;
+      const zd r = buf[s * LS + k] - t * sg;
+      G[gidx(k) + e] = r;
+      if constexpr (MIR && AXIS == 1) {
+        if (e < P) G[((int64_t)fixed + (int64_t)Nx * k) * BS + e + 2 * P] = r;
+        else if (e >= 4 * P) G[((int64_t)fixed + (int64_t)Nx * k) * BS + e + NN] = r;
+      }
     }
   }
 }
@@ -603,23 +729,28 @@ static void make_tw64(int L, int dir, zd** d) {
   G2G_HIP(hipMemcpy(*d, h.data(), sizeof(zd) * L, hipMemcpyHostToDevice));
 }
 
-void op_tensor_fft(Operator& op, zd* G) {
+void op_tensor_fft(Operator& op, zd* G, bool mir) {
   const int Nx2 = 2 * op.Nx, Ny2 = 2 * op.Ny;
   zd *twx, *twy;
   make_tw64(Nx2, -1, &twx);
   make_tw64(Ny2, -1, &twy);
   const FftPlan py = fft_plan(Ny2), px = fft_plan(Nx2);
-  len_dispatch(Ny2, [&](auto LC) {
-    constexpr int LL = decltype(LC)::value;
+  const int64_t P = (int64_t)op.Nz * (op.Nz + 1) / 2, ne = mir ? 3 * P + (int64_t)op.Nz * op.Nz : op.BS;
+  auto pass = [&](auto LC, auto AX, auto MR, const zd* tw, const FftPlan& plan) {
+    constexpr int LL = decltype(LC)::value, axis = decltype(AX)::value;
     constexpr int NE = ne_for<LL>();
-    hipLaunchKernelGGL((k_tfft<LL, 0, decltype(LC)::rt>), dim3(op.Nx, (unsigned)((op.BS + NE - 1) / NE)),
-                       dim3(256), 0, op.stream, G, twy, op.Nx, op.Ny, op.Nz, op.BS, py);
+    hipLaunchKernelGGL((k_tfft<LL, axis, decltype(LC)::rt, decltype(MR)::value>),
+                       dim3(axis == 0 ? op.Nx : op.Ny, (unsigned)((ne + NE - 1) / NE)), dim3(256), 0, op.stream, G, tw,
+                       op.Nx, op.Ny, op.Nz, op.BS, plan);
+  };
+  using std::integral_constant;
+  len_dispatch(Ny2, [&](auto LC) {
+    if (mir) pass(LC, integral_constant<int, 0>{}, std::true_type{}, twy, py);
+    else pass(LC, integral_constant<int, 0>{}, std::false_type{}, twy, py);
   });
   len_dispatch(Nx2, [&](auto LC) {
-    constexpr int LL = decltype(LC)::value;
-    constexpr int NE = ne_for<LL>();
-    hipLaunchKernelGGL((k_tfft<LL, 1, decltype(LC)::rt>), dim3(op.Ny, (unsigned)((op.BS + NE - 1) / NE)),
-                       dim3(256), 0, op.stream, G, twx, op.Nx, op.Ny, op.Nz, op.BS, px);
+    if (mir) pass(LC, integral_constant<int, 1>{}, std::true_type{}, twx, px);
+    else pass(LC, integral_constant<int, 1>{}, std::false_type{}, twx, px);
   });
   G2G_HIP(hipGetLastError());
   G2G_HIP(hipStreamSynchronize(op.stream));
@@ -635,7 +766,7 @@ void op_free_tensor_scratch(Operator& op) {
   op.have_wts = false;
 }
 
-void op_build_tensor(Operator& op) {
+void op_build_tensor(Operator& op, bool half) {
   G2G_CHECK(op.have_bkg, -4, "background not set");
   G2G_CHECK(op.Nl <= 64 && op.Nz <= MAX_NZ, -3, "tensor build supports Nl <= 64 and Nz <= 256");
   const int64_t M = (int64_t)op.Nx * op.Ny;
@@ -654,10 +785,12 @@ void op_build_tensor(Operator& op) {
     zd *tw, *f1;
     make_tw64(VBN, -1, &tw);
     G2G_HIP(hipMalloc(&f1, sizeof(zd) * VBN));
-    if (!op.wts) G2G_HIP(hipMalloc(&op.wts, sizeof(double) * 6 * NTAPS * M));
+    // the weights, then every offset's window of taps
+    if (!op.wts) G2G_HIP(hipMalloc(&op.wts, sizeof(double) * 6 * NTAPS * M + sizeof(int2) * M));
     hipLaunchKernelGGL(k_f1, dim3(1), dim3(256), 0, op.stream, f1, tw);
     WParams wp{op.Nx, op.Ny, op.dx, op.dy, rmin, std::log(rmin)};
-    hipLaunchKernelGGL(k_weights, dim3((unsigned)M), dim3(256), 0, op.stream, op.wts, f1, tw, d_lms, wp);
+    hipLaunchKernelGGL(k_weights, dim3((unsigned)M), dim3(256), 0, op.stream, op.wts,
+                       (int2*)(op.wts + 6 * NTAPS * M), f1, tw, d_lms, wp);
     G2G_HIP(hipGetLastError());
     G2G_HIP(hipStreamSynchronize(op.stream));
     (void)hipFree(tw);
@@ -714,19 +847,26 @@ void op_build_tensor(Operator& op) {
   const double* W = op.wts;
   auto Wc = [&](int c) { return W + (int64_t)c * NTAPS * M; };
   const double scale = 1.0 / PI_D / 4.0;
-  struct Job { int coff, Ne, nseg; GemmSeg a, b; };
-  const Job jobs[6] = {
-      {0, P, 2, {Wc(IE_DXX), T}, {Wc(IE_D0), T + P}},
-      {P, P, 1, {Wc(IE_DXY), T}, {nullptr, nullptr}},
-      {2 * P, P, 2, {Wc(IE_DYY), T}, {Wc(IE_D0), T + P}},
-      {3 * P, P, 1, {Wc(IE_D0), T + 2 * P}, {nullptr, nullptr}},
-      {4 * P, Nz * Nz, 1, {Wc(IE_DX), T + 3 * P}, {nullptr, nullptr}},
-      {4 * P + Nz * Nz, Nz * Nz, 1, {Wc(IE_DY), T + 3 * P}, {nullptr, nullptr}},
-  };
-  for (const Job& j : jobs) {
-    dim3 grid((unsigned)((M + 63) / 64), (unsigned)((j.Ne + 31) / 32));
-    hipLaunchKernelGGL(k_wgemm, grid, dim3(256), 0, op.stream, op.d64.G, M, op.BS, j.coff, j.Ne, ldb,
-                       j.a, j.b, j.nseg, scale);
+  const int NN = Nz * Nz, xz = 4 * P, yz = 4 * P + NN;
+  // half: only xx, xy, zz and xz, summed for the offsets lx >= ly and stored
+  // at both places of the x-y mirror (the sums of yy and yz at (lx,ly) are xx
+  // and xz at (ly,lx)); these blocks differ from sums of their own by the
+  // weights' rounding, as the mirrored contraction's do
+  const WJobs jobs = {6,
+                      {{0, -1, P, 2, Wc(IE_DXX), Wc(IE_D0), T, T + P},
+                       {P, P, P, 1, Wc(IE_DXY), nullptr, T, nullptr},
+                       {half ? -1 : 2 * P, 0, P, 2, Wc(IE_DYY), Wc(IE_D0), T, T + P},
+                       {3 * P, 3 * P, P, 1, Wc(IE_D0), nullptr, T + 2 * P, nullptr},
+                       {xz, -1, NN, 1, Wc(IE_DX), nullptr, T + 3 * P, nullptr},
+                       {half ? -1 : yz, xz, NN, 1, Wc(IE_DY), nullptr, T + 3 * P, nullptr}}};
+  const int2* win = (const int2*)(W + 6 * NTAPS * M);
+  if (half) {
+    const int64_t rows = (int64_t)op.Nx * (op.Nx + 1) / 2;
+    hipLaunchKernelGGL(k_wgemm<true>, wgemm_grid(rows, jobs), dim3(256), 0, op.stream, op.d64.G, rows, M, op.BS, ldb, win,
+                       op.Nx, scale, jobs);
+  } else {
+    hipLaunchKernelGGL(k_wgemm<false>, wgemm_grid(M, jobs), dim3(256), 0, op.stream, op.d64.G, M, M, op.BS, ldb, win,
+                       op.Nx, scale, jobs);
   }
   G2G_HIP(hipGetLastError());
   G2G_HIP(hipEventRecord(e1, op.stream));
@@ -816,7 +956,7 @@ struct RcWParams {
 // wts[c][K][p] in IE order, masked (1e-12 of the largest weight of the
 // offset, calc_rc_tensor_module.F90:202-212) and lambda-scaled (:214-219);
 // zero on the ix = Nx and iy = Ny offsets.
-__global__ __launch_bounds__(256) void k_rc_weights(double* __restrict__ wts,
+__global__ __launch_bounds__(256) void k_rc_weights(double* __restrict__ wts, int2* __restrict__ win,
                                                     const zd* __restrict__ f1,
                                                     const zd* __restrict__ twg,
                                                     const double* __restrict__ lms, RcWParams P) {
@@ -830,6 +970,7 @@ __global__ __launch_bounds__(256) void k_rc_weights(double* __restrict__ wts,
   const int p = blockIdx.x, ix = p / Ny2, iy = p - ix * Ny2;
   if (ix == P.Nx || iy == P.Ny) {
     for (int i = threadIdx.x; i < 6 * NTAPS; i += 256) wts[(int64_t)i * NP + p] = 0.0;
+    if (threadIdx.x == 0) win[p] = make_int2(NTAPS, 0);
     return;
   }
   const int lx = ix < P.Nx ? ix : ix - 2 * P.Nx, ly = iy < P.Ny ? iy : iy - Ny2;
@@ -877,6 +1018,9 @@ __global__ __launch_bounds__(256) void k_rc_weights(double* __restrict__ wts,
   double m = 0;
   for (int i = threadIdx.x; i < 6 * NTAPS; i += 256) m = fmax(m, fabs(wt[i / NTAPS][i % NTAPS]));
   const double W0 = block_max(m, red);
+  __shared__ int kw[2];
+  if (threadIdx.x < 2) kw[threadIdx.x] = threadIdx.x == 0 ? NTAPS : 0;
+  __syncthreads();
   for (int K = threadIdx.x; K < NTAPS; K += 256) {
     double Wm = 0;
     for (int c = 0; c < 6; c++) Wm = fmax(Wm, fabs(wt[c][K] / W0));
@@ -890,7 +1034,10 @@ __global__ __launch_bounds__(256) void k_rc_weights(double* __restrict__ wts,
     o[IE_DY] = wt[IE_DY][K] * lm;
     o[IE_D0] = wt[IE_D0][K] * lm;
     for (int c = 0; c < 6; c++) wts[((int64_t)c * NTAPS + K) * NP + p] = on ? o[c] : 0.0;
+    tap_window(kw, K, on);
   }
+  __syncthreads();
+  if (threadIdx.x == 0) win[p] = make_int2(kw[0], kw[1]);
 }
 
 // kernel functions of one receiver per tap, table [K][f][z]
@@ -1072,7 +1219,7 @@ void rc_build_tensor(RcOperator& rc) {
   G2G_CHECK(op.Nl <= 64 && op.Nz <= MAX_NZ, -3, "tensor build supports Nl <= 64 and Nz <= 256");
   rc_prepare_receivers(rc);
   const int Nz = op.Nz, Nr = rc.Nr;
-  const int64_t NP = rc.NP, BS = rc.BS, WS = (int64_t)6 * NTAPS * NP;  // weights per receiver
+  const int64_t NP = rc.NP, BS = rc.BS, WS = (int64_t)6 * NTAPS * NP + NP;  // weights per receiver, then the points' windows of taps
   const double rmin = std::sqrt(op.dx * op.dx + op.dy * op.dy) / 2.0;  // :67
   std::vector<double> lms(NTAPS);
   for (int j = 0; j < NTAPS; j++) lms[j] = std::exp(VB_XI + (double)(j + NFIRST - 512) * VB_YSTEP) / rmin;
@@ -1098,7 +1245,8 @@ void rc_build_tensor(RcOperator& rc) {
   }
   auto weights = [&](int r, double* dst) {
     RcWParams wp{op.Nx, op.Ny, op.dx, op.dy, rc.xs[r], rc.ys[r], std::log(rmin)};
-    hipLaunchKernelGGL(k_rc_weights, dim3((unsigned)NP), dim3(256), 0, op.stream, dst, f1, tw, d_lms, wp);
+    hipLaunchKernelGGL(k_rc_weights, dim3((unsigned)NP), dim3(256), 0, op.stream, dst,
+                       (int2*)(dst + 6 * NTAPS * NP), f1, tw, d_lms, wp);
   };
   if (!rc.have_wts && cache)
     for (int r = 0; r < Nr; r++) weights(r, rc.wts + r * WS);
@@ -1142,30 +1290,33 @@ void rc_build_tensor(RcOperator& rc) {
     hipLaunchKernelGGL(k_rc_lambda, dim3(NTAPS), dim3(64), 0, op.stream, rc.tabs, d_lms, d_dz, d_z, d_ln, lp);
     auto Wc = [&](int c) { return W + (int64_t)c * NTAPS * NP; };
     auto Tf = [&](int f) { return (const zd*)rc.tabs + (int64_t)f * Nz; };
-    const GemmSeg none{nullptr, nullptr};
-    // Calc_Integral_U accumulation (rc_kernel_hankel_module.F90:116-145)
-    const struct { int e, nseg; GemmSeg a, b; } jobs[15] = {
-        {0, 2, {Wc(IE_D0), Tf(RF_G11)}, {Wc(IE_DXX), Tf(RF_G3DZ_G11)}},   // REXX
-        {1, 1, {Wc(IE_DXY), Tf(RF_G3DZ_G11)}, none},                      // REXY
-        {2, 1, {Wc(IE_DX), Tf(RF_G2DZ)}, none},                           // REXZ
-        {3, 2, {Wc(IE_D0), Tf(RF_G11)}, {Wc(IE_DYY), Tf(RF_G3DZ_G11)}},   // REYY
-        {4, 1, {Wc(IE_DY), Tf(RF_G2DZ)}, none},                           // REYZ
-        {5, 1, {Wc(IE_DX), Tf(RF_G2DZ0)}, none},                          // REZX
-        {6, 1, {Wc(IE_DY), Tf(RF_G2DZ0)}, none},                          // REZY
-        {7, 1, {Wc(IE_D0), Tf(RF_G2G2DZZ)}, none},                        // REZZ
-        {8, 1, {Wc(IE_DXY), Tf(RF_G3)}, none},                            // RHXX
-        {9, 2, {Wc(IE_DYY), Tf(RF_G3)}, {Wc(IE_D0), Tf(RF_NG1DZ)}},       // RHXY
-        {10, 1, {Wc(IE_DY), Tf(RF_G2)}, none},                            // RHXZ
-        {11, 2, {Wc(IE_D0), Tf(RF_G1DZ)}, {Wc(IE_DXX), Tf(RF_NG3)}},      // RHYX
-        {12, 1, {Wc(IE_DX), Tf(RF_NG2)}, none},                           // RHYZ
-        {13, 1, {Wc(IE_DY), Tf(RF_NG1)}, none},                           // RHZX
-        {14, 1, {Wc(IE_DX), Tf(RF_G1)}, none},                            // RHZY
+    auto J1 = [&](int e, int c, int f) {
+      const int o = (e * Nr + r) * Nz;
+      return WJob{o, o, Nz, 1, Wc(c), nullptr, Tf(f), nullptr};
     };
-    for (const auto& j : jobs) {
-      dim3 grid((unsigned)((NP + 63) / 64), (unsigned)((Nz + 31) / 32));
-      hipLaunchKernelGGL(k_wgemm, grid, dim3(256), 0, op.stream, rc.G, NP, BS, (int)((j.e * Nr + r) * Nz),
-                         Nz, ldb, j.a, j.b, j.nseg, scale);
-    }
+    auto J2 = [&](int e, int c, int f, int c2, int f2) {
+      const int o = (e * Nr + r) * Nz;
+      return WJob{o, o, Nz, 2, Wc(c), Wc(c2), Tf(f), Tf(f2)};
+    };
+    // Calc_Integral_U accumulation (rc_kernel_hankel_module.F90:116-145)
+    const WJobs jobs = {15,
+                        {J2(0, IE_D0, RF_G11, IE_DXX, RF_G3DZ_G11),   // REXX
+                         J1(1, IE_DXY, RF_G3DZ_G11),                  // REXY
+                         J1(2, IE_DX, RF_G2DZ),                       // REXZ
+                         J2(3, IE_D0, RF_G11, IE_DYY, RF_G3DZ_G11),   // REYY
+                         J1(4, IE_DY, RF_G2DZ),                       // REYZ
+                         J1(5, IE_DX, RF_G2DZ0),                      // REZX
+                         J1(6, IE_DY, RF_G2DZ0),                      // REZY
+                         J1(7, IE_D0, RF_G2G2DZZ),                    // REZZ
+                         J1(8, IE_DXY, RF_G3),                        // RHXX
+                         J2(9, IE_DYY, RF_G3, IE_D0, RF_NG1DZ),       // RHXY
+                         J1(10, IE_DY, RF_G2),                        // RHXZ
+                         J2(11, IE_D0, RF_G1DZ, IE_DXX, RF_NG3),      // RHYX
+                         J1(12, IE_DX, RF_NG2),                       // RHYZ
+                         J1(13, IE_DY, RF_NG1),                       // RHZX
+                         J1(14, IE_DX, RF_G1)}};                      // RHZY
+    hipLaunchKernelGGL(k_wgemm<false>, wgemm_grid(NP, jobs), dim3(256), 0, op.stream, rc.G, NP, NP, BS, ldb,
+                       (const int2*)(W + 6 * NTAPS * NP), 0, scale, jobs);
   }
   G2G_HIP(hipGetLastError());
   G2G_HIP(hipEventRecord(e1, op.stream));

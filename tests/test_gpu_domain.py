@@ -145,3 +145,41 @@ def test_commemi3d3_lateral_grid(oracle):
     print("  apply %.2e" % e, flush=True)
     assert e < 1e-12
     op.close()
+
+
+@pytest.mark.parametrize("N,Nz", [(8, 1), (8, 3), (12, 9), (22, 17), (34, 6), (64, 33)])
+def test_half_tensor_spectrum(oracle, N, Nz):
+    """On a square grid with dx = dy a build straight to the spectrum sums the
+    offsets lx >= ly only and takes yy and yz from xx and xz with the axes
+    exchanged; the two separate stages sum every block.  Tiles of 128 offsets
+    and 32 entries with remainders in both.  Bar: the 1e-10 over the tensor
+    that the GPU tensor is held to against the oracle's (here the oracle's
+    spectrum for the small grids, the stages' for all)."""
+    from giem2g_amd import models, operator as gop
+    print("half", N, Nz, flush=True)
+    m = models.small(N, N, Nz, seed=N + Nz, freq=1.0, dz=20.0)
+    op = gop.IEOperator.from_model(m)
+    op.set_background(m.csigb(), m.thick, m.omega)
+    op.build_tensor()
+    Gb = op.get_tensor()
+    op.tensor_stage(0)
+    op.tensor_stage(1)
+    Gs = op.get_tensor()
+    e = rel(Gb, Gs)
+    print("  build against stages %.2e" % e, flush=True)
+    assert e < 1e-10
+    if N <= 12:
+        om = oracle_model(oracle, m)
+        assert rel(Gb, om.tensor_fft(om.tensor_realspace())) < 1e-10
+    # the mirror itself: xx(kx,ky) = yy(ky,kx), xz(kx,ky) = yz(ky,kx) to rounding
+    P, B = Nz * (Nz + 1) // 2, Gb.reshape(N, N, -1)
+    assert np.array_equal(B[:, :, :P], B[:, :, 2 * P:3 * P].transpose(1, 0, 2))
+    assert np.array_equal(B[:, :, 4 * P:4 * P + Nz * Nz], B[:, :, 4 * P + Nz * Nz:].transpose(1, 0, 2))
+    # no mirror where dx differs from dy
+    op.set_geometry(m.dx, 1.5 * m.dy, m.z)
+    op.build_tensor()
+    Gb = op.get_tensor()
+    op.tensor_stage(0)
+    op.tensor_stage(1)
+    assert np.array_equal(Gb, op.get_tensor())
+    op.close()
