@@ -692,156 +692,6 @@ __global__ __launch_bounds__(NT) void k_contract(cx_t<R>* __restrict__ S,
 #undef G2G_STASH
 }
 
-// Layer counts above 64 (up to MAX_NZ): the products of k_contract with
-// every tensor component staged through LDS in tiles of TJ source columns,
-// which are contiguous in the packed-upper and in the column-major storage
-// alike.  Thread (row i, part) owns receiver layer i of all four points.
-// For a symmetric component S a tile of columns [j0, j1) gives row i the
-// upper terms S(i,j) v(j), j >= i, from column j, and, when j0 <= i < j1,
-// the lower terms S(k,i) v(k), k < i, from column i; for a full component A
-// (xz, yz) row i takes A(i,j) v_z(j) of the tile's columns and, when i is in
-// the tile, the transposed terms A(k,i) v(k) over all k from column i.  So
-// every stored entry enters each product it belongs to exactly once.
-template <typename R>
-__global__ __launch_bounds__(NT) void k_contract_tiled(cx_t<R>* __restrict__ S,
-                                                       const cx_t<R>* __restrict__ G, Geo g,
-                                                       int64_t BS, int split_log, int TJ) {
-  using T2 = cx_t<R>;
-  extern __shared__ unsigned char smem_raw[];
-  const int Nz = g.Nz, Nz3 = g.Nz3;
-  const int64_t P = (int64_t)Nz * (Nz + 1) / 2;
-  T2* vin = reinterpret_cast<T2*>(smem_raw);  // [4][3Nz]
-  T2* tile = vin + 4 * Nz3;                   // at most TJ*Nz entries
-  const int b = blockIdx.x, kx = b % g.Nx, ky = b / g.Nx;
-  const int Nx2 = 2 * g.Nx, Ny2 = 2 * g.Ny;
-  const int gNx = g.Nx, gNy = g.Ny;
-#define PX(p) (((p) & 1) ? (kx == 0 ? gNx : Nx2 - kx) : kx)
-#define PY(p) (((p) & 2) ? (ky == 0 ? gNy : Ny2 - ky) : ky)
-#define VAL(p) ((!((p) & 1) || kx > 0) && (!((p) & 2) || ky > 0))
-  const T2* blk = G + (int64_t)b * BS;
-  const T2 zero = mk<T2>(0, 0);
-  for (int t = threadIdx.x; t < 4 * Nz3; t += NT) {
-    const int p = t / Nz3, e = t - p * Nz3;
-    T2 vv = zero;
-    if (VAL(p)) vv = S[((int64_t)PX(p) * Ny2 + PY(p)) * Nz3 + e];
-    vin[t] = vv;
-  }
-  const int split = 1 << split_log;
-  const int part = threadIdx.x & (split - 1);
-  const int i = threadIdx.x >> split_log;
-  const bool active = i < Nz;
-#define G2G_SG(p) (((p) & 1) ? R(-1) : R(1))
-#define G2G_MR(p) (((p) & 2) ? R(-1) : R(1))
-#define G2G_ACC(p) T2 ax##p = zero, ay##p = zero, az##p = zero;
-  G2G_FOR4(G2G_ACC)
-#undef G2G_ACC
-  for (int comp = 0; comp < 6; comp++) {
-    const bool sym = comp < 4;
-    const T2* src = sym ? blk + comp * P : blk + 4 * P + (int64_t)(comp - 4) * Nz * Nz;
-    // t1: the component acting on its source (x for xx, y for xy and yy, z
-    // for zz, xz and yz); t2: xy on x, or the transposed xz / yz
-    const int off1 = comp == 0 ? 0 : (comp == 3 || comp >= 4 ? 2 * Nz : Nz);
-    const int off2 = comp == 5 ? Nz : 0;
-#define G2G_T(p) T2 t1##p = zero, t2##p = zero;
-    G2G_FOR4(G2G_T)
-#undef G2G_T
-    for (int j0 = 0; j0 < Nz; j0 += TJ) {
-      const int j1 = min(j0 + TJ, Nz);
-      const int64_t base = sym ? (int64_t)j0 * (j0 + 1) / 2 : (int64_t)j0 * Nz;
-      const int64_t len = sym ? (int64_t)j1 * (j1 + 1) / 2 - base : (int64_t)(j1 - j0) * Nz;
-      __syncthreads();  // the previous tile (and, first time, vin) is consumed / written
-      for (int64_t t = threadIdx.x; t < len; t += NT) tile[t] = ld_stream(src + base + t);
-      __syncthreads();
-      if (active) {
-        if (sym) {
-          for (int j = max(j0, i) + part; j < j1; j += split) {
-            const T2 sv = tile[i + (int64_t)j * (j + 1) / 2 - base];
-#define G2G_UP(p)                                     \
-  {                                                   \
-    const T2* v = vin + (p) * Nz3;                    \
-    cmac(t1##p, sv, v[off1 + j]);                     \
-    if (comp == 1) cmac(t2##p, sv, v[j]);             \
-  }
-            G2G_FOR4(G2G_UP)
-#undef G2G_UP
-          }
-          if (i >= j0 && i < j1) {
-            const T2* col = tile + (int64_t)i * (i + 1) / 2 - base;
-            for (int k = part; k < i; k += split) {
-              const T2 sv = col[k];
-#define G2G_LO(p)                                     \
-  {                                                   \
-    const T2* v = vin + (p) * Nz3;                    \
-    cmac(t1##p, sv, v[off1 + k]);                     \
-    if (comp == 1) cmac(t2##p, sv, v[k]);             \
-  }
-              G2G_FOR4(G2G_LO)
-#undef G2G_LO
-            }
-          }
-        } else {
-          for (int j = j0 + part; j < j1; j += split) {
-            const T2 a = tile[(int64_t)(j - j0) * Nz + i];  // A(i,j)
-#define G2G_AF(p) cmac(t1##p, a, vin[(p) * Nz3 + off1 + j]);
-            G2G_FOR4(G2G_AF)
-#undef G2G_AF
-          }
-          if (i >= j0 && i < j1) {
-            const T2* col = tile + (int64_t)(i - j0) * Nz;
-            for (int k = part; k < Nz; k += split) {
-              const T2 at = col[k];  // A(k,i)
-#define G2G_AT(p) cmac(t2##p, at, vin[(p) * Nz3 + off2 + k]);
-              G2G_FOR4(G2G_AT)
-#undef G2G_AT
-            }
-          }
-        }
-      }
-    }
-#define G2G_FOLD(p)                                                  \
-  if (comp == 0) ax##p = ax##p + t1##p;                              \
-  else if (comp == 1) {                                              \
-    ax##p = ax##p + t1##p * (G2G_SG(p) * G2G_MR(p));                 \
-    ay##p = ay##p + t2##p * (G2G_SG(p) * G2G_MR(p));                 \
-  } else if (comp == 2) ay##p = ay##p + t1##p;                       \
-  else if (comp == 3) az##p = az##p + t1##p;                         \
-  else if (comp == 4) {                                              \
-    ax##p = ax##p + t1##p * G2G_SG(p);                               \
-    az##p = az##p - t2##p * G2G_SG(p);                               \
-  } else {                                                           \
-    ay##p = ay##p + t1##p * G2G_MR(p);                               \
-    az##p = az##p - t2##p * G2G_MR(p);                               \
-  }
-    G2G_FOR4(G2G_FOLD)
-#undef G2G_FOLD
-  }
-  for (int o = 1; o < split; o <<= 1) {
-#define G2G_RED(p)                                                       \
-  ax##p.x += __shfl_xor(ax##p.x, o); ax##p.y += __shfl_xor(ax##p.y, o);  \
-  ay##p.x += __shfl_xor(ay##p.x, o); ay##p.y += __shfl_xor(ay##p.y, o);  \
-  az##p.x += __shfl_xor(az##p.x, o); az##p.y += __shfl_xor(az##p.y, o);
-    G2G_FOR4(G2G_RED)
-#undef G2G_RED
-  }
-  if (active && part == 0) {
-#define G2G_OUT(p)                                                  \
-  {                                                                 \
-    T2* dst = S + ((int64_t)PX(p) * Ny2 + PY(p)) * Nz3;             \
-    if (!VAL(p)) ax##p = ay##p = az##p = zero;                      \
-    dst[i] = ax##p;                                                 \
-    dst[Nz + i] = ay##p;                                            \
-    dst[2 * Nz + i] = az##p;                                        \
-  }
-    G2G_FOR4(G2G_OUT)
-#undef G2G_OUT
-  }
-#undef G2G_SG
-#undef G2G_MR
-#undef PX
-#undef PY
-#undef VAL
-}
-
 // Two-deep variant of k_contract: two tensor components in flight in
 // registers while a third is computed from LDS.
 // NZT > 0: Nz known at compile time (a power of two dividing NTC, with
@@ -1043,6 +893,248 @@ __device__ inline v4t<float>::t mma4(float a, float b, v4t<float>::t c) {
 template <typename R> __device__ inline int mma_row(int kq, int q);
 template <> __device__ inline int mma_row<float>(int kq, int q) { return 4 * kq + q; }
 template <> __device__ inline int mma_row<double>(int kq, int q) { return kq + 4 * q; }
+
+// ---------------------------------------- K3 above 64 layers: strips ----
+// out_p = D_p G0 (D_p v_p) for 64 < Nz <= 16 NTM, whose tensor blocks (FP64: 0.9
+// MB at Nz = 118) fit no LDS.  One workgroup per (kx,ky) block streams it in
+// strips of CW source columns, one component after the other: the columns come
+// from HBM whole (contiguous: 16x16 tiles loaded by the waves that use them
+// fetched 1.65 times the tensor, half a cache line too much at each end of
+// their 256-byte rows), by way of registers (two chunks ahead) into one of two LDS
+// buffers.  Wave r owns receiver layers 16 r .. 16 r + 15 and uses each element
+// of its rows in both places that it stands for:
+//   - as stored: out[r] += G(r, strip) v[strip], in registers to the end;
+//   - transposed (S(j,i) = S(i,j); -A^T of xz, yz): out[strip] += G^T v[r], summed
+//     over the waves in a fixed order when the strip's six components are done.
+// Operand columns as in k_contract3 (4 points x Re, Im; G's real and imaginary
+// parts one product each); xy fills all sixteen with v_y -> x and v_x -> y.
+// Layers past Nz have zero inputs and no output.  The column stride of an odd
+// number of elements keeps both kinds of operand reads free of bank conflicts.
+// Bound by the chain of each chunk (LDS reads, then 16 matrix products a wave,
+// then the barrier): 10.0 ms of 10.9 without the loads, 7.9 ms without the
+// products (176x224x118 FP64, 35.3 GB, 3.3 TB/s; a vector-ALU kernel that staged
+// tiles of columns for the whole block, where a tile's transposed products all
+// fell to the tile's own rows: 49 ms).  Measured and not taken: 16 waves with
+// one kind of product each (11.4 ms), alternating the two kinds' products (11.0).
+template <typename R, int NTM> struct StripCfg {
+  static constexpr int CW = NTM <= 8 ? 16 : 8;      // columns per strip
+  static constexpr int ROWS = 16 * NTM, CS = ROWS + 1;
+  static constexpr int NTH = 64 * NTM, LD = CW * ROWS / NTH;  // loads per thread and chunk
+  static constexpr size_t buf_bytes = sizeof(cx_t<R>) * CW * CS, vec_bytes = sizeof(R) * 3 * ROWS * 8;
+  static constexpr size_t smem = 2 * buf_bytes + vec_bytes;
+  static_assert(sizeof(R) * NTM * 4 * CW * 8 <= buf_bytes, "the strip's partial sums use a buffer");
+};
+
+template <typename R, int NTM>
+__global__ __launch_bounds__(64 * NTM) void k_contract_strips(cx_t<R>* __restrict__ S, const cx_t<R>* __restrict__ G, Geo g,
+                                                              int64_t BS) {
+  using T2 = cx_t<R>;
+  using V4 = typename v4t<R>::t;
+  using C = StripCfg<R, NTM>;
+  constexpr int CW = C::CW, ROWS = C::ROWS, CS = C::CS, NTH = C::NTH, LD = C::LD, KS = CW / 4;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T2* buf = reinterpret_cast<T2*>(smem_raw);                       // [2][CW][CS]
+  R* vL = reinterpret_cast<R*>(smem_raw + 2 * C::buf_bytes);       // [3][ROWS][8], point-signed inputs
+  R* oL = vL;  // the strips' sums take the place of the strip's inputs, which its last chunk has used
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, kq = lane >> 4;
+  const int Nz = g.Nz, Nz3 = g.Nz3, nt = (Nz + 15) >> 4, ns = (Nz + CW - 1) / CW;
+  const int kx = blockIdx.x / g.Ny, ky = blockIdx.x - kx * g.Ny;
+  const int Nx2 = 2 * g.Nx, Ny2 = 2 * g.Ny, gNx = g.Nx, gNy = g.Ny;
+#define PX(p) (((p) & 1) ? (kx == 0 ? gNx : Nx2 - kx) : kx)
+#define PY(p) (((p) & 2) ? (ky == 0 ? gNy : Ny2 - ky) : ky)
+#define VAL(p) ((!((p) & 1) || kx > 0) && (!((p) & 2) || ky > 0))
+#define SGN(p, c) ((((c) == 0 && ((p) & 1)) || ((c) == 1 && ((p) & 2))) ? R(-1) : R(1))
+  const T2* blk = G + ((int64_t)kx + (int64_t)g.Nx * ky) * BS;
+  const int P = Nz * (Nz + 1) / 2;
+  // Chunk (strip, component): LD elements of this thread, row e % ROWS of
+  // column e / ROWS.  Rows past the column's end (and columns past Nz) repeat
+  // an element of it: they meet zero inputs or give no output.
+  auto load = [&](T2 (&d)[LD], int s, int c) {
+    const T2* src = blk + (c < 4 ? c * P : 4 * P + (c - 4) * Nz * Nz);
+#pragma unroll
+    for (int u = 0; u < LD; u++) {
+      const int e = tid + u * NTH, j = min(s * CW + e / ROWS, Nz - 1), i = e % ROWS;
+      d[u] = ld_stream(src + (c < 4 ? j * (j + 1) / 2 + min(i, j) : j * Nz + min(i, Nz - 1)));
+    }
+  };
+  auto stash = [&](const T2 (&d)[LD], int b) {
+#pragma unroll
+    for (int u = 0; u < LD; u++) {
+      const int e = tid + u * NTH;
+      buf[b * CW * CS + e / ROWS * CS + e % ROWS] = d[u];
+    }
+  };
+  // components in the order of the strips' chunks (even and odd ones use
+  // buffers and registers 0 and 1)
+  constexpr int ORD[6] = {0, 4, 2, 5, 3, 1};
+  T2 r0[LD], r1[LD];
+  load(r0, 0, ORD[0]);
+  load(r1, 0, ORD[1]);
+  for (int t = tid; t < 12 * ROWS; t += NTH) {
+    const int z = t % ROWS, q = t / ROWS, c = q % 3, p = q / 3;
+    T2 v = mk<T2>(0, 0);
+    if (z < Nz && VAL(p)) v = S[((int64_t)PX(p) * Ny2 + PY(p)) * Nz3 + c * Nz + z] * SGN(p, c);
+    vL[(c * ROWS + z) * 8 + p * 2] = v.x;
+    vL[(c * ROWS + z) * 8 + p * 2 + 1] = v.y;
+  }
+  stash(r0, 0);
+  __syncthreads();
+  const int n = col & 7;
+  const R s2 = (n & 1) ? R(1) : R(-1);  // sign of the Gi product's operand
+  const V4 zero4 = {0, 0, 0, 0};
+  V4 oX = zero4, oY = zero4, oZ = zero4, oXY = zero4;      // sums of the wave's own layers
+  V4 tX = zero4, tY = zero4, tZ = zero4, tN = zero4, tXY = zero4;  // its share of the strip's
+  // inputs of the wave's own layers, operand of the transposed products
+  R w1[3][4], w2[3][4];
+#pragma unroll
+  for (int c = 0; c < 3; c++)
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const R* v = vL + (c * ROWS + wave * 16 + 4 * k + kq) * 8;
+      w1[c][k] = v[n];
+      w2[c][k] = s2 * v[n ^ 1];
+    }
+  // D += (wave's rows of the chunk) v[strip]; columns past the eighth take input comp2
+  auto direct = [&](int b, int s, bool dia, int comp, int comp2, V4& D) {
+    const R* v = vL + ((col < 8 ? comp : comp2) * ROWS + s * CW + kq) * 8;
+    const T2* bp = buf + b * CW * CS;
+#pragma unroll
+    for (int k = 0; k < KS; k++) {
+      int r = wave * 16 + col, j = 4 * k + kq;
+      const bool below = dia && r > s * CW + j;  // below the diagonal: the element's mirror image
+      const int jj = r - s * CW;
+      const bool there = CW == 16 || !below || jj < CW;  // in this strip, or a later strip's transposed product
+      if (below && there) {
+        r = s * CW + j;
+        j = jj;
+      }
+      T2 a = bp[j * CS + r];
+      if (!there) a = mk<T2>(0, 0);
+      D = mma4(a.x, v[4 * k * 8 + n], D);
+      D = mma4(a.y, s2 * v[4 * k * 8 + (n ^ 1)], D);
+    }
+  };
+  // D += (wave's rows of the chunk, those below row lim)^T v[wave]
+  auto transposed = [&](int b, int lim, int comp, int comp2, V4& D) {
+    const T2* bp = buf + b * CW * CS + (CW == 16 ? col : (col & 7)) * CS + wave * 16 + kq;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      T2 a = bp[4 * k];
+      if (CW < 16 && wave * 16 + 4 * k + kq >= lim) a = mk<T2>(0, 0);
+      D = mma4(a.x, col < 8 ? w1[comp][k] : w1[comp2][k], D);
+      D = mma4(a.y, col < 8 ? w2[comp][k] : w2[comp2][k], D);
+    }
+  };
+  // one chunk: its products, with the loads of the chunk after the next before
+  // them and the next chunk's way into LDS after them
+  auto chunk = [&](int q, int s, T2 (&ra)[LD], T2 (&rb)[LD]) {
+    const int b = q & 1, c = ORD[q];
+    const int qn = q + 2 < 6 ? q + 2 : q - 4, sn = q + 2 < 6 ? s : s + 1;
+    if (sn < ns) load(ra, sn, ORD[qn]);
+    const int d = s * CW >> 4;  // row tile of the strip's diagonal
+    if (wave < nt && (c >= 4 || wave <= d)) {
+      const bool dia = c < 4 && wave == d;
+      // (strips of 8: the second one of a diagonal tile has 8 rows of the tile above it)
+      const bool tr = c >= 4 || wave < d || (CW < 16 && (s & 1));
+      const int lim = c >= 4 ? ROWS : s * CW;
+      if (c == 0) {
+        direct(b, s, dia, 0, 0, oX);
+        if (tr) transposed(b, lim, 0, 0, tX);
+      } else if (c == 2) {
+        direct(b, s, dia, 1, 1, oY);
+        if (tr) transposed(b, lim, 1, 1, tY);
+      } else if (c == 3) {
+        direct(b, s, dia, 2, 2, oZ);
+        if (tr) transposed(b, lim, 2, 2, tZ);
+      } else if (c == 1) {
+        direct(b, s, dia, 1, 0, oXY);
+        if (tr) transposed(b, lim, 1, 0, tXY);
+      } else if (c == 4) {
+        direct(b, s, false, 2, 2, oX);
+        transposed(b, lim, 0, 0, tN);
+      } else {
+        direct(b, s, false, 2, 2, oY);
+        transposed(b, lim, 1, 1, tN);
+      }
+    }
+    if (q < 5 || s + 1 < ns) stash(rb, b ^ 1);
+    __syncthreads();
+  };
+  for (int s = 0; s < ns; s++) {
+    chunk(0, s, r0, r1);
+    chunk(1, s, r1, r0);
+    chunk(2, s, r0, r1);
+    chunk(3, s, r1, r0);
+    chunk(4, s, r0, r1);
+    chunk(5, s, r1, r0);
+    // the waves' shares, by way of the buffer that chunk 5 has left: [wave][x, y, z, y of xy][layer][8]
+    R* red = reinterpret_cast<R*>(buf + CW * CS);
+    tZ -= tN;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int row = mma_row<R>(kq, k);
+      R* d = red + (wave * 4 * CW + row) * 8 + n;
+      if (row < CW) {
+        if (col < 8) {
+          d[0] = tX[k] + tXY[k];
+          d[CW * 8] = tY[k];
+          d[2 * CW * 8] = tZ[k];
+        } else {
+          d[3 * CW * 8] = tXY[k];
+        }
+      }
+    }
+    tX = tY = tZ = tN = tXY = zero4;
+    __syncthreads();
+    for (int t = tid; t < 3 * CW * 8; t += NTH) {
+      const int c = t / (CW * 8), e = t - c * CW * 8;
+      R sum = 0;
+      for (int w = 0; w < nt; w++) {
+        const R* d = red + w * 4 * CW * 8 + e;
+        sum += c == 1 ? d[CW * 8] + d[3 * CW * 8] : d[c * CW * 8];
+      }
+      oL[(c * ROWS + s * CW) * 8 + e] = sum;
+    }
+    __syncthreads();
+  }
+  if (wave < nt) {
+    R* o = oL + wave * 16 * 8 + n;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int row = mma_row<R>(kq, k) * 8;
+      if (col < 8) {
+        o[row] += oX[k] + oXY[k];
+        o[2 * ROWS * 8 + row] += oZ[k];
+        o[ROWS * 8 + row] += oY[k];
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (col >= 8) o[ROWS * 8 + mma_row<R>(kq, k) * 8] += oXY[k];
+  }
+  __syncthreads();
+  for (int t = tid; t < 12 * Nz; t += NTH) {
+    const int z = t % Nz, q = t / Nz, c = q % 3, p = q / 3;
+    const R* o = oL + (c * ROWS + z) * 8 + p * 2;
+    T2 v = mk<T2>(o[0], o[1]) * SGN(p, c);
+    if (!VAL(p)) v = mk<T2>(0, 0);
+    S[((int64_t)PX(p) * Ny2 + PY(p)) * Nz3 + c * Nz + z] = v;
+  }
+#undef PX
+#undef PY
+#undef VAL
+#undef SGN
+}
+
+template <typename R> void launch_strips(const Operator& op, const cx_t<R>* G, cx_t<R>* S, const Geo& g, hipStream_t s) {
+  auto go = [&](auto kern, size_t sm, int nth) {
+    G2G_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
+    hipLaunchKernelGGL(kern, dim3(op.Nx * op.Ny), dim3(nth), sm, s, S, G, g, op.BS);
+  };
+  if (op.Nz <= 128) go(k_contract_strips<R, 8>, StripCfg<R, 8>::smem, 512);
+  else go(k_contract_strips<R, 16>, StripCfg<R, 16>::smem, 1024);
+}
 
 // The work of every tensor component is spread over all NW waves: wave w
 // takes the source layers [w Nz/NW, (w+1) Nz/NW) of every output tile, so
@@ -2026,16 +2118,7 @@ void op_apply(Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* vout, 
   if (timed) G2G_HIP(hipEventRecord(op.ev[1], s));
   if (prof) pe[1] = op.prof.record(s);
   if (op.Nz > 64) {
-    // tiles of TJ source columns; the four points' rows and one tile in LDS
-    int split_log = 0;
-    while ((op.Nz << (split_log + 1)) <= NT) split_log++;
-    const size_t es = sizeof(cx_t<R>), vb = es * 4 * (size_t)Nz3;
-    const int TJ = (int)std::max<size_t>(4, std::min<size_t>(32, (96 * 1024 - vb) / (es * op.Nz)));
-    const size_t sm = vb + es * (size_t)TJ * op.Nz;
-    auto kern = k_contract_tiled<R>;
-    if (sm > 65536)
-      G2G_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    hipLaunchKernelGGL(kern, dim3(op.Nx * op.Ny), dim3(NT), sm, s, b.S, b.G, g, op.BS, split_log, TJ);
+    launch_strips<R>(op, b.G, b.S, g, s);
   } else {
     // vector ALU: rows = Nz layers, split lanes per row (power of two)
     int split_log = 0;

@@ -183,3 +183,34 @@ def test_half_tensor_spectrum(oracle, N, Nz):
     op.tensor_stage(1)
     assert np.array_equal(Gb, op.get_tensor())
     op.close()
+
+
+@pytest.mark.parametrize("Nx,Ny,Nz", [(8, 10, 65), (10, 8, 80), (8, 8, 113), (8, 12, 127), (8, 8, 128), (8, 10, 129),
+                                      (8, 8, 136), (8, 8, 185), (10, 8, 255)])
+def test_strip_contraction(oracle, Nx, Ny, Nz):
+    """The contraction above 64 layers at the edges of its tiles of 16 layers
+    and of its strips (16 columns up to 128 layers, 8 above): one apply on a
+    random spectrum against the oracle's, FP64 within 1e-12 and complex64
+    within 2e-6 (the bars of the applies above), and the same bits twice."""
+    torch = _torch()
+    from giem2g_amd import models, operator as gop
+    print("strips", Nx, Ny, Nz, flush=True)
+    m = models.small(Nx, Ny, Nz, seed=Nz, freq=0.8, dz=20.0)
+    om = oracle_model(oracle, m)
+    op = gop.IEOperator.from_model(m)
+    op.set_background(m.csigb(), m.thick, m.omega)
+    Gs = rand_vec(Nx * Ny * op.block_size, Nz) * (20.0 / np.sqrt(3.0 * Nz))
+    op.put_tensor(Gs, spectral=True)
+    op.set_sigma(m.csiga())
+    v = rand_vec(3 * m.ncell, Nz + 1)
+    ref = om.apply(Gs, m.csiga(), v)
+    r = op.apply_host(v)
+    vt = torch.from_numpy(v).cuda().to(torch.complex64)
+    o32 = torch.empty_like(vt)
+    op.apply_dev_f32(vt, o32)
+    op.sync()
+    e64, e32 = rel(r, ref), rel(o32.cpu().numpy().astype(np.complex128), ref)
+    print("  FP64 %.2e complex64 %.2e" % (e64, e32), flush=True)
+    assert e64 < 1e-12 and e32 < 2e-6
+    assert np.array_equal(op.apply_host(v), r)
+    op.close()
