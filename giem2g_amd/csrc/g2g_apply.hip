@@ -39,7 +39,7 @@ template <typename R> constexpr int nr_for(int L) {
 // rows per block of a pass over rows of length L: that of L's buffer
 // capacity (L itself for powers of two, the next power of two otherwise)
 template <typename R> int nr_rt(int L) { return nr_for<R>(len_capacity(L)); }
-template <typename R> int nr_half_rt(int L) { return nr_for<R>(L / 2); }
+template <typename R> int nr_half_rt(int L) { return nr_for<R>(len_capacity(L) / 2); }
 // Nz for which the matrix-core contraction of nrhs right-hand sides exists:
 // up to 64 layers for one or two, up to 32 for four or eight; at least C3_MIN_NZ
 // (a layer count that is not a multiple of 16 is padded to the next one)
@@ -48,9 +48,14 @@ inline bool c3_supported(int nz, int nrhs) { return nz >= C3_MIN_NZ && nz <= (nr
 // Half-length passes (two N-point transforms per zero-padded 2N-point one)
 // for rows of 32 points or more.  Measured against the 2N-point passes: at
 // 256x256 (512-point rows) the FP64 and complex64 passes together 15% faster,
-// at 128x128 FP64 5-7% faster and complex64 within 4%.  Powers of two only.
+// at 128x128 FP64 5-7% faster and complex64 within 4%.  Factor-plan lengths:
+// complex64 above 128 points only (148x172x27 336 -> 156 us, 96x96x32 40 -> 37 us
+// per direction, 60x60x20 18 -> 22); FP64 never (148x172x27 188 -> 197 us,
+// 38x38x32 25 -> 29 us: the passes of a half-full chip wait for each other).
 template <typename R> bool use_half_fft(int Lx, int Ly) {
-  return Lx >= 32 && Ly >= 32 && is_pow2(Lx) && is_pow2(Ly);
+  if (Lx < 32 || Ly < 32) return false;
+  if (is_pow2(Lx) && is_pow2(Ly)) return true;
+  return sizeof(R) == 4 && (Lx > Ly ? Lx : Ly) > 128;
 }
 
 struct Geo {
@@ -58,7 +63,10 @@ struct Geo {
   int nrx_log;  // X tile rows = 1 << nrx_log
   int64_t nc;   // cells
   int slot[3];
-  FftPlan px, py;  // factors of 2Nx and 2Ny (used where they are not powers of two)
+  // factors of 2Nx and 2Ny, or of Nx and Ny for the half-length passes (used
+  // where they are not powers of two), and the multiplier of i / Nx
+  FftPlan px, py;
+  unsigned mx;
   // x passes: chunks of NR rows per field component when NR divides Nz
   // (then the three components of a layer range run as consecutive blocks
   // and share the per-cell scalings in cache), else 0
@@ -111,11 +119,15 @@ __device__ inline void load_tw(T2* tw, const T2* g, int L) {
   for (int i = threadIdx.x; i < L; i += NT) tw[i] = g[i];
 }
 
+// Waves per SIMD asked of the compiler for the factor-plan passes, as many as
+// their LDS allows (complex64 148x172x27, 194x194x19: 6-8% faster than with two)
+template <typename R, int L, bool RT> constexpr int rt_waves() { return !RT ? 1 : (sizeof(R) == 8 && L >= 512 ? 3 : 4); }
+
 // ---------------------------------------------------------------- K1 ----
 // L is the buffer capacity; with RT the rows are 2Nx <= L points long
 // (a length that is not a power of two, transformed by its factor plan).
 template <typename R, int L, bool RT = false>
-__global__ __launch_bounds__(NT) void k_fwd_x(const cx_t<R>* __restrict__ v,
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_fwd_x(const cx_t<R>* __restrict__ v,
                                               const cx_t<R>* __restrict__ gsig,
                                               cx_t<R>* __restrict__ X,
                                               const cx_t<R>* __restrict__ twg, Geo g) {
@@ -128,7 +140,7 @@ __global__ __launch_bounds__(NT) void k_fwd_x(const cx_t<R>* __restrict__ v,
   const int Lr = RT ? 2 * Nx : L;
   load_tw<T2>(tw, twg, Lr);
   for (int i = threadIdx.x; i < NR * Nx; i += NT) {
-    const int s = i / Nx, x = i - s * Nx, cz = chunk * NR + s;
+    const int s = fast_div(i, Nx, g.mx), x = i - s * Nx, cz = chunk * NR + s;
     T2 val = mk<T2>(0, 0);
     if (cz < g.Nz3) {
       const int c = cz / g.Nz, z = cz - c * g.Nz;
@@ -153,7 +165,7 @@ __global__ __launch_bounds__(NT) void k_fwd_x(const cx_t<R>* __restrict__ v,
 // otherwise the x- and y-Nyquist lines, which the IE operator never uses,
 // are skipped.
 template <typename R, int L, bool FULL = false, bool RT = false>
-__global__ __launch_bounds__(NT) void k_fwd_y(const cx_t<R>* __restrict__ X,
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_fwd_y(const cx_t<R>* __restrict__ X,
                                               cx_t<R>* __restrict__ S,
                                               const cx_t<R>* __restrict__ twg, Geo g) {
   using T2 = cx_t<R>;
@@ -180,7 +192,7 @@ __global__ __launch_bounds__(NT) void k_fwd_y(const cx_t<R>* __restrict__ X,
 
 // ---------------------------------------------------------------- K4 ----
 template <typename R, int L, bool FULL = false, bool RT = false>
-__global__ __launch_bounds__(NT) void k_inv_y(const cx_t<R>* __restrict__ S,
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_inv_y(const cx_t<R>* __restrict__ S,
                                               cx_t<R>* __restrict__ X,
                                               const cx_t<R>* __restrict__ twg, Geo g) {
   using T2 = cx_t<R>;
@@ -212,7 +224,7 @@ __global__ __launch_bounds__(NT) void k_inv_y(const cx_t<R>* __restrict__ S,
 
 // ---------------------------------------------------------------- K5 ----
 template <typename R, int L, bool RT = false>
-__global__ __launch_bounds__(NT) void k_inv_x(const cx_t<R>* __restrict__ X,
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_inv_x(const cx_t<R>* __restrict__ X,
                                               const cx_t<R>* __restrict__ vin,
                                               const cx_t<R>* __restrict__ asiga,
                                               const R* __restrict__ sq,
@@ -235,7 +247,7 @@ __global__ __launch_bounds__(NT) void k_inv_x(const cx_t<R>* __restrict__ X,
   __syncthreads();
   lds_fft_any<T2, L, NR, LS, NT, +1, RT>(buf, tw, g.px);
   for (int i = threadIdx.x; i < NR * Nx; i += NT) {
-    const int s = i / Nx, x = i - s * Nx, cz = chunk * NR + s;
+    const int s = fast_div(i, Nx, g.mx), x = i - s * Nx, cz = chunk * NR + s;
     if (cz < g.Nz3) {
       const int c = cz / g.Nz, z = cz - c * g.Nz;
       const int64_t ci = ((int64_t)z * g.Ny + y) * Nx + x;
@@ -271,33 +283,34 @@ template <typename R> constexpr int ls_half(int N) { return sizeof(R) == 4 ? N +
 // them from the global table).
 template <typename R> constexpr bool wh_in_lds() { return sizeof(R) == 4; }
 
-template <typename T2, int N, bool WH>
-__device__ inline void load_tw_half(T2* twN, T2* wh, const T2* g) {
+template <typename T2, bool WH>
+__device__ inline void load_tw_half(T2* twN, T2* wh, const T2* g, int N) {
   for (int i = threadIdx.x; i < N; i += NT) {
     twN[i] = g[2 * i];  // exp(-2 pi i t/N)
     if constexpr (WH) wh[i] = g[i];
   }
 }
 
-template <typename R, int L>
-__global__ __launch_bounds__(NT) void k_fwd_x_h(const cx_t<R>* __restrict__ v,
+template <typename R, int L, bool RT = false>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_fwd_x_h(const cx_t<R>* __restrict__ v,
                                                 const cx_t<R>* __restrict__ gsig,
                                                 cx_t<R>* __restrict__ X,
                                                 const cx_t<R>* __restrict__ twg, Geo g) {
   using T2 = cx_t<R>;
-  constexpr int N = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(N), PER = (NR * N + NT - 1) / NT;
+  constexpr int NC = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(NC), PER = (NR * NC + NT - 1) / NT;
   __shared__ T2 buf[NR * LS];
-  __shared__ T2 twN[N], whs[wh_in_lds<R>() ? N : 1];
+  __shared__ T2 twN[NC], whs[wh_in_lds<R>() ? NC : 1];
+  const int N = RT ? g.Nx : NC, Lr = 2 * N;
   const T2* __restrict__ wh = wh_in_lds<R>() ? whs : twg;
-  const int y = blockIdx.x, chunk = x_chunk(g, blockIdx.y);  // Nx = N
-  load_tw_half<T2, N, wh_in_lds<R>()>(twN, whs, twg);
+  const int y = blockIdx.x, chunk = x_chunk(g, blockIdx.y);
+  load_tw_half<T2, wh_in_lds<R>()>(twN, whs, twg, N);
   T2 xin[PER];
 #pragma unroll
   for (int q = 0; q < PER; q++) {
     const int i = threadIdx.x + q * NT;
     xin[q] = mk<T2>(0, 0);
     if (i < NR * N) {
-      const int s = i / N, x = i - s * N, cz = chunk * NR + s;
+      const int s = RT ? fast_div(i, N, g.mx) : i / NC, x = i - s * N, cz = chunk * NR + s;
       if (cz < g.Nz3) {
         const int c = cz / g.Nz, z = cz - c * g.Nz;
         const int64_t ci = ((int64_t)z * g.Ny + y) * N + x;
@@ -307,12 +320,12 @@ __global__ __launch_bounds__(NT) void k_fwd_x_h(const cx_t<R>* __restrict__ v,
     }
   }
   __syncthreads();
-  lds_fft<T2, N, NR, LS, NT, -1>(buf, twN);
+  lds_fft_any<T2, NC, NR, LS, NT, -1, RT>(buf, twN, g.px);
   // X tile for this chunk: [y][kx][s].  The even kx stay in registers until
   // the odd ones are done, so the two halves of each stored pair (64 B each
   // for eight complex64 rows) reach the cache together and no line is
   // written twice
-  T2* dst = X + (((int64_t)chunk * g.Ny + y) * L) * NR;
+  T2* dst = X + (((int64_t)chunk * g.Ny + y) * Lr) * NR;
   T2 ev[PER];
 #pragma unroll
   for (int q = 0; q < PER; q++) {
@@ -328,12 +341,12 @@ __global__ __launch_bounds__(NT) void k_fwd_x_h(const cx_t<R>* __restrict__ v,
   for (int q = 0; q < PER; q++) {
     const int i = threadIdx.x + q * NT;
     if (i < NR * N) {
-      const int s = i / N, x = i - s * N;
+      const int s = RT ? fast_div(i, N, g.mx) : i / NC, x = i - s * N;
       buf[s * LS + x] = xin[q] * wh[x];
     }
   }
   __syncthreads();
-  lds_fft<T2, N, NR, LS, NT, -1>(buf, twN);
+  lds_fft_any<T2, NC, NR, LS, NT, -1, RT>(buf, twN, g.px);
 #pragma unroll
   for (int q = 0; q < PER; q++) {
     const int i = threadIdx.x + q * NT;
@@ -345,19 +358,20 @@ __global__ __launch_bounds__(NT) void k_fwd_x_h(const cx_t<R>* __restrict__ v,
   }
 }
 
-template <typename R, int L>
-__global__ __launch_bounds__(NT) void k_fwd_y_h(const cx_t<R>* __restrict__ X,
+template <typename R, int L, bool RT = false>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_fwd_y_h(const cx_t<R>* __restrict__ X,
                                                 cx_t<R>* __restrict__ S,
                                                 const cx_t<R>* __restrict__ twg, Geo g) {
   using T2 = cx_t<R>;
-  constexpr int N = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(N), PER = (NR * N + NT - 1) / NT;
+  constexpr int NC = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(NC), PER = (NR * NC + NT - 1) / NT;
   __shared__ T2 buf[NR * LS];
-  __shared__ T2 twN[N], whs[wh_in_lds<R>() ? N : 1];
+  __shared__ T2 twN[NC], whs[wh_in_lds<R>() ? NC : 1];
+  const int N = RT ? g.Ny : NC, Lr = 2 * N;
   const T2* __restrict__ wh = wh_in_lds<R>() ? whs : twg;
-  int kx, chunk;  // Ny = N
+  int kx, chunk;
   y_tile<NR * sizeof(T2) < 128>(kx, chunk);
   if (kx == g.Nx) return;  // x-Nyquist column is never used
-  load_tw_half<T2, N, wh_in_lds<R>()>(twN, whs, twg);
+  load_tw_half<T2, wh_in_lds<R>()>(twN, whs, twg, N);
   T2 xin[PER];
 #pragma unroll
   for (int q = 0; q < PER; q++) {
@@ -370,10 +384,10 @@ __global__ __launch_bounds__(NT) void k_fwd_y_h(const cx_t<R>* __restrict__ X,
     }
   }
   __syncthreads();
-  lds_fft<T2, N, NR, LS, NT, -1>(buf, twN);
+  lds_fft_any<T2, NC, NR, LS, NT, -1, RT>(buf, twN, g.py);
   for (int i = threadIdx.x; i < NR * N; i += NT) {
     const int k = i / NR, s = i - k * NR, cz = chunk * NR + s;
-    if (2 * k != N && cz < g.Nz3) S[((int64_t)kx * L + 2 * k) * g.Nz3 + cz] = buf[s * LS + k];
+    if (2 * k != N && cz < g.Nz3) S[((int64_t)kx * Lr + 2 * k) * g.Nz3 + cz] = buf[s * LS + k];
   }
   __syncthreads();
 #pragma unroll
@@ -385,23 +399,24 @@ __global__ __launch_bounds__(NT) void k_fwd_y_h(const cx_t<R>* __restrict__ X,
     }
   }
   __syncthreads();
-  lds_fft<T2, N, NR, LS, NT, -1>(buf, twN);
+  lds_fft_any<T2, NC, NR, LS, NT, -1, RT>(buf, twN, g.py);
   for (int i = threadIdx.x; i < NR * N; i += NT) {
     const int k = i / NR, s = i - k * NR, cz = chunk * NR + s;
-    if (cz < g.Nz3) S[((int64_t)kx * L + 2 * k + 1) * g.Nz3 + cz] = buf[s * LS + k];
+    if (cz < g.Nz3) S[((int64_t)kx * Lr + 2 * k + 1) * g.Nz3 + cz] = buf[s * LS + k];
   }
 }
 
-template <typename R, int L>
-__global__ __launch_bounds__(NT) void k_inv_y_h(const cx_t<R>* __restrict__ S,
+template <typename R, int L, bool RT = false>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_inv_y_h(const cx_t<R>* __restrict__ S,
                                                 cx_t<R>* __restrict__ X,
                                                 const cx_t<R>* __restrict__ twg, Geo g) {
   using T2 = cx_t<R>;
-  constexpr int N = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(N), PER = (NR * N + NT - 1) / NT;
+  constexpr int NC = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(NC), PER = (NR * NC + NT - 1) / NT;
   __shared__ T2 buf[NR * LS];
-  __shared__ T2 twN[N], whs[wh_in_lds<R>() ? N : 1];
+  __shared__ T2 twN[NC], whs[wh_in_lds<R>() ? NC : 1];
+  const int N = RT ? g.Ny : NC, Lr = 2 * N;
   const T2* __restrict__ wh = wh_in_lds<R>() ? whs : twg;
-  int kx, chunk;  // Ny = N
+  int kx, chunk;
   y_tile<NR * sizeof(T2) < 128>(kx, chunk);
   if (kx == g.Nx) {  // x-Nyquist: zero (InitialTransposeRepack, Distributed_FFT.F90:723-724)
     for (int i = threadIdx.x; i < NR * N; i += NT) {
@@ -410,13 +425,13 @@ __global__ __launch_bounds__(NT) void k_inv_y_h(const cx_t<R>* __restrict__ S,
     }
     return;
   }
-  load_tw_half<T2, N, wh_in_lds<R>()>(twN, whs, twg);
+  load_tw_half<T2, wh_in_lds<R>()>(twN, whs, twg, N);
   for (int i = threadIdx.x; i < NR * N; i += NT) {
     const int m = i / NR, s = i - m * NR, cz = chunk * NR + s;
-    buf[s * LS + m] = (cz < g.Nz3) ? S[((int64_t)kx * L + 2 * m) * g.Nz3 + cz] : mk<T2>(0, 0);
+    buf[s * LS + m] = (cz < g.Nz3) ? S[((int64_t)kx * Lr + 2 * m) * g.Nz3 + cz] : mk<T2>(0, 0);
   }
   __syncthreads();
-  lds_fft<T2, N, NR, LS, NT, +1>(buf, twN);
+  lds_fft_any<T2, NC, NR, LS, NT, +1, RT>(buf, twN, g.py);
   T2 acc[PER];
 #pragma unroll
   for (int q = 0; q < PER; q++) {
@@ -430,10 +445,10 @@ __global__ __launch_bounds__(NT) void k_inv_y_h(const cx_t<R>* __restrict__ S,
   __syncthreads();
   for (int i = threadIdx.x; i < NR * N; i += NT) {
     const int m = i / NR, s = i - m * NR, cz = chunk * NR + s;
-    buf[s * LS + m] = (cz < g.Nz3) ? S[((int64_t)kx * L + 2 * m + 1) * g.Nz3 + cz] : mk<T2>(0, 0);
+    buf[s * LS + m] = (cz < g.Nz3) ? S[((int64_t)kx * Lr + 2 * m + 1) * g.Nz3 + cz] : mk<T2>(0, 0);
   }
   __syncthreads();
-  lds_fft<T2, N, NR, LS, NT, +1>(buf, twN);
+  lds_fft_any<T2, NC, NR, LS, NT, +1, RT>(buf, twN, g.py);
 #pragma unroll
   for (int q = 0; q < PER; q++) {
     const int i = threadIdx.x + q * NT;
@@ -446,8 +461,8 @@ __global__ __launch_bounds__(NT) void k_inv_y_h(const cx_t<R>* __restrict__ S,
   }
 }
 
-template <typename R, int L>
-__global__ __launch_bounds__(NT) void k_inv_x_h(const cx_t<R>* __restrict__ X,
+template <typename R, int L, bool RT = false>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_inv_x_h(const cx_t<R>* __restrict__ X,
                                                 const cx_t<R>* __restrict__ vin,
                                                 const cx_t<R>* __restrict__ asiga,
                                                 const R* __restrict__ sq,
@@ -455,13 +470,14 @@ __global__ __launch_bounds__(NT) void k_inv_x_h(const cx_t<R>* __restrict__ X,
                                                 cx_t<R>* __restrict__ vout,
                                                 const cx_t<R>* __restrict__ twg, Geo g) {
   using T2 = cx_t<R>;
-  constexpr int N = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(N), PER = (NR * N + NT - 1) / NT;
+  constexpr int NC = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(NC), PER = (NR * NC + NT - 1) / NT;
   __shared__ T2 buf[NR * LS];
-  __shared__ T2 twN[N], whs[wh_in_lds<R>() ? N : 1];
+  __shared__ T2 twN[NC], whs[wh_in_lds<R>() ? NC : 1];
+  const int N = RT ? g.Nx : NC, Lr = 2 * N;
   const T2* __restrict__ wh = wh_in_lds<R>() ? whs : twg;
-  const int y = blockIdx.x, chunk = x_chunk(g, blockIdx.y);  // Nx = N
-  load_tw_half<T2, N, wh_in_lds<R>()>(twN, whs, twg);
-  const T2* src = X + (((int64_t)chunk * g.Ny + y) * L) * NR;
+  const int y = blockIdx.x, chunk = x_chunk(g, blockIdx.y);
+  load_tw_half<T2, wh_in_lds<R>()>(twN, whs, twg, N);
+  const T2* src = X + (((int64_t)chunk * g.Ny + y) * Lr) * NR;
   // even and odd kx of each stored pair are read together (the odd ones
   // wait in registers), so each line of X is fetched once
   T2 od[PER];
@@ -476,14 +492,14 @@ __global__ __launch_bounds__(NT) void k_inv_x_h(const cx_t<R>* __restrict__ X,
     }
   }
   __syncthreads();
-  lds_fft<T2, N, NR, LS, NT, +1>(buf, twN);
+  lds_fft_any<T2, NC, NR, LS, NT, +1, RT>(buf, twN, g.px);
   T2 acc[PER];
 #pragma unroll
   for (int q = 0; q < PER; q++) {
     const int i = threadIdx.x + q * NT;
     acc[q] = mk<T2>(0, 0);
     if (i < NR * N) {
-      const int s = i / N, x = i - s * N;
+      const int s = RT ? fast_div(i, N, g.mx) : i / NC, x = i - s * N;
       acc[q] = buf[s * LS + x];
     }
   }
@@ -497,12 +513,12 @@ __global__ __launch_bounds__(NT) void k_inv_x_h(const cx_t<R>* __restrict__ X,
     }
   }
   __syncthreads();
-  lds_fft<T2, N, NR, LS, NT, +1>(buf, twN);
+  lds_fft_any<T2, NC, NR, LS, NT, +1, RT>(buf, twN, g.px);
 #pragma unroll
   for (int q = 0; q < PER; q++) {
     const int i = threadIdx.x + q * NT;
     if (i < NR * N) {
-      const int s = i / N, x = i - s * N, cz = chunk * NR + s;
+      const int s = RT ? fast_div(i, N, g.mx) : i / NC, x = i - s * N, cz = chunk * NR + s;
       if (cz < g.Nz3) {
         T2 w = wh[x];
         w.y = -w.y;
@@ -876,23 +892,7 @@ __global__ __launch_bounds__(NTC) void k_contract2(cx_t<R>* __restrict__ S,
 // accumulate Re(G0 v_p) and columns 4-7 Im(G0 v_p) in one
 // v_mfma_{f64,f32}_16x16x4 tile; columns 8-15 carry a second right-hand
 // side (NRHS = 2: two vectors read the tensor once) or repeat the first.
-// Lane l supplies A[row l%16][k l/16] and B[k l/16][col l%16] and receives
-// four rows of column l%16 (mma_row).
-template <typename R> struct v4t;
-template <> struct v4t<double> { typedef double t __attribute__((ext_vector_type(4))); };
-template <> struct v4t<float> { typedef float t __attribute__((ext_vector_type(4))); };
-__device__ inline v4t<double>::t mma4(double a, double b, v4t<double>::t c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ inline v4t<float>::t mma4(float a, float b, v4t<float>::t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// result row of accumulator element q in lane group kq = lane/16: the FP32
-// tile holds rows 4*kq + q, the FP64 tile rows kq + 4*q (both measured)
-template <typename R> __device__ inline int mma_row(int kq, int q);
-template <> __device__ inline int mma_row<float>(int kq, int q) { return 4 * kq + q; }
-template <> __device__ inline int mma_row<double>(int kq, int q) { return kq + 4 * q; }
+// (Lane layouts: mma4, mma_row.)
 
 // ---------------------------------------- K3 above 64 layers: strips ----
 // out_p = D_p G0 (D_p v_p) for 64 < Nz <= 16 NTM, whose tensor blocks (FP64: 0.9
@@ -1987,7 +1987,7 @@ template <typename R> bool c3_auto(int nz) {
 }
 template <typename R, template <typename, int> class KF> struct Dummy {};
 
-static Geo make_geo(const Operator& op, int nrx) {
+static Geo make_geo(const Operator& op, int nrx, bool half) {
   Geo g;
   g.Nx = op.Nx;
   g.Ny = op.Ny;
@@ -1996,8 +1996,9 @@ static Geo make_geo(const Operator& op, int nrx) {
   g.nrx_log = ilog2(nrx);
   g.nc = op.ncell();
   for (int c = 0; c < 3; c++) g.slot[c] = op.comp_slot[c];
-  g.px = op.px;
-  g.py = op.py;
+  g.px = half ? op.hx : op.px;
+  g.py = half ? op.hy : op.py;
+  g.mx = div_mul(op.Nx);
   g.chz = (op.Nz % nrx == 0) ? op.Nz / nrx : 0;
   return g;
 }
@@ -2060,19 +2061,28 @@ static void fft_forward(const Operator& op, OpBuffers<R>& b, const cx_t<R>* vin,
   len_dispatch(Nx2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     constexpr bool RT = decltype(LC)::rt;
-    if (!RT && b.half)
-      hipLaunchKernelGGL((k_fwd_x_h<R, LL>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, vin, b.gsig, b.X, b.twx, g);
-    else
+    // (FP64 factor-plan rows are never half-length)
+    if constexpr (RT && sizeof(R) == 8) {
       hipLaunchKernelGGL((k_fwd_x<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, vin, b.gsig, b.X, b.twx,
                          g);
+    } else if (b.half) {
+      hipLaunchKernelGGL((k_fwd_x_h<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, vin, b.gsig, b.X, b.twx, g);
+    } else {
+      hipLaunchKernelGGL((k_fwd_x<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, vin, b.gsig, b.X, b.twx,
+                         g);
+    }
   });
   len_dispatch(Ny2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     constexpr bool RT = decltype(LC)::rt;
-    if (!RT && b.half)
-      hipLaunchKernelGGL((k_fwd_y_h<R, LL>), dim3(Nx2, chy), dim3(NT), 0, s, b.X, S, b.twy, g);
-    else
+    // (FP64 factor-plan rows are never half-length)
+    if constexpr (RT && sizeof(R) == 8) {
       hipLaunchKernelGGL((k_fwd_y<R, LL, false, RT>), dim3(Nx2, chy), dim3(NT), 0, s, b.X, S, b.twy, g);
+    } else if (b.half) {
+      hipLaunchKernelGGL((k_fwd_y_h<R, LL, RT>), dim3(Nx2, chy), dim3(NT), 0, s, b.X, S, b.twy, g);
+    } else {
+      hipLaunchKernelGGL((k_fwd_y<R, LL, false, RT>), dim3(Nx2, chy), dim3(NT), 0, s, b.X, S, b.twy, g);
+    }
   });
 }
 
@@ -2085,20 +2095,29 @@ static void fft_inverse(const Operator& op, OpBuffers<R>& b, const cx_t<R>* S, c
   len_dispatch(Ny2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     constexpr bool RT = decltype(LC)::rt;
-    if (!RT && b.half)
-      hipLaunchKernelGGL((k_inv_y_h<R, LL>), dim3(Nx2, chy), dim3(NT), 0, s, S, b.X, b.twy, g);
-    else
+    // (FP64 factor-plan rows are never half-length)
+    if constexpr (RT && sizeof(R) == 8) {
       hipLaunchKernelGGL((k_inv_y<R, LL, false, RT>), dim3(Nx2, chy), dim3(NT), 0, s, S, b.X, b.twy, g);
+    } else if (b.half) {
+      hipLaunchKernelGGL((k_inv_y_h<R, LL, RT>), dim3(Nx2, chy), dim3(NT), 0, s, S, b.X, b.twy, g);
+    } else {
+      hipLaunchKernelGGL((k_inv_y<R, LL, false, RT>), dim3(Nx2, chy), dim3(NT), 0, s, S, b.X, b.twy, g);
+    }
   });
   len_dispatch(Nx2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     constexpr bool RT = decltype(LC)::rt;
-    if (!RT && b.half)
-      hipLaunchKernelGGL((k_inv_x_h<R, LL>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, b.X, vin, b.asiga, b.sq,
-                         b.dzn, vout, b.twx, g);
-    else
+    // (FP64 factor-plan rows are never half-length)
+    if constexpr (RT && sizeof(R) == 8) {
       hipLaunchKernelGGL((k_inv_x<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, b.X, vin, b.asiga, b.sq,
                          b.dzn, vout, b.twx, g);
+    } else if (b.half) {
+      hipLaunchKernelGGL((k_inv_x_h<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, b.X, vin, b.asiga, b.sq,
+                         b.dzn, vout, b.twx, g);
+    } else {
+      hipLaunchKernelGGL((k_inv_x<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, b.X, vin, b.asiga, b.sq,
+                         b.dzn, vout, b.twx, g);
+    }
   });
 }
 
@@ -2107,7 +2126,7 @@ void op_apply(Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* vout, 
               bool timed, bool mirror) {
   G2G_CHECK(op.have_tensor && op.have_sigma, -4, "operator not ready: tensor or conductivity missing");
   const int Nz3 = 3 * op.Nz;
-  Geo g = make_geo(op, b.NR);
+  Geo g = make_geo(op, b.NR, b.half);
   // profiling: events around the three stages (flushed into op.cnt later)
   const bool prof = op.prof.on && !timed;
   const int prec = sizeof(R) == 8 ? 0 : 1;
@@ -2219,7 +2238,7 @@ static void op_apply_k(Operator& op, OpBuffers<R>& b, int k, const cx_t<R>* cons
     hipLaunchKernelGGL((k_zero<T2>), dim3((unsigned)std::min<int64_t>(4096, (nz + NT - 1) / NT)), dim3(NT), 0, s,
                        b.SB + nS * k, nz);
   }
-  Geo g = make_geo(op, b.NR);
+  Geo g = make_geo(op, b.NR, b.half);
   const bool prof = op.prof.on;
   const int prec = sizeof(R) == 8 ? 0 : 1;
   int pe[4] = {0, 0, 0, 0};
@@ -2609,7 +2628,7 @@ void rc_apply(RcOperator& rc, const zd* E, zd* Ea, zd* Ha, hipStream_t s) {
   G2G_CHECK(rc.have_sigma && rc.sigma_version == op.bkg_version, -4,
             "receiver conductivity not set for the current frequency");
   const int Nx2 = 2 * op.Nx, Ny2 = 2 * op.Ny, Nr = rc.Nr;
-  Geo gf = make_geo(op, rc.NR);
+  Geo gf = make_geo(op, rc.NR, false);
   Geo gi = gf;
   gi.Nz3 = 6 * Nr;
   const int nry = nr_rt<double>(Ny2);

@@ -118,6 +118,8 @@ void op_init(Operator& op, int Nx, int Ny, int Nz, double dx, double dy, const d
   op.BS = 4 * (int64_t)Nz * (Nz + 1) / 2 + 2 * (int64_t)Nz * Nz;
   op.px = fft_plan(2 * Nx);
   op.py = fft_plan(2 * Ny);
+  op.hx = fft_plan(Nx);
+  op.hy = fft_plan(Ny);
   op.stream = nullptr;  // the default stream orders with torch's default stream
   for (auto& e : op.ev) G2G_HIP(hipEventCreate(&e));
   op_alloc_buffers<double>(op, op.d64, true);

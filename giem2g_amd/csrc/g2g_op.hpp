@@ -179,6 +179,7 @@ struct Operator {
   std::vector<double> z, dz;
   int comp_slot[3] = {0, 1, 2};  // memory slot of physical component x,y,z
   FftPlan px, py;                // factor plans of the 2Nx- and 2Ny-point transforms
+  FftPlan hx, hy;                // and of the Nx- and Ny-point ones (half-length passes)
   // background of the current frequency
   int Nl = 0;
   double omega = 0;

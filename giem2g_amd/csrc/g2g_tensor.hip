@@ -671,9 +671,9 @@ template <int L> constexpr int ne_for() { return L <= 64 ? 32 : (L <= 128 ? 16 :
 // of the bytes.  HBM bound (128x128x32: 1180 -> 790 us for the two passes,
 // 4.0 TB/s).
 template <int L, int AXIS, bool RT, bool MIR>
-__global__ __launch_bounds__(256) void k_tfft(zd* __restrict__ G, const zd* __restrict__ twg,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT ? 2 : 1))) void k_tfft(zd* __restrict__ G, const zd* __restrict__ twg,
                                               int Nx, int Ny, int Nz, int64_t BS, FftPlan plan) {
-  constexpr int NE = ne_for<L>(), LS = L + 1;
+  constexpr int NE = ne_for<L>(), LS = L + 1, NT = 256;
   __shared__ zd buf[NE * LS];
   __shared__ zd tw[L];
   const int Lr = RT ? plan.L : L;
@@ -681,12 +681,12 @@ __global__ __launch_bounds__(256) void k_tfft(zd* __restrict__ G, const zd* __re
   const int fixed = blockIdx.x;
   const int64_t e0 = (int64_t)blockIdx.y * NE;
   const int64_t P = (int64_t)Nz * (Nz + 1) / 2, NN = (int64_t)Nz * Nz, ne = MIR ? 3 * P + NN : BS;
-  for (int i = threadIdx.x; i < Lr; i += 256) tw[i] = twg[i];
+  for (int i = threadIdx.x; i < Lr; i += NT) tw[i] = twg[i];
   auto gidx = [&](int l) -> int64_t {
     return AXIS == 0 ? ((int64_t)fixed + (int64_t)Nx * l) * BS : ((int64_t)l + (int64_t)Nx * fixed) * BS;
   };
   auto entry = [&](int64_t e) -> int64_t { return MIR && e >= 2 * P ? e + P : e; };
-  for (int i = threadIdx.x; i < NE * N; i += 256) {
+  for (int i = threadIdx.x; i < NE * N; i += NT) {
     const int l = i / NE, s = i - l * NE;
     zd g = mkz(0, 0);
     double sx = 1, sy = 1;
@@ -701,8 +701,8 @@ __global__ __launch_bounds__(256) void k_tfft(zd* __restrict__ G, const zd* __re
     else buf[s * LS + N] = mkz(0, 0);
   }
   __syncthreads();
-  lds_fft_any<zd, L, NE, LS, 256, -1, RT>(buf, tw, plan);
-  for (int i = threadIdx.x; i < NE * N; i += 256) {
+  lds_fft_any<zd, L, NE, LS, NT, -1, RT>(buf, tw, plan);
+  for (int i = threadIdx.x; i < NE * N; i += NT) {
     const int k = i / NE, s = i - k * NE;
     if (e0 + s < ne) {
       const int64_t e = entry(e0 + s);
@@ -1158,25 +1158,25 @@ __global__ __launch_bounds__(64) void k_rc_lambda(zd* __restrict__ tabs,
 // In-place forward FFT of every tensor column along y for a fixed ix
 // (AXIS 0) or along x for a fixed iy (AXIS 1), points p = ix*Ny2 + iy.
 template <int L, int AXIS, bool RT = false>
-__global__ __launch_bounds__(256) void k_rc_tfft(zd* __restrict__ G, const zd* __restrict__ twg, int Ny2,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT ? 2 : 1))) void k_rc_tfft(zd* __restrict__ G, const zd* __restrict__ twg, int Ny2,
                                                  int64_t BS, FftPlan plan) {
-  constexpr int NE = ne_for<L>(), LS = L + 1;
+  constexpr int NE = ne_for<L>(), LS = L + 1, NT = 256;
   __shared__ zd buf[NE * LS];
   __shared__ zd tw[L];
   const int Lr = RT ? plan.L : L;
   const int fixed = blockIdx.x;
   const int64_t e0 = (int64_t)blockIdx.y * NE;
-  for (int i = threadIdx.x; i < Lr; i += 256) tw[i] = twg[i];
+  for (int i = threadIdx.x; i < Lr; i += NT) tw[i] = twg[i];
   auto gidx = [&](int l) -> int64_t {
     return AXIS == 0 ? ((int64_t)fixed * Ny2 + l) * BS : ((int64_t)l * Ny2 + fixed) * BS;
   };
-  for (int i = threadIdx.x; i < NE * Lr; i += 256) {
+  for (int i = threadIdx.x; i < NE * Lr; i += NT) {
     const int l = i / NE, s = i - l * NE;
     buf[s * LS + l] = (e0 + s < BS) ? G[gidx(l) + e0 + s] : mkz(0, 0);
   }
   __syncthreads();
-  lds_fft_any<zd, L, NE, LS, 256, -1, RT>(buf, tw, plan);
-  for (int i = threadIdx.x; i < NE * Lr; i += 256) {
+  lds_fft_any<zd, L, NE, LS, NT, -1, RT>(buf, tw, plan);
+  for (int i = threadIdx.x; i < NE * Lr; i += NT) {
     const int k = i / NE, s = i - k * NE;
     if (e0 + s < BS) G[gidx(k) + e0 + s] = buf[s * LS + k];
   }

@@ -214,3 +214,40 @@ def test_strip_contraction(oracle, Nx, Ny, Nz):
     assert e64 < 1e-12 and e32 < 2e-6
     assert np.array_equal(op.apply_host(v), r)
     op.close()
+
+
+@pytest.mark.parametrize("p", [3, 5, 7, 11, 13, 17, 31, 37, 47, 61, 83, 97, 127, 251])
+def test_prime_lengths(oracle, p):
+    """Transforms of 4p points (and 2p-point halves where complex64 takes
+    them), alone and beside a length of other radices: registers up to 7, the
+    matrix-core stage from 11 (tiles of 16 outputs by 8 butterflies with
+    remainders at every prime here).  One apply on a random spectrum and the
+    tensor's spectrum against the oracle's, with the bars of the tests above."""
+    torch = _torch()
+    from giem2g_amd import models, operator as gop
+    N = 2 * p if p > 3 else 18
+    Nx, Ny, Nz = (N, 12, 3) if p % 4 == 1 else (8, N, 3)
+    if p == 31:
+        Nx, Ny = 62, 66
+    print("prime", p, Nx, Ny, flush=True)
+    m = models.small(Nx, Ny, Nz, seed=p, freq=0.8, dz=20.0)
+    om = oracle_model(oracle, m)
+    op = gop.IEOperator.from_model(m)
+    op.set_background(m.csigb(), m.thick, m.omega)
+    Gs = rand_vec(Nx * Ny * op.block_size, p) * (20.0 / 3.0)
+    op.put_tensor(Gs, spectral=True)
+    op.set_sigma(m.csiga())
+    v = rand_vec(3 * m.ncell, p + 1)
+    ref = om.apply(Gs, m.csiga(), v)
+    e64 = rel(op.apply_host(v), ref)
+    vt = torch.from_numpy(v).cuda().to(torch.complex64)
+    o32 = torch.empty_like(vt)
+    op.apply_dev_f32(vt, o32)
+    op.sync()
+    e32 = rel(o32.cpu().numpy().astype(np.complex128), ref)
+    op.put_tensor(Gs, spectral=False)
+    op.tensor_stage(1)
+    et = rel(op.get_tensor(), om.tensor_fft(Gs))
+    print("  FP64 %.2e complex64 %.2e tensor %.2e" % (e64, e32, et), flush=True)
+    assert e64 < 1e-12 and e32 < 2e-6 and et < 1e-12
+    op.close()
