@@ -106,6 +106,14 @@ template <bool PAIR> __device__ inline void y_tile(int& kx, int& chunk) {
   chunk = 2 * (st / hb) + (r >> 1);
 }
 
+// Distances (elements) between the vectors of one pass launch (blockIdx.z): of
+// inputs, outputs, slots of X and slots of S.  The kernels branch on the vector
+// number, so that an apply of one vector does not wait for these arguments
+// (32x32x8 21.1 us; without the branch 21.5, with a table of pointers 21.8).
+struct Steps {
+  int64_t in, out, x, s;
+};
+
 __device__ inline int64_t xidx(const Geo& g, int cz, int y, int kx) {
   const int nrx = 1 << g.nrx_log;
   return ((((int64_t)(cz >> g.nrx_log) * g.Ny + y) * (2 * g.Nx) + kx) << g.nrx_log) + (cz & (nrx - 1));
@@ -130,8 +138,12 @@ template <typename R, int L, bool RT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_fwd_x(const cx_t<R>* __restrict__ v,
                                               const cx_t<R>* __restrict__ gsig,
                                               cx_t<R>* __restrict__ X,
-                                              const cx_t<R>* __restrict__ twg, Geo g) {
+                                              const cx_t<R>* __restrict__ twg, Geo g, Steps st) {
   using T2 = cx_t<R>;
+  if (blockIdx.z) {
+    v += st.in * blockIdx.z;
+    X += st.x * blockIdx.z;
+  }
   constexpr int NR = nr_for<R>(L);
   constexpr int LS = L + 1;
   __shared__ T2 buf[NR * LS];
@@ -167,8 +179,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, 
 template <typename R, int L, bool FULL = false, bool RT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_fwd_y(const cx_t<R>* __restrict__ X,
                                               cx_t<R>* __restrict__ S,
-                                              const cx_t<R>* __restrict__ twg, Geo g) {
+                                              const cx_t<R>* __restrict__ twg, Geo g, Steps st) {
   using T2 = cx_t<R>;
+  if (blockIdx.z) {
+    X += st.x * blockIdx.z;
+    S += st.s * blockIdx.z;
+  }
   constexpr int NR = nr_for<R>(L);
   constexpr int LS = L + 1;
   __shared__ T2 buf[NR * LS];
@@ -194,8 +210,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, 
 template <typename R, int L, bool FULL = false, bool RT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_inv_y(const cx_t<R>* __restrict__ S,
                                               cx_t<R>* __restrict__ X,
-                                              const cx_t<R>* __restrict__ twg, Geo g) {
+                                              const cx_t<R>* __restrict__ twg, Geo g, Steps st) {
   using T2 = cx_t<R>;
+  if (blockIdx.z) {
+    X += st.x * blockIdx.z;
+    S += st.s * blockIdx.z;
+  }
   constexpr int NR = nr_for<R>(L);
   constexpr int LS = L + 1;
   __shared__ T2 buf[NR * LS];
@@ -230,8 +250,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, 
                                               const R* __restrict__ sq,
                                               const R* __restrict__ dzn,
                                               cx_t<R>* __restrict__ vout,
-                                              const cx_t<R>* __restrict__ twg, Geo g) {
+                                              const cx_t<R>* __restrict__ twg, Geo g, Steps st) {
   using T2 = cx_t<R>;
+  if (blockIdx.z) {
+    vin += st.in * blockIdx.z;
+    vout += st.out * blockIdx.z;
+    X += st.x * blockIdx.z;
+  }
   constexpr int NR = nr_for<R>(L);
   constexpr int LS = L + 1;
   __shared__ T2 buf[NR * LS];
@@ -295,8 +320,12 @@ template <typename R, int L, bool RT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_fwd_x_h(const cx_t<R>* __restrict__ v,
                                                 const cx_t<R>* __restrict__ gsig,
                                                 cx_t<R>* __restrict__ X,
-                                                const cx_t<R>* __restrict__ twg, Geo g) {
+                                                const cx_t<R>* __restrict__ twg, Geo g, Steps st) {
   using T2 = cx_t<R>;
+  if (blockIdx.z) {
+    v += st.in * blockIdx.z;
+    X += st.x * blockIdx.z;
+  }
   constexpr int NC = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(NC), PER = (NR * NC + NT - 1) / NT;
   __shared__ T2 buf[NR * LS];
   __shared__ T2 twN[NC], whs[wh_in_lds<R>() ? NC : 1];
@@ -361,8 +390,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, 
 template <typename R, int L, bool RT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_fwd_y_h(const cx_t<R>* __restrict__ X,
                                                 cx_t<R>* __restrict__ S,
-                                                const cx_t<R>* __restrict__ twg, Geo g) {
+                                                const cx_t<R>* __restrict__ twg, Geo g, Steps st) {
   using T2 = cx_t<R>;
+  if (blockIdx.z) {
+    X += st.x * blockIdx.z;
+    S += st.s * blockIdx.z;
+  }
   constexpr int NC = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(NC), PER = (NR * NC + NT - 1) / NT;
   __shared__ T2 buf[NR * LS];
   __shared__ T2 twN[NC], whs[wh_in_lds<R>() ? NC : 1];
@@ -409,8 +442,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, 
 template <typename R, int L, bool RT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_inv_y_h(const cx_t<R>* __restrict__ S,
                                                 cx_t<R>* __restrict__ X,
-                                                const cx_t<R>* __restrict__ twg, Geo g) {
+                                                const cx_t<R>* __restrict__ twg, Geo g, Steps st) {
   using T2 = cx_t<R>;
+  if (blockIdx.z) {
+    X += st.x * blockIdx.z;
+    S += st.s * blockIdx.z;
+  }
   constexpr int NC = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(NC), PER = (NR * NC + NT - 1) / NT;
   __shared__ T2 buf[NR * LS];
   __shared__ T2 twN[NC], whs[wh_in_lds<R>() ? NC : 1];
@@ -464,12 +501,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, 
 template <typename R, int L, bool RT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_inv_x_h(const cx_t<R>* __restrict__ X,
                                                 const cx_t<R>* __restrict__ vin,
-                                                const cx_t<R>* __restrict__ asiga,
+                                              const cx_t<R>* __restrict__ asiga,
                                                 const R* __restrict__ sq,
                                                 const R* __restrict__ dzn,
                                                 cx_t<R>* __restrict__ vout,
-                                                const cx_t<R>* __restrict__ twg, Geo g) {
+                                                const cx_t<R>* __restrict__ twg, Geo g, Steps st) {
   using T2 = cx_t<R>;
+  if (blockIdx.z) {
+    vin += st.in * blockIdx.z;
+    vout += st.out * blockIdx.z;
+    X += st.x * blockIdx.z;
+  }
   constexpr int NC = L / 2, NR = nr_half<R>(L), LS = ls_half<R>(NC), PER = (NR * NC + NT - 1) / NT;
   __shared__ T2 buf[NR * LS];
   __shared__ T2 twN[NC], whs[wh_in_lds<R>() ? NC : 1];
@@ -2046,15 +2088,16 @@ template <typename R> void op_free_buffers(OpBuffers<R>& b) {
     if (p) (void)hipFree((void*)p);
     p = nullptr;
   };
-  F(b.G); F(b.X); F(b.S); F(b.SB); F(b.gsig); F(b.asiga); F(b.sq); F(b.dzn); F(b.twx); F(b.twy);
+  F(b.G); F(b.X); F(b.S); F(b.SB); F(b.XB); F(b.gsig); F(b.asiga); F(b.sq); F(b.dzn); F(b.twx); F(b.twy);
 }
 
 // The forward (pre-scale, pad, x then y) and inverse (y then x, post-scale)
 // transforms of one vector between its cells and the spectrum S, with the
 // half-length kernels where b.half is set.
+// n vectors, st apart: inputs through X to S, and back
 template <typename R>
-static void fft_forward(const Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* S, const Geo& g,
-                        hipStream_t s) {
+static void fft_forward(const Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* X, cx_t<R>* S, const Geo& g, int n,
+                        const Steps& st, hipStream_t s) {
   const int Nx2 = 2 * op.Nx, Ny2 = 2 * op.Ny, Nz3 = 3 * op.Nz;
   const int nry = b.half ? nr_half_rt<R>(Ny2) : nr_rt<R>(Ny2);
   const int chy = (Nz3 + nry - 1) / nry;
@@ -2063,13 +2106,11 @@ static void fft_forward(const Operator& op, OpBuffers<R>& b, const cx_t<R>* vin,
     constexpr bool RT = decltype(LC)::rt;
     // (FP64 factor-plan rows are never half-length)
     if constexpr (RT && sizeof(R) == 8) {
-      hipLaunchKernelGGL((k_fwd_x<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, vin, b.gsig, b.X, b.twx,
-                         g);
+      hipLaunchKernelGGL((k_fwd_x<R, LL, RT>), dim3(op.Ny, b.nchunk, n), dim3(NT), 0, s, vin, b.gsig, X, b.twx, g, st);
     } else if (b.half) {
-      hipLaunchKernelGGL((k_fwd_x_h<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, vin, b.gsig, b.X, b.twx, g);
+      hipLaunchKernelGGL((k_fwd_x_h<R, LL, RT>), dim3(op.Ny, b.nchunk, n), dim3(NT), 0, s, vin, b.gsig, X, b.twx, g, st);
     } else {
-      hipLaunchKernelGGL((k_fwd_x<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, vin, b.gsig, b.X, b.twx,
-                         g);
+      hipLaunchKernelGGL((k_fwd_x<R, LL, RT>), dim3(op.Ny, b.nchunk, n), dim3(NT), 0, s, vin, b.gsig, X, b.twx, g, st);
     }
   });
   len_dispatch(Ny2, [&](auto LC) {
@@ -2077,18 +2118,18 @@ static void fft_forward(const Operator& op, OpBuffers<R>& b, const cx_t<R>* vin,
     constexpr bool RT = decltype(LC)::rt;
     // (FP64 factor-plan rows are never half-length)
     if constexpr (RT && sizeof(R) == 8) {
-      hipLaunchKernelGGL((k_fwd_y<R, LL, false, RT>), dim3(Nx2, chy), dim3(NT), 0, s, b.X, S, b.twy, g);
+      hipLaunchKernelGGL((k_fwd_y<R, LL, false, RT>), dim3(Nx2, chy, n), dim3(NT), 0, s, X, S, b.twy, g, st);
     } else if (b.half) {
-      hipLaunchKernelGGL((k_fwd_y_h<R, LL, RT>), dim3(Nx2, chy), dim3(NT), 0, s, b.X, S, b.twy, g);
+      hipLaunchKernelGGL((k_fwd_y_h<R, LL, RT>), dim3(Nx2, chy, n), dim3(NT), 0, s, X, S, b.twy, g, st);
     } else {
-      hipLaunchKernelGGL((k_fwd_y<R, LL, false, RT>), dim3(Nx2, chy), dim3(NT), 0, s, b.X, S, b.twy, g);
+      hipLaunchKernelGGL((k_fwd_y<R, LL, false, RT>), dim3(Nx2, chy, n), dim3(NT), 0, s, X, S, b.twy, g, st);
     }
   });
 }
 
 template <typename R>
-static void fft_inverse(const Operator& op, OpBuffers<R>& b, const cx_t<R>* S, const cx_t<R>* vin,
-                        cx_t<R>* vout, const Geo& g, hipStream_t s) {
+static void fft_inverse(const Operator& op, OpBuffers<R>& b, cx_t<R>* X, const cx_t<R>* S, const cx_t<R>* vin,
+                        cx_t<R>* vout, const Geo& g, int n, const Steps& st, hipStream_t s) {
   const int Nx2 = 2 * op.Nx, Ny2 = 2 * op.Ny, Nz3 = 3 * op.Nz;
   const int nry = b.half ? nr_half_rt<R>(Ny2) : nr_rt<R>(Ny2);
   const int chy = (Nz3 + nry - 1) / nry;
@@ -2097,11 +2138,11 @@ static void fft_inverse(const Operator& op, OpBuffers<R>& b, const cx_t<R>* S, c
     constexpr bool RT = decltype(LC)::rt;
     // (FP64 factor-plan rows are never half-length)
     if constexpr (RT && sizeof(R) == 8) {
-      hipLaunchKernelGGL((k_inv_y<R, LL, false, RT>), dim3(Nx2, chy), dim3(NT), 0, s, S, b.X, b.twy, g);
+      hipLaunchKernelGGL((k_inv_y<R, LL, false, RT>), dim3(Nx2, chy, n), dim3(NT), 0, s, S, X, b.twy, g, st);
     } else if (b.half) {
-      hipLaunchKernelGGL((k_inv_y_h<R, LL, RT>), dim3(Nx2, chy), dim3(NT), 0, s, S, b.X, b.twy, g);
+      hipLaunchKernelGGL((k_inv_y_h<R, LL, RT>), dim3(Nx2, chy, n), dim3(NT), 0, s, S, X, b.twy, g, st);
     } else {
-      hipLaunchKernelGGL((k_inv_y<R, LL, false, RT>), dim3(Nx2, chy), dim3(NT), 0, s, S, b.X, b.twy, g);
+      hipLaunchKernelGGL((k_inv_y<R, LL, false, RT>), dim3(Nx2, chy, n), dim3(NT), 0, s, S, X, b.twy, g, st);
     }
   });
   len_dispatch(Nx2, [&](auto LC) {
@@ -2109,35 +2150,21 @@ static void fft_inverse(const Operator& op, OpBuffers<R>& b, const cx_t<R>* S, c
     constexpr bool RT = decltype(LC)::rt;
     // (FP64 factor-plan rows are never half-length)
     if constexpr (RT && sizeof(R) == 8) {
-      hipLaunchKernelGGL((k_inv_x<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, b.X, vin, b.asiga, b.sq,
-                         b.dzn, vout, b.twx, g);
+      hipLaunchKernelGGL((k_inv_x<R, LL, RT>), dim3(op.Ny, b.nchunk, n), dim3(NT), 0, s, X, vin, b.asiga, b.sq, b.dzn, vout, b.twx, g, st);
     } else if (b.half) {
-      hipLaunchKernelGGL((k_inv_x_h<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, b.X, vin, b.asiga, b.sq,
-                         b.dzn, vout, b.twx, g);
+      hipLaunchKernelGGL((k_inv_x_h<R, LL, RT>), dim3(op.Ny, b.nchunk, n), dim3(NT), 0, s, X, vin, b.asiga, b.sq, b.dzn, vout, b.twx, g, st);
     } else {
-      hipLaunchKernelGGL((k_inv_x<R, LL, RT>), dim3(op.Ny, b.nchunk), dim3(NT), 0, s, b.X, vin, b.asiga, b.sq,
-                         b.dzn, vout, b.twx, g);
+      hipLaunchKernelGGL((k_inv_x<R, LL, RT>), dim3(op.Ny, b.nchunk, n), dim3(NT), 0, s, X, vin, b.asiga, b.sq, b.dzn, vout, b.twx, g, st);
     }
   });
 }
 
+// the contraction of one vector's spectrum S, in place
 template <typename R>
-void op_apply(Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* vout, hipStream_t s,
-              bool timed, bool mirror) {
-  G2G_CHECK(op.have_tensor && op.have_sigma, -4, "operator not ready: tensor or conductivity missing");
+static void contract_one(const Operator& op, OpBuffers<R>& b, cx_t<R>* S, const Geo& g, bool mirror, hipStream_t s) {
   const int Nz3 = 3 * op.Nz;
-  Geo g = make_geo(op, b.NR, b.half);
-  // profiling: events around the three stages (flushed into op.cnt later)
-  const bool prof = op.prof.on && !timed;
-  const int prec = sizeof(R) == 8 ? 0 : 1;
-  int pe[4] = {0, 0, 0, 0};
-  if (prof) pe[0] = op.prof.record(s);
-  if (timed) G2G_HIP(hipEventRecord(op.ev[0], s));
-  fft_forward<R>(op, b, vin, b.S, g, s);
-  if (timed) G2G_HIP(hipEventRecord(op.ev[1], s));
-  if (prof) pe[1] = op.prof.record(s);
   if (op.Nz > 64) {
-    launch_strips<R>(op, b.G, b.S, g, s);
+    launch_strips<R>(op, b.G, S, g, s);
   } else {
     // vector ALU: rows = Nz layers, split lanes per row (power of two)
     int split_log = 0;
@@ -2148,7 +2175,7 @@ void op_apply(Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* vout, 
         G2G_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     160 * 1024));
       }
-      hipLaunchKernelGGL(kern, dim3(op.Nx * op.Ny), dim3(NT), sm, s, b.S, b.G, g, op.BS, split_log);
+      hipLaunchKernelGGL(kern, dim3(op.Nx * op.Ny), dim3(NT), sm, s, S, b.G, g, op.BS, split_log);
     };
     // matrix cores for Nz from 8 to 64 (complex64: where c3_auto says so)
     // unless a vector-ALU kernel is requested (FP64 at 128x128x32:
@@ -2158,11 +2185,11 @@ void op_apply(Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* vout, 
     const bool mir = mirror && op_mirror_ok(op);
     bool done = false;
     if (op.contraction == 4 || op.contraction == 5 || (op.contraction == 0 && c1_auto<R>(op.Nz)))
-      done = launch_contract1<R>(op, b.G, b.S, g, op.contraction != 4 && mir, s);
+      done = launch_contract1<R>(op, b.G, S, g, op.contraction != 4 && mir, s);
     if (!done && mir && (op.contraction == 6 || op.contraction == 0) && c3_supported(op.Nz, 2))
-      done = launch_contract3<R, 2, true>(op, b.G, b.S, 0, g, s);
+      done = launch_contract3<R, 2, true>(op, b.G, S, 0, g, s);
     if (!done && (op.contraction == 2 || op.contraction == 6 || (op.contraction == 0 && c3_auto<R>(op.Nz))))
-      done = launch_contract3<R, 1>(op, b.G, b.S, 0, g, s);
+      done = launch_contract3<R, 1>(op, b.G, S, 0, g, s);
     if (done) {
     } else if (op.contraction == 3) {
       if (op.Nz * op.Nz <= 4 * NT) launch(k_contract<R, 4>);
@@ -2185,12 +2212,29 @@ void op_apply(Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* vout, 
         G2G_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     160 * 1024));
       }
-      hipLaunchKernelGGL(kern, dim3(op.Nx * op.Ny), dim3(2 * NT), sm, s, b.S, b.G, g, op.BS, sl2);
+      hipLaunchKernelGGL(kern, dim3(op.Nx * op.Ny), dim3(2 * NT), sm, s, S, b.G, g, op.BS, sl2);
     }
   }
+}
+
+template <typename R>
+void op_apply(Operator& op, OpBuffers<R>& b, const cx_t<R>* vin, cx_t<R>* vout, hipStream_t s,
+              bool timed, bool mirror) {
+  G2G_CHECK(op.have_tensor && op.have_sigma, -4, "operator not ready: tensor or conductivity missing");
+  Geo g = make_geo(op, b.NR, b.half);
+  // profiling: events around the three stages (flushed into op.cnt later)
+  const bool prof = op.prof.on && !timed;
+  const int prec = sizeof(R) == 8 ? 0 : 1;
+  int pe[4] = {0, 0, 0, 0};
+  if (prof) pe[0] = op.prof.record(s);
+  if (timed) G2G_HIP(hipEventRecord(op.ev[0], s));
+  fft_forward<R>(op, b, vin, b.X, b.S, g, 1, Steps{}, s);
+  if (timed) G2G_HIP(hipEventRecord(op.ev[1], s));
+  if (prof) pe[1] = op.prof.record(s);
+  contract_one<R>(op, b, b.S, g, mirror, s);
   if (timed) G2G_HIP(hipEventRecord(op.ev[2], s));
   if (prof) pe[2] = op.prof.record(s);
-  fft_inverse<R>(op, b, b.S, vin, vout, g, s);
+  fft_inverse<R>(op, b, b.X, b.S, vin, vout, g, 1, Steps{}, s);
   if (timed) G2G_HIP(hipEventRecord(op.ev[3], s));
   if (prof) {
     pe[3] = op.prof.record(s);
@@ -2210,6 +2254,61 @@ template <typename T2> __global__ void k_zero(T2* __restrict__ a, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) a[i] = mk<T2>(0, 0);
 }
 
+// Vectors one launch of each FFT pass takes: as many as keep their slots of X
+// and S within BATCH_PASS_BYTES.  A launch over one vector leaves the chip
+// idle on small grids (eight vectors at 16x16x8 in complex64: 48 -> 22 us a
+// batch, at 64x64x16 235 -> 114, FP64 333 -> 217) and has a tail on large ones
+// (128x128x32 1258 -> 1125 and 2180 -> 2075 us).  Limits of 64, 128, 256, 512
+// and 1024 MB gave 1188, 947, 911, 859, 859 us at 106x94x24 in complex64 and
+// 2180, 2180, 2180, 2076, 2013 at 128x128x32 in FP64; the slots of X take a
+// third of the limit, and above 512 MB what is left does not pay for them.
+constexpr size_t BATCH_PASS_BYTES = size_t(512) << 20;
+template <typename R> static int pass_vectors(const Operator& op, const OpBuffers<R>& b, int k) {
+  const size_t one = sizeof(cx_t<R>) * ((size_t)b.nchunk * b.NR * op.Ny * 2 * op.Nx + (size_t)12 * op.Nx * op.Ny * op.Nz);
+  return (int)std::max<size_t>(1, std::min<size_t>(k, BATCH_PASS_BYTES / one));
+}
+// Whether the k vectors can share launches: equal distances, and no output
+// over another vector's input (the vectors' passes keep their order then).
+template <typename T2> static bool in_step(int k, const T2* const* vins, T2* const* vouts, int64_t nv) {
+  for (int i = 0; i < k; i++) {
+    if (i && ((const char*)vins[i] - (const char*)vins[0] != i * ((const char*)vins[1] - (const char*)vins[0]) ||
+              (char*)vouts[i] - (char*)vouts[0] != i * ((char*)vouts[1] - (char*)vouts[0])))
+      return false;
+    for (int j = 0; j < k; j++)
+      if (i != j && vouts[i] < vins[j] + nv && vins[j] < vouts[i] + nv) return false;
+  }
+  return k < 2 || (((const char*)vins[1] - (const char*)vins[0]) % (int64_t)sizeof(T2) == 0 &&
+                   ((char*)vouts[1] - (char*)vouts[0]) % (int64_t)sizeof(T2) == 0);
+}
+
+// The slots of X for merged passes (and of S, where each vector has its own
+// contraction).  Made once, for the largest batch, so that a captured graph
+// keeps valid addresses; false when they cannot be made (stream under
+// capture, no memory): the vectors go one after the other then, which needs
+// no memory.
+template <typename R> static bool pass_slots(const Operator& op, OpBuffers<R>& b, hipStream_t s) {
+  using T2 = cx_t<R>;
+  if (b.x_fixed || b.xb_cap) return true;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (st != hipStreamCaptureStatusNone) return false;
+  const int m = pass_vectors(op, b, 8);
+  const bool own = op_batch_max(op) == 1;
+  const size_t nX = (size_t)b.nchunk * b.NR * op.Ny * 2 * op.Nx, nS = (size_t)12 * op.Nx * op.Ny * op.Nz;
+  T2* p = nullptr;
+  if (hipMalloc((void**)&p, sizeof(T2) * m * (nX + (own ? nS : 0))) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  b.bytes += sizeof(T2) * m * (nX + (own ? nS : 0));
+  b.XB = p;
+  b.xb_cap = m;
+  return true;
+}
+
 // k right-hand sides (1 <= k <= 8, k <= op_batch_max) through one tensor read:
 // each vector is transformed into its own slot of the batch spectrum
 // buffer, one contraction with k operand columns serves all of them, then
@@ -2227,10 +2326,18 @@ static void op_apply_k(Operator& op, OpBuffers<R>& b, int k, const cx_t<R>* cons
       (void)hipFree(b.SB);
       b.bytes -= sizeof(T2) * (size_t)nS * b.sb_cap;
     }
+    b.SB = nullptr;
+    b.sb_cap = 0;
     G2G_HIP(hipMalloc((void**)&b.SB, sizeof(T2) * (size_t)nS * kk));
     b.bytes += sizeof(T2) * (size_t)nS * kk;
     b.sb_cap = kk;
   }
+  const int64_t nX = (int64_t)b.nchunk * b.NR * op.Ny * Nx2;
+  int m = pass_vectors(op, b, k);
+  if (b.x_fixed) m = std::min(m, b.x_fixed);
+  if (m > 1 && (!in_step(k, vins, vouts, 3 * (int64_t)op.ncell()) || !pass_slots<R>(op, b, s))) m = 1;
+  T2* X = b.x_fixed || m == 1 ? b.X : b.XB;
+  const Steps st = m == 1 ? Steps{} : Steps{vins[1] - vins[0], vouts[1] - vouts[0], nX, nS};
   // unused slots hold zero spectra (a fill kernel, not a memset node, so
   // that a caller may capture the apply in a graph)
   if (kk > k) {
@@ -2243,7 +2350,10 @@ static void op_apply_k(Operator& op, OpBuffers<R>& b, int k, const cx_t<R>* cons
   const int prec = sizeof(R) == 8 ? 0 : 1;
   int pe[4] = {0, 0, 0, 0};
   if (prof) pe[0] = op.prof.record(s);
-  for (int r = 0; r < k; r++) fft_forward<R>(op, b, vins[r], b.SB + nS * r, g, s);
+  for (int r = 0; r < k; r += m) {
+    const int n = std::min(m, k - r);
+    fft_forward<R>(op, b, vins[r], X, b.SB + nS * r, g, n, st, s);
+  }
   if (prof) pe[1] = op.prof.record(s);
   bool ok = false;
   switch (kk) {
@@ -2272,12 +2382,42 @@ static void op_apply_k(Operator& op, OpBuffers<R>& b, int k, const cx_t<R>* cons
   }
   G2G_CHECK(ok, -3, "batched contraction not available for this Nz");
   if (prof) pe[2] = op.prof.record(s);
-  for (int r = 0; r < k; r++) fft_inverse<R>(op, b, b.SB + nS * r, vins[r], vouts[r], g, s);
+  for (int r = 0; r < k; r += m) {
+    const int n = std::min(m, k - r);
+    fft_inverse<R>(op, b, X, b.SB + nS * r, vins[r], vouts[r], g, n, st, s);
+  }
   if (prof) {
     pe[3] = op.prof.record(s);
     op.prof.mark(Prof::FWD, prec, k, pe[0], pe[1]);
     op.prof.mark(Prof::CONTR, prec, k, pe[1], pe[2]);
     op.prof.mark(Prof::BWD, prec, k, pe[2], pe[3]);
+  }
+  G2G_HIP(hipGetLastError());
+}
+
+// n right-hand sides that share the FFT passes alone (op_batch_max == 1);
+// pass_slots must hold.
+template <typename R>
+static void op_apply_passes(Operator& op, OpBuffers<R>& b, int n, const cx_t<R>* vin, cx_t<R>* vout, hipStream_t s) {
+  const int64_t nX = (int64_t)b.nchunk * b.NR * op.Ny * 2 * op.Nx, nS = (int64_t)12 * op.Nx * op.Ny * op.Nz;
+  const int64_t nv = 3 * (int64_t)op.ncell();
+  const Steps st{nv, nv, nX, nS};
+  cx_t<R>* S = b.XB + nX * b.xb_cap;
+  const Geo g = make_geo(op, b.NR, b.half);
+  const bool prof = op.prof.on;
+  const int prec = sizeof(R) == 8 ? 0 : 1;
+  int pe[4] = {0, 0, 0, 0};
+  if (prof) pe[0] = op.prof.record(s);
+  fft_forward<R>(op, b, vin, b.XB, S, g, n, st, s);
+  if (prof) pe[1] = op.prof.record(s);
+  for (int r = 0; r < n; r++) contract_one<R>(op, b, S + nS * r, g, false, s);
+  if (prof) pe[2] = op.prof.record(s);
+  fft_inverse<R>(op, b, b.XB, S, vin, vout, g, n, st, s);
+  if (prof) {
+    pe[3] = op.prof.record(s);
+    op.prof.mark(Prof::FWD, prec, n, pe[0], pe[1]);
+    op.prof.mark(Prof::CONTR, prec, n, pe[1], pe[2]);
+    op.prof.mark(Prof::BWD, prec, n, pe[2], pe[3]);
   }
   G2G_HIP(hipGetLastError());
 }
@@ -2306,11 +2446,19 @@ void op_apply_batch(Operator& op, OpBuffers<R>& b, int nrhs, const cx_t<R>* vin,
   // FP64 takes at most four per tensor read: an eight-vector FP64 kernel
   // held 360 registers per lane (one wave per SIMD) and measured 22% slower
   // per vector than four at 128x128x32
-  const int kmax = std::min(op_batch_max(op), sizeof(R) == 8 ? 4 : 8);
+  // (layer counts with no contraction of several vectors share the FFT passes
+  // where these take several; an output over another vector's input keeps
+  // the vectors one after the other)
+  int kmax = std::min(op_batch_max(op), sizeof(R) == 8 ? 4 : 8);
+  const bool apart = vin == vout || vout + nv * nrhs <= vin || vin + nv * nrhs <= vout;
+  const bool passes = kmax == 1 && nrhs > 1 && apart && pass_vectors(op, b, 8) > 1 && pass_slots<R>(op, b, s);
+  if (passes) kmax = b.xb_cap;
   for (int r0 = 0; r0 < nrhs;) {
     const int k = std::min(kmax, nrhs - r0);
     if (k == 1) {
       op_apply<R>(op, b, vin + nv * r0, vout + nv * r0, s, false, false);
+    } else if (passes) {
+      op_apply_passes<R>(op, b, k, vin + nv * r0, vout + nv * r0, s);
     } else {
       const cx_t<R>* vins[8];
       cx_t<R>* vouts[8];
@@ -2395,8 +2543,10 @@ void op_apply_batch_noalloc(Operator& op, OpBuffers<R>& b, int nrhs, const cx_t<
   OpBuffers<R> bl = b;
   T2* base = static_cast<T2*>(scratch_dev[dev]);
   const size_t nX = (size_t)b.nchunk * b.NR * op.Ny * 2 * op.Nx;
+  const size_t nS = (size_t)4 * op.Nx * op.Ny * 3 * op.Nz, all = NOALLOC_SCRATCH_BYTES / sizeof(T2);
+  bl.x_fixed = (int)std::min<size_t>(8, (all - nS * kcap) / nX);
   bl.X = base;
-  bl.SB = base + nX;
+  bl.SB = base + nX * bl.x_fixed;
   bl.S = bl.SB;
   bl.sb_cap = kcap;
   const int64_t nv = 3 * (int64_t)op.ncell();
@@ -2638,12 +2788,12 @@ void rc_apply(RcOperator& rc, const zd* E, zd* Ea, zd* Ha, hipStream_t s) {
   len_dispatch(Nx2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     hipLaunchKernelGGL((k_fwd_x<double, LL, decltype(LC)::rt>), dim3(op.Ny, rc.nchunk_f), dim3(NT), 0, s, E,
-                       rc.dsig, rc.Xf, twx, gf);
+                       rc.dsig, rc.Xf, twx, gf, Steps{});
   });
   len_dispatch(Ny2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     hipLaunchKernelGGL((k_fwd_y<double, LL, true, decltype(LC)::rt>), dim3(Nx2, (3 * op.Nz + nry - 1) / nry),
-                       dim3(NT), 0, s, rc.Xf, rc.S, twy, gf);
+                       dim3(NT), 0, s, rc.Xf, rc.S, twy, gf, Steps{});
   });
   G2G_HIP(hipEventRecord(op.ev[7], s));
   {
@@ -2671,7 +2821,7 @@ void rc_apply(RcOperator& rc, const zd* E, zd* Ea, zd* Ha, hipStream_t s) {
   len_dispatch(Ny2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     hipLaunchKernelGGL((k_inv_y<double, LL, true, decltype(LC)::rt>), dim3(Nx2, (6 * Nr + nry - 1) / nry),
-                       dim3(NT), 0, s, rc.So, rc.Xi, twy, gi);
+                       dim3(NT), 0, s, rc.So, rc.Xi, twy, gi, Steps{});
   });
   len_dispatch(Nx2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;

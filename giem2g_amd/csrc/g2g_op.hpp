@@ -162,6 +162,9 @@ template <typename R> struct OpBuffers {
   T2* S = nullptr;      // 2Nx*2Ny*3Nz
   T2* SB = nullptr;     // spectra of batched applies, sb_cap slots (allocated on first use)
   int sb_cap = 0;
+  T2* XB = nullptr;     // X of the batched applies' passes, xb_cap slots (allocated on first use)
+  int xb_cap = 0;
+  int x_fixed = 0;      // > 0: X itself has that many slots and nothing is allocated
   T2* gsig = nullptr;   // Nx*Ny*Nz
   T2* asiga = nullptr;  // Nx*Ny*Nz
   R* sq = nullptr;      // Nz: sqrt(Re sigma_b)

@@ -562,3 +562,36 @@ def test_adjoint_apply(oracle, Nx, Ny, Nz):
         torch.cuda.synchronize()
         assert rel(out, A.conj().T @ w) < 1e-11
     op.close()
+
+
+@pytest.mark.parametrize("Nx,Ny,Nz,nrhs", [(8, 10, 1, 9), (10, 8, 5, 17), (14, 10, 7, 2), (10, 8, 70, 11), (34, 22, 8, 7),
+                                            (64, 64, 8, 13), (96, 80, 6, 8), (48, 32, 66, 3)])
+def test_batch_shares_passes(Nx, Ny, Nz, nrhs):
+    """Batches whose vectors share launches of the FFT passes (whole groups,
+    ragged last groups, and grids of which fewer than eight fit one launch):
+    every row against a one-vector apply (FP64 1e-14, complex64 2e-6, the bars
+    of the oracle test above), in place with the same bits as out of place,
+    and the allocation-free apply with the same bits."""
+    torch = _torch()
+    from giem2g_amd import models, operator as gop
+    print("passes", Nx, Ny, Nz, nrhs, flush=True)
+    m = models.small(Nx, Ny, Nz, seed=Nx + Nz, freq=0.7, dz=25.0)
+    op = gop.operator_for(m)
+    g = torch.Generator(device="cuda").manual_seed(Nx + nrhs)
+    V = torch.complex(*torch.randn(2, nrhs, op.nvec, dtype=torch.float64, device="cuda", generator=g))
+    for dt, tol in ((torch.complex128, 1e-14), (torch.complex64, 2e-6)):
+        vin = V.to(dt).contiguous()
+        vout, one, na = torch.empty_like(vin), torch.empty_like(vin[0]), torch.empty_like(vin)
+        op.apply_batch_dev(vin, vout)
+        apply = op.apply_dev if dt == torch.complex128 else op.apply_dev_f32
+        for r in range(nrhs):
+            apply(vin[r], one)
+            op.sync()
+            e = float((vout[r] - one).abs().pow(2).sum().sqrt() / one.abs().pow(2).sum().sqrt())
+            assert e < tol, (dt, r, e)
+        op.apply_batch_dev_noalloc(vin, na)
+        op.apply_batch_dev(vin, vin)
+        op.sync()
+        assert torch.equal(torch.view_as_real(vin), torch.view_as_real(vout))
+        assert torch.equal(torch.view_as_real(na), torch.view_as_real(vout))
+    op.close()
