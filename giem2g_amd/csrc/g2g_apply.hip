@@ -2166,9 +2166,10 @@ static void contract_one(const Operator& op, OpBuffers<R>& b, cx_t<R>* S, const 
   if (op.Nz > 64) {
     launch_strips<R>(op, b.G, S, g, s);
   } else {
-    // vector ALU: rows = Nz layers, split lanes per row (power of two)
+    // vector ALU: rows = Nz layers, split lanes per row (power of two, of one
+    // wave: the lanes' sums are combined by shuffles)
     int split_log = 0;
-    while ((op.Nz << (split_log + 1)) <= NT) split_log++;
+    while (split_log < 6 && (op.Nz << (split_log + 1)) <= NT) split_log++;
     const size_t sm = sizeof(cx_t<R>) * (4 * (size_t)Nz3 + 2 * (size_t)op.Nz * (op.Nz + 1));
     auto launch = [&](auto kern) {
       if (sm > 65536) {

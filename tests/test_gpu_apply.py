@@ -595,3 +595,25 @@ def test_batch_shares_passes(Nx, Ny, Nz, nrhs):
         assert torch.equal(torch.view_as_real(vin), torch.view_as_real(vout))
         assert torch.equal(torch.view_as_real(na), torch.view_as_real(vout))
     op.close()
+
+
+@pytest.mark.parametrize("Nx,Ny,Nz", [(8, 8, 1), (8, 10, 1), (16, 8, 2), (8, 14, 2), (8, 8, 3)])
+def test_fewest_layers(oracle, Nx, Ny, Nz):
+    """One to three layers: a receiver row's lanes have to stay in one wave
+    (FP64 1e-12, complex64 2e-6, against the oracle)."""
+    torch = _torch()
+    from giem2g_amd import models, operator as gop
+    print("layers", Nx, Ny, Nz, flush=True)
+    m = models.small(Nx, Ny, Nz, seed=Nx + Nz, freq=0.8, dz=20.0)
+    om = oracle_model(oracle, m)
+    Gs = om.tensor_fft(om.tensor_realspace())
+    v = rand_vec(3 * m.ncell, Nz)
+    ref = om.apply(Gs, m.csiga(), v)
+    op = gop.operator_for(m)
+    assert rel(op.apply_host(v), ref) < 1e-12
+    vt = torch.from_numpy(v).cuda().to(torch.complex64)
+    o32 = torch.empty_like(vt)
+    op.apply_dev_f32(vt, o32)
+    op.sync()
+    assert rel(o32.cpu().numpy().astype(np.complex128), ref) < 2e-6
+    op.close()
