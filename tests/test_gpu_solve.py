@@ -182,3 +182,26 @@ def test_inner_tolerance(prec):
     with pytest.raises(L.G2GError, match="inner_tol"):
         op.solve(E, inner_tol=1.5, **kw)
     op.close()
+
+
+@pytest.mark.parametrize("Nx,Ny,Nz,m", [(8, 8, 1, 4), (8, 10, 2, 8), (10, 8, 3, 9), (16, 14, 5, 17)])
+def test_short_vectors_and_basis_sizes(oracle, Nx, Ny, Nz, m):
+    """Gram-Schmidt passes whose vectors fill less than one block or end inside
+    one, with bases at the edges of the groups of eight columns: the FP64
+    solve against the oracle's (1e-6 and equal counts, as above) and the
+    mixed solve's true residual."""
+    from giem2g_amd import models, operator as gop
+    print("short", Nx, Ny, Nz, m, flush=True)
+    md = models.small(Nx, Ny, Nz, seed=Nx + Nz, freq=0.8, dz=20.0)
+    om = oracle_model(oracle, md)
+    E = om.plane_wave(1)
+    Eo, info = om.solve(om.tensor_fft(om.tensor_realspace()), md.csiga(), E, m_out=m, m_in=m, maxit=100, tol=1e-8)
+    op = gop.operator_for(md)
+    Es, gi = op.solve(E, outer_m=m, inner_m=m, max_restart=100, tol=1e-8)
+    assert gi["status"] == 1 and gi["true_residual"] < 1e-8
+    assert (gi["outer_iterations"], gi["matvecs_fp64"]) == (info.iterations, info.matvecs)
+    assert rel(Es, Eo) < 1e-6
+    Em, gm = op.solve(E, outer_m=m, inner_m=m, max_restart=100, tol=1e-8, inner_precision=1)
+    assert gm["status"] == 1 and gm["true_residual"] < 1e-8
+    assert rel(Em, Eo) < 1e-6
+    op.close()
