@@ -2753,21 +2753,22 @@ void rc_fini(RcOperator& rc) {
   }
   if (rc.wts) (void)hipFree(rc.wts);
   rc.wts = nullptr;
+  rc.par.release();
 }
 
 // FinalizeRCOperator (:168-196): the conductivity of the current frequency
 void rc_set_sigma(RcOperator& rc, const zd* d_csiga) {
   Operator& op = *rc.op;
   G2G_CHECK(op.have_bkg, -4, "background not set");
-  zd* d_csigb;
-  G2G_HIP(hipMalloc(&d_csigb, sizeof(zd) * op.Nz));
-  G2G_HIP(hipMemcpy(d_csigb, op.csigb.data(), sizeof(zd) * op.Nz, hipMemcpyHostToDevice));
+  rc.par.h.clear();
+  const size_t o0 = rc.par.add(op.csigb.data(), op.Nz);
+  rc.par.send();
+  const zd* d_csigb = rc.par.at<zd>(o0);
   const int64_t n = op.ncell();
   hipLaunchKernelGGL(k_dsig, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, op.stream, d_csiga, d_csigb,
                      rc.dsig, (int64_t)op.Nx * op.Ny, op.Nz);
   G2G_HIP(hipGetLastError());
   G2G_HIP(hipStreamSynchronize(op.stream));
-  (void)hipFree(d_csigb);
   rc.have_sigma = true;
   rc.sigma_version = op.bkg_version;
 }
@@ -2947,12 +2948,11 @@ void op_set_sigma(Operator& op, const zd* d_csiga) {
   if (!op.csiga) G2G_HIP(hipMalloc(&op.csiga, sizeof(zd) * op.ncell()));
   if (d_csiga != op.csiga)
     G2G_HIP(hipMemcpyAsync(op.csiga, d_csiga, sizeof(zd) * op.ncell(), hipMemcpyDeviceToDevice, op.stream));
-  zd* d_csigb;
-  double* d_sq;
-  G2G_HIP(hipMalloc(&d_csigb, sizeof(zd) * Nz));
-  G2G_HIP(hipMalloc(&d_sq, sizeof(double) * Nz));
-  G2G_HIP(hipMemcpy(d_csigb, op.csigb.data(), sizeof(zd) * Nz, hipMemcpyHostToDevice));
-  G2G_HIP(hipMemcpy(d_sq, op.sqsigb.data(), sizeof(double) * Nz, hipMemcpyHostToDevice));
+  op.spar.h.clear();
+  const size_t o0 = op.spar.add(op.csigb.data(), Nz), o1 = op.spar.add(op.sqsigb.data(), Nz);
+  op.spar.send();
+  const zd* d_csigb = op.spar.at<zd>(o0);
+  const double* d_sq = op.spar.at<double>(o1);
   const int64_t n = op.ncell(), ncxy = (int64_t)op.Nx * op.Ny;
   const int blocks = (int)((n + 255) / 256);
   hipLaunchKernelGGL((k_sigma<double>), dim3(blocks), dim3(256), 0, op.stream, op.csiga, d_csigb,
@@ -2962,8 +2962,6 @@ void op_set_sigma(Operator& op, const zd* d_csiga) {
   if (op.d32.gsig) op_sigma_to_f32(op);
   G2G_HIP(hipGetLastError());
   G2G_HIP(hipStreamSynchronize(op.stream));
-  (void)hipFree(d_csigb);
-  (void)hipFree(d_sq);
 }
 
 template <typename R> static void upload_dzn(const Operator& op, OpBuffers<R>& b) {

@@ -183,18 +183,20 @@ void build_tensor(Operator& op, int stage) {
     op.tensor_own = true;
   }
   if (stage != 0) {
-    hipEvent_t a, b;
-    G2G_HIP(hipEventCreate(&a));
-    G2G_HIP(hipEventCreate(&b));
-    G2G_HIP(hipEventRecord(a, op.stream));
+    if (stage > 0) G2G_HIP(hipEventRecord(op.ev[1], op.stream));
     op_tensor_fft(op, op.d64.G, half);
-    G2G_HIP(hipEventRecord(b, op.stream));
-    G2G_HIP(hipEventSynchronize(b));
-    float ms = 0;
-    G2G_HIP(hipEventElapsedTime(&ms, a, b));
+    G2G_HIP(hipEventRecord(op.ev[2], op.stream));
+  }
+  // one wait for both stages
+  G2G_HIP(hipStreamSynchronize(op.stream));
+  float ms = 0;
+  if (stage <= 0) {
+    G2G_HIP(hipEventElapsedTime(&ms, op.ev[0], op.ev[1]));
+    op.cnt.t_tensor = ms * 1e-3;
+  }
+  if (stage != 0) {
+    G2G_HIP(hipEventElapsedTime(&ms, op.ev[1], op.ev[2]));
     op.cnt.t_tensor_fft = ms * 1e-3;
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
     op.have_tensor = true;
     if (op.d32.G) op_make_g32(op);
   }

@@ -176,6 +176,38 @@ template <typename R> struct OpBuffers {
   size_t bytes = 0;
 };
 
+// Small host tables that a kernel reads, in one device buffer that its owner
+// keeps: add() each, then one copy.  (A buffer, a copy and a free of their own
+// for every table, and transform twiddles made anew, took the next frequency
+// at 128x128x32 0.2 ms of 2.5.)  The kernels that read the tables of one
+// send() must have ended before the next.
+struct DevTables {
+  char* d = nullptr;
+  size_t cap = 0;
+  std::vector<char> h;
+  template <typename T> size_t add(const T* v, size_t n) {
+    const size_t at = (h.size() + 15) & ~size_t(15);
+    h.resize(at + sizeof(T) * n);
+    std::memcpy(h.data() + at, v, sizeof(T) * n);
+    return at;
+  }
+  template <typename T> const T* at(size_t o) const { return reinterpret_cast<const T*>(d + o); }
+  void send() {
+    if (cap < h.size()) {
+      release();
+      G2G_HIP(hipMalloc((void**)&d, h.size()));
+      cap = h.size();
+    }
+    G2G_HIP(hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice));
+    h.clear();
+  }
+  void release() {
+    if (d) (void)hipFree(d);
+    d = nullptr;
+    cap = 0;
+  }
+};
+
 struct Operator {
   int Nx = 0, Ny = 0, Nz = 0;
   double dx = 0, dy = 0;
@@ -215,7 +247,8 @@ struct Operator {
   // solve runs two); kept between solves, freed with the operator
   Arena ws[2];
   size_t tabs_bytes = 0;
-  hipEvent_t ev[8] = {};
+  DevTables par, spar;  // tables of the tensor build, of the conductivity
+  hipEvent_t ev[8] = {};  // (0, 1 and 2 also time the tensor builds)
 
   int64_t ncell() const { return (int64_t)Nx * Ny * Nz; }
   int64_t nvec() const { return 3 * ncell(); }
@@ -238,6 +271,7 @@ struct RcOperator {
   zd* G = nullptr;        // tensor, NP*BS
   double* wts = nullptr;  // masked, lambda-scaled weights [r][6][501][NP] (frequency independent)
   zd* tabs = nullptr;     // per-tap kernel tables of one receiver [501][13][Nz]
+  DevTables par;          // tables of the tensor build, of the conductivity
   zd* dsig = nullptr;     // sigma_a - sigma_b per cell
   zd *Xf = nullptr, *S = nullptr, *So = nullptr, *Xi = nullptr;  // FFT work buffers
   int NR = 0, nchunk_f = 0, nchunk_i = 0;
@@ -316,6 +350,7 @@ void op_make_g32(Operator& op);
 // half (a square grid with dx = dy, nobody reads the real-space tensor): only
 // the components and offsets from which op_tensor_fft(half) makes the whole
 // spectrum by the x-y mirror
+// (queued between events 0 and 1; the caller waits before the next)
 void op_build_tensor(Operator& op, bool half);
 void op_tensor_fft(Operator& op, zd* G, bool half);
 void op_free_tensor_scratch(Operator& op);

@@ -718,23 +718,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT ? 2 : 1)
   }
 }
 
-static void make_tw64(int L, int dir, zd** d) {
+static void make_tw64(int L, zd** d) {
   std::vector<zd> h(L);
   for (int t = 0; t < L; t++) {
     long double a = -2.0L * 3.14159265358979323846264338327950288L * t / L;
     h[t] = mkz((double)cosl(a), (double)sinl(a));
   }
-  (void)dir;
   G2G_HIP(hipMalloc(d, sizeof(zd) * L));
   G2G_HIP(hipMemcpy(*d, h.data(), sizeof(zd) * L, hipMemcpyHostToDevice));
 }
 
 void op_tensor_fft(Operator& op, zd* G, bool mir) {
   const int Nx2 = 2 * op.Nx, Ny2 = 2 * op.Ny;
-  zd *twx, *twy;
-  make_tw64(Nx2, -1, &twx);
-  make_tw64(Ny2, -1, &twy);
-  const FftPlan py = fft_plan(Ny2), px = fft_plan(Nx2);
+  const zd *twx = op.d64.twx, *twy = op.d64.twy;
+  const FftPlan &py = op.py, &px = op.px;
   const int64_t P = (int64_t)op.Nz * (op.Nz + 1) / 2, ne = mir ? 3 * P + (int64_t)op.Nz * op.Nz : op.BS;
   auto pass = [&](auto LC, auto AX, auto MR, const zd* tw, const FftPlan& plan) {
     constexpr int LL = decltype(LC)::value, axis = decltype(AX)::value;
@@ -753,12 +750,11 @@ void op_tensor_fft(Operator& op, zd* G, bool mir) {
     else pass(LC, integral_constant<int, 1>{}, std::false_type{}, twx, px);
   });
   G2G_HIP(hipGetLastError());
-  G2G_HIP(hipStreamSynchronize(op.stream));
-  (void)hipFree(twx);
-  (void)hipFree(twy);
 }
 
 void op_free_tensor_scratch(Operator& op) {
+  op.par.release();
+  op.spar.release();
   if (op.wts) (void)hipFree(op.wts);
   if (op.tabs) (void)hipFree(op.tabs);
   op.wts = nullptr;
@@ -766,43 +762,20 @@ void op_free_tensor_scratch(Operator& op) {
   op.have_wts = false;
 }
 
-void op_build_tensor(Operator& op, bool half) {
-  G2G_CHECK(op.have_bkg, -4, "background not set");
-  G2G_CHECK(op.Nl <= 64 && op.Nz <= MAX_NZ, -3, "tensor build supports Nl <= 64 and Nz <= 256");
-  const int64_t M = (int64_t)op.Nx * op.Ny;
-  const int Nz = op.Nz, P = Nz * (Nz + 1) / 2;
-  const double rmin = std::sqrt(op.dx * op.dx + op.dy * op.dy) / 2.0;  // :102
-  std::vector<double> lms(NTAPS);
+// Tables of a tensor build on the device: the taps' lambda, layer thicknesses
+// (1-based), borders, layer numbers and the background's arrays
+struct BuildTables {
+  const double *lms, *dz, *z;
+  const int* ln;
+  const zd* bk;  // sigma, i sigma mu0 w, (thickness, depth): Nl + 1 each
+  double mw;
+};
+static BuildTables build_tables(const Operator& op, DevTables& t, double rmin) {
+  const int Nz = op.Nz;
+  std::vector<double> lms(NTAPS), dz1(Nz + 1, 0.0);
   for (int j = 0; j < NTAPS; j++) lms[j] = std::exp(VB_XI + (double)(j + NFIRST - 512) * VB_YSTEP) / rmin;
-  double* d_lms;
-  G2G_HIP(hipMalloc(&d_lms, sizeof(double) * NTAPS));
-  G2G_HIP(hipMemcpy(d_lms, lms.data(), sizeof(double) * NTAPS, hipMemcpyHostToDevice));
-  hipEvent_t e0, e1;
-  G2G_HIP(hipEventCreate(&e0));
-  G2G_HIP(hipEventCreate(&e1));
-  G2G_HIP(hipEventRecord(e0, op.stream));
-  if (!op.have_wts) {
-    zd *tw, *f1;
-    make_tw64(VBN, -1, &tw);
-    G2G_HIP(hipMalloc(&f1, sizeof(zd) * VBN));
-    // the weights, then every offset's window of taps
-    if (!op.wts) G2G_HIP(hipMalloc(&op.wts, sizeof(double) * 6 * NTAPS * M + sizeof(int2) * M));
-    hipLaunchKernelGGL(k_f1, dim3(1), dim3(256), 0, op.stream, f1, tw);
-    WParams wp{op.Nx, op.Ny, op.dx, op.dy, rmin, std::log(rmin)};
-    hipLaunchKernelGGL(k_weights, dim3((unsigned)M), dim3(256), 0, op.stream, op.wts,
-                       (int2*)(op.wts + 6 * NTAPS * M), f1, tw, d_lms, wp);
-    G2G_HIP(hipGetLastError());
-    G2G_HIP(hipStreamSynchronize(op.stream));
-    (void)hipFree(tw);
-    (void)hipFree(f1);
-    op.have_wts = true;
-  }
-  // lambda tables
-  LParams lp;
-  lp.Nl = op.Nl;
-  lp.Nz = Nz;
+  for (int i = 1; i <= Nz; i++) dz1[i] = op.dz[i - 1];
   const double mw = 4.0 * PI_D * 1e-7 * op.omega;
-  lp.iwm = mkz(0.0, mw);
   std::vector<zd> bk(3 * (op.Nl + 1), mkz(0, 0));
   for (int i = 0; i <= op.Nl; i++) {
     bk[i] = op.csigma[i];
@@ -815,31 +788,54 @@ void op_build_tensor(Operator& op, bool half) {
       bk[2 * (op.Nl + 1) + i] = mkz(op.thick[i], depth);
     }
   }
-  zd* d_bk;
-  G2G_HIP(hipMalloc(&d_bk, sizeof(zd) * bk.size()));
-  G2G_HIP(hipMemcpy(d_bk, bk.data(), sizeof(zd) * bk.size(), hipMemcpyHostToDevice));
-  lp.bk = d_bk;
+  t.h.clear();
+  const size_t o0 = t.add(lms.data(), NTAPS), o1 = t.add(dz1.data(), Nz + 1), o2 = t.add(op.z.data(), Nz + 1),
+               o3 = t.add(op.lnum.data(), Nz + 1), o4 = t.add(bk.data(), bk.size());
+  t.send();
+  return {t.at<double>(o0), t.at<double>(o1), t.at<double>(o2), t.at<int>(o3), t.at<zd>(o4), mw};
+}
+
+void op_build_tensor(Operator& op, bool half) {
+  G2G_CHECK(op.have_bkg, -4, "background not set");
+  G2G_CHECK(op.Nl <= 64 && op.Nz <= MAX_NZ, -3, "tensor build supports Nl <= 64 and Nz <= 256");
+  const int64_t M = (int64_t)op.Nx * op.Ny;
+  const int Nz = op.Nz, P = Nz * (Nz + 1) / 2;
+  const double rmin = std::sqrt(op.dx * op.dx + op.dy * op.dy) / 2.0;  // :102
+  const BuildTables bt = build_tables(op, op.par, rmin);
+  G2G_HIP(hipEventRecord(op.ev[0], op.stream));
+  if (!op.have_wts) {
+    zd *tw, *f1;
+    make_tw64(VBN, &tw);
+    G2G_HIP(hipMalloc(&f1, sizeof(zd) * VBN));
+    // the weights, then every offset's window of taps
+    if (!op.wts) G2G_HIP(hipMalloc(&op.wts, sizeof(double) * 6 * NTAPS * M + sizeof(int2) * M));
+    hipLaunchKernelGGL(k_f1, dim3(1), dim3(256), 0, op.stream, f1, tw);
+    WParams wp{op.Nx, op.Ny, op.dx, op.dy, rmin, std::log(rmin)};
+    hipLaunchKernelGGL(k_weights, dim3((unsigned)M), dim3(256), 0, op.stream, op.wts,
+                       (int2*)(op.wts + 6 * NTAPS * M), f1, tw, bt.lms, wp);
+    G2G_HIP(hipGetLastError());
+    G2G_HIP(hipStreamSynchronize(op.stream));
+    (void)hipFree(tw);
+    (void)hipFree(f1);
+    op.have_wts = true;
+  }
+  // lambda tables
+  LParams lp;
+  lp.Nl = op.Nl;
+  lp.Nz = Nz;
+  lp.iwm = mkz(0.0, bt.mw);
+  lp.bk = bt.bk;
   const size_t tab_n = (size_t)NTAPS * (3 * P + Nz * Nz);
   if (!op.tabs || op.tabs_bytes < tab_n * sizeof(zd)) {
     if (op.tabs) (void)hipFree(op.tabs);
     G2G_HIP(hipMalloc(&op.tabs, tab_n * sizeof(zd)));
     op.tabs_bytes = tab_n * sizeof(zd);
   }
-  double *d_dz, *d_z;
-  int* d_ln;
-  std::vector<double> dz1(Nz + 1, 0.0);
-  for (int i = 1; i <= Nz; i++) dz1[i] = op.dz[i - 1];
-  G2G_HIP(hipMalloc(&d_dz, sizeof(double) * (Nz + 1)));
-  G2G_HIP(hipMalloc(&d_z, sizeof(double) * (Nz + 1)));
-  G2G_HIP(hipMalloc(&d_ln, sizeof(int) * (Nz + 1)));
-  G2G_HIP(hipMemcpy(d_dz, dz1.data(), sizeof(double) * (Nz + 1), hipMemcpyHostToDevice));
-  G2G_HIP(hipMemcpy(d_z, op.z.data(), sizeof(double) * (Nz + 1), hipMemcpyHostToDevice));
-  G2G_HIP(hipMemcpy(d_ln, op.lnum.data(), sizeof(int) * (Nz + 1), hipMemcpyHostToDevice));
   const size_t sm = sizeof(zd) * (size_t)(Nz + 1) * 20;
   if (sm > 65536)
     G2G_HIP(hipFuncSetAttribute((const void*)k_lambda, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
-  hipLaunchKernelGGL(k_lambda, dim3(NTAPS), dim3(64), sm, op.stream, (zd*)op.tabs, d_lms, d_dz,
-                     d_z, d_ln, lp);
+  hipLaunchKernelGGL(k_lambda, dim3(NTAPS), dim3(64), sm, op.stream, (zd*)op.tabs, bt.lms, bt.dz,
+                     bt.z, bt.ln, lp);
   G2G_HIP(hipGetLastError());
   // weighted sums into the real-space tensor (stored in d64.G), x 1/(4 pi)
   const zd* T = (const zd*)op.tabs;
@@ -869,18 +865,7 @@ void op_build_tensor(Operator& op, bool half) {
                        op.Nx, scale, jobs);
   }
   G2G_HIP(hipGetLastError());
-  G2G_HIP(hipEventRecord(e1, op.stream));
-  G2G_HIP(hipStreamSynchronize(op.stream));
-  float ms = 0;
-  G2G_HIP(hipEventElapsedTime(&ms, e0, e1));
-  op.cnt.t_tensor = ms * 1e-3;
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  (void)hipFree(d_lms);
-  (void)hipFree(d_bk);
-  (void)hipFree(d_dz);
-  (void)hipFree(d_z);
-  (void)hipFree(d_ln);
+  G2G_HIP(hipEventRecord(op.ev[1], op.stream));
 }
 
 // ====================================================================== //
@@ -1221,21 +1206,14 @@ void rc_build_tensor(RcOperator& rc) {
   const int Nz = op.Nz, Nr = rc.Nr;
   const int64_t NP = rc.NP, BS = rc.BS, WS = (int64_t)6 * NTAPS * NP + NP;  // weights per receiver, then the points' windows of taps
   const double rmin = std::sqrt(op.dx * op.dx + op.dy * op.dy) / 2.0;  // :67
-  std::vector<double> lms(NTAPS);
-  for (int j = 0; j < NTAPS; j++) lms[j] = std::exp(VB_XI + (double)(j + NFIRST - 512) * VB_YSTEP) / rmin;
-  double* d_lms;
-  G2G_HIP(hipMalloc(&d_lms, sizeof(double) * NTAPS));
-  G2G_HIP(hipMemcpy(d_lms, lms.data(), sizeof(double) * NTAPS, hipMemcpyHostToDevice));
-  hipEvent_t e0, e1;
-  G2G_HIP(hipEventCreate(&e0));
-  G2G_HIP(hipEventCreate(&e1));
-  G2G_HIP(hipEventRecord(e0, op.stream));
+  const BuildTables bt = build_tables(op, rc.par, rmin);
+  G2G_HIP(hipEventRecord(op.ev[0], op.stream));
   // The weights do not depend on frequency: all receivers' weights are kept
   // when they fit in 8 GB, else one receiver's are recomputed per build.
   const bool cache = (double)Nr * WS * sizeof(double) <= 8.0 * (1 << 30);
   zd *tw = nullptr, *f1 = nullptr;
   if (!rc.have_wts) {
-    make_tw64(VBN, -1, &tw);
+    make_tw64(VBN, &tw);
     G2G_HIP(hipMalloc(&f1, sizeof(zd) * VBN));
     hipLaunchKernelGGL(k_f1, dim3(1), dim3(256), 0, op.stream, f1, tw);
     if (!rc.wts) {
@@ -1246,48 +1224,21 @@ void rc_build_tensor(RcOperator& rc) {
   auto weights = [&](int r, double* dst) {
     RcWParams wp{op.Nx, op.Ny, op.dx, op.dy, rc.xs[r], rc.ys[r], std::log(rmin)};
     hipLaunchKernelGGL(k_rc_weights, dim3((unsigned)NP), dim3(256), 0, op.stream, dst,
-                       (int2*)(dst + 6 * NTAPS * NP), f1, tw, d_lms, wp);
+                       (int2*)(dst + 6 * NTAPS * NP), f1, tw, bt.lms, wp);
   };
   if (!rc.have_wts && cache)
     for (int r = 0; r < Nr; r++) weights(r, rc.wts + r * WS);
-  // background arrays, as for the IE tensor
-  const double mw = 4.0 * PI_D * 1e-7 * op.omega;
-  std::vector<zd> bk(3 * (op.Nl + 1), mkz(0, 0));
-  for (int i = 0; i <= op.Nl; i++) {
-    bk[i] = op.csigma[i];
-    bk[op.Nl + 1 + i] = mkz(-op.csigma[i].y * mw, op.csigma[i].x * mw);
-  }
-  {
-    double depth = 0;
-    for (int i = 1; i <= op.Nl - 1; i++) {
-      depth += op.thick[i];
-      bk[2 * (op.Nl + 1) + i] = mkz(op.thick[i], depth);
-    }
-  }
-  zd* d_bk;
-  G2G_HIP(hipMalloc(&d_bk, sizeof(zd) * bk.size()));
-  G2G_HIP(hipMemcpy(d_bk, bk.data(), sizeof(zd) * bk.size(), hipMemcpyHostToDevice));
   if (!rc.tabs) {
     G2G_HIP(hipMalloc(&rc.tabs, sizeof(zd) * NTAPS * RF_COUNT * Nz));
     rc.bytes += sizeof(zd) * NTAPS * RF_COUNT * Nz;
   }
-  double *d_dz, *d_z;
-  int* d_ln;
-  std::vector<double> dz1(Nz + 1, 0.0);
-  for (int i = 1; i <= Nz; i++) dz1[i] = op.dz[i - 1];
-  G2G_HIP(hipMalloc(&d_dz, sizeof(double) * (Nz + 1)));
-  G2G_HIP(hipMalloc(&d_z, sizeof(double) * (Nz + 1)));
-  G2G_HIP(hipMalloc(&d_ln, sizeof(int) * (Nz + 1)));
-  G2G_HIP(hipMemcpy(d_dz, dz1.data(), sizeof(double) * (Nz + 1), hipMemcpyHostToDevice));
-  G2G_HIP(hipMemcpy(d_z, op.z.data(), sizeof(double) * (Nz + 1), hipMemcpyHostToDevice));
-  G2G_HIP(hipMemcpy(d_ln, op.lnum.data(), sizeof(int) * (Nz + 1), hipMemcpyHostToDevice));
   const double scale = 1.0 / PI_D / 4.0;  // :223-224
   const int64_t ldb = RF_COUNT * Nz;
   for (int r = 0; r < Nr; r++) {
     double* W = rc.wts + (cache ? r * WS : 0);
     if (!cache) weights(r, W);
-    RcLParams lp{op.Nl, Nz, rc.layer[r], rc.cell[r], rc.zr[r], mkz(0.0, mw), d_bk};
-    hipLaunchKernelGGL(k_rc_lambda, dim3(NTAPS), dim3(64), 0, op.stream, rc.tabs, d_lms, d_dz, d_z, d_ln, lp);
+    RcLParams lp{op.Nl, Nz, rc.layer[r], rc.cell[r], rc.zr[r], mkz(0.0, bt.mw), bt.bk};
+    hipLaunchKernelGGL(k_rc_lambda, dim3(NTAPS), dim3(64), 0, op.stream, rc.tabs, bt.lms, bt.dz, bt.z, bt.ln, lp);
     auto Wc = [&](int c) { return W + (int64_t)c * NTAPS * NP; };
     auto Tf = [&](int f) { return (const zd*)rc.tabs + (int64_t)f * Nz; };
     auto J1 = [&](int e, int c, int f) {
@@ -1319,38 +1270,26 @@ void rc_build_tensor(RcOperator& rc) {
                        (const int2*)(W + 6 * NTAPS * NP), 0, scale, jobs);
   }
   G2G_HIP(hipGetLastError());
-  G2G_HIP(hipEventRecord(e1, op.stream));
+  G2G_HIP(hipEventRecord(op.ev[1], op.stream));
   G2G_HIP(hipStreamSynchronize(op.stream));
   float ms = 0;
-  G2G_HIP(hipEventElapsedTime(&ms, e0, e1));
+  G2G_HIP(hipEventElapsedTime(&ms, op.ev[0], op.ev[1]));
   rc.t_tensor = ms * 1e-3;
   rc.have_wts = rc.have_wts || cache;
   rc.have_tensor = true;
   rc.spectral = false;
   rc.tensor_version = op.bkg_version;
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
   if (tw) (void)hipFree(tw);
   if (f1) (void)hipFree(f1);
-  (void)hipFree(d_lms);
-  (void)hipFree(d_bk);
-  (void)hipFree(d_dz);
-  (void)hipFree(d_z);
-  (void)hipFree(d_ln);
 }
 
 void rc_tensor_fft(RcOperator& rc) {
   Operator& op = *rc.op;
   G2G_CHECK(rc.have_tensor && !rc.spectral, -4, "receiver tensor not built (or already transformed)");
   const int Nx2 = 2 * op.Nx, Ny2 = 2 * op.Ny;
-  zd *twx, *twy;
-  make_tw64(Nx2, -1, &twx);
-  make_tw64(Ny2, -1, &twy);
-  hipEvent_t a, b;
-  G2G_HIP(hipEventCreate(&a));
-  G2G_HIP(hipEventCreate(&b));
-  G2G_HIP(hipEventRecord(a, op.stream));
-  const FftPlan py = fft_plan(Ny2), px = fft_plan(Nx2);
+  const zd *twx = op.d64.twx, *twy = op.d64.twy;
+  const FftPlan &py = op.py, &px = op.px;
+  G2G_HIP(hipEventRecord(op.ev[0], op.stream));
   len_dispatch(Ny2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     constexpr int NE = ne_for<LL>();
@@ -1364,15 +1303,11 @@ void rc_tensor_fft(RcOperator& rc) {
                        dim3(256), 0, op.stream, rc.G, twx, Ny2, rc.BS, px);
   });
   G2G_HIP(hipGetLastError());
-  G2G_HIP(hipEventRecord(b, op.stream));
+  G2G_HIP(hipEventRecord(op.ev[1], op.stream));
   G2G_HIP(hipStreamSynchronize(op.stream));
   float ms = 0;
-  G2G_HIP(hipEventElapsedTime(&ms, a, b));
+  G2G_HIP(hipEventElapsedTime(&ms, op.ev[0], op.ev[1]));
   rc.t_fft = ms * 1e-3;
-  (void)hipEventDestroy(a);
-  (void)hipEventDestroy(b);
-  (void)hipFree(twx);
-  (void)hipFree(twy);
   rc.spectral = true;
 }
 
