@@ -511,19 +511,26 @@ __global__ __launch_bounds__(192 * NCI) void k_dw(DwArgs a) {
     }
 }
 
-// g[i] = sum over the np slots of part[slot][i], in a fixed order, in double
-__global__ __launch_bounds__(UB) void k_dw_reduce(const float* __restrict__ part, int np, int64_t n, float* __restrict__ g) {
-  __shared__ double red[UB];
-  const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+// g[i] = sum over the np slots of part[slot][i], in a fixed order, in double:
+// 64 sums per block, 16 threads each (4 threads each left most of the chip
+// idle: 123 us a gradient at 8 x 64x64x16, 8 threads 83, 16 threads 76)
+constexpr int DWR = 16;
+__global__ __launch_bounds__(64 * DWR) void k_dw_reduce(const float* __restrict__ part, int np, int64_t n, float* __restrict__ g) {
+  __shared__ double red[DWR][64];
+  const int t = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t i = (int64_t)blockIdx.x * 64 + t;
   double s = 0;
   if (i < n) {
 #pragma unroll 8
-    for (int k = threadIdx.x >> 6; k < np; k += UB / 64) s += (double)part[k * n + i];
+    for (int k = w; k < np; k += DWR) s += (double)part[k * n + i];
   }
-  red[threadIdx.x] = s;
+  red[w][t] = s;
   __syncthreads();
-  if (threadIdx.x < 64 && i < n)
-    g[i] = (float)((red[threadIdx.x] + red[threadIdx.x + 64]) + (red[threadIdx.x + 128] + red[threadIdx.x + 192]));
+  if (w == 0 && i < n) {
+    double sum = 0;
+    for (int k = 0; k < DWR; k++) sum += red[k][t];
+    g[i] = (float)sum;
+  }
 }
 
 // forward weights w[co][tap*cin+ci] and transposed weights
@@ -583,61 +590,58 @@ __global__ void k_pool(const bf16* __restrict__ src, bf16* __restrict__ dst, int
   *reinterpret_cast<bf16x8*>(dst + (bat * nc + q) * C + c8 * 8) = o;
 }
 
-// dz = dy * (y > 0) (or dy when y is null), FP32 and bf16 copies; channels
-// c >= C of the bf16 copy (row length Cp) are zero.
-__global__ void k_relu_back(const float* __restrict__ dy, int ldy, const bf16* __restrict__ y,
-                            int C, int Cp, float* __restrict__ dzf, bf16* __restrict__ dzb, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * Cp) return;
-  const int64_t p = i / Cp;
-  const int c = (int)(i % Cp);
-  float g = 0.f;
-  if (c < C) {
-    g = dy[p * ldy + c];
-    if (y && !((float)y[p * C + c] > 0.f)) g = 0.f;
-  }
-  dzf[i] = g;
-  dzb[i] = (bf16)g;
-}
-
-// split the gradient of a concatenation [up(src), skip] (row length C1+C2):
-// dsrc[q][c] = sum of the 8 children (c < C1), dskip[p][c] = dcat[p][C1+c]
-__global__ void k_split_cat(const float* __restrict__ dcat, int C1, int C2, float* __restrict__ dsrc,
-                            float* __restrict__ dskip, int nx, int ny, int nz, int64_t nb) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nf = (int64_t)nx * ny * nz, nc = nf / 8;
-  const int Ct = C1 + C2;
-  const int64_t n1 = nb * nc * C1, n2 = nb * nf * C2;
-  if (i < n1) {
-    const int c = (int)(i % C1);
-    const int64_t q = (i / C1) % nc, bat = i / (C1 * nc);
-    const int nxh = nx / 2, nyh = ny / 2;
-    const int x = (int)(q % nxh), y = (int)((q / nxh) % nyh), z = (int)(q / ((int64_t)nxh * nyh));
-    float s = 0.f;
+// dz = g * (y > 0) (or g when y is null), FP32 and bf16 copies, four channels
+// per thread; channels c >= C of the copies (row length Cp = 4 << sh) are zero.
+// The gradient g of the layer's output, taken from where the other layers left
+// it, so that it needs no pass of its own:
+//   GradPlain     g = dy (rows of ldy)
+//   GradUpsample  the output went, upsampled, into a concatenation: the sum of
+//                 its eight children in dy, the concatenation's gradient
+//   GradPool      the output went into a concatenation and a pooling: dy (the
+//                 concatenation's part) plus an eighth of dc, the pooled one's
+// Memory bounds it: with the sums and copies in kernels of their own, an
+// element and two 64-bit divisions per thread, 240 us of a gradient at 8 x
+// 64x64x16, now 132.
+enum GradSource { GradPlain, GradUpsample, GradPool };
+template <GradSource SRC>
+__global__ void k_relu_back(const float* __restrict__ dy, int ldy, const float* __restrict__ dc, const bf16* __restrict__ y,
+                            int C, int sh, float* __restrict__ dzf, bf16* __restrict__ dzb, int nx, int ny) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int xy = i >> sh, c = (i & ((1 << sh) - 1)) * 4, nz = gridDim.y, z = blockIdx.y;
+  if (xy >= nx * ny) return;
+  const int64_t bat = blockIdx.z, p = (bat * nz + z) * nx * ny + xy;
+  f32x4 g;
+  if constexpr (SRC == GradUpsample) {
+    const int yy = xy / nx, x = xy - yy * nx;
+    g = f32x4{0, 0, 0, 0};
+#pragma unroll
     for (int d = 0; d < 8; d++) {
-      const int X = 2 * x + (d & 1), Y = 2 * y + ((d >> 1) & 1), Z = 2 * z + (d >> 2);
-      s += dcat[(bat * nf + ((int64_t)Z * ny + Y) * nx + X) * Ct + c];
+      const int X = 2 * x + (d & 1), Y = 2 * yy + ((d >> 1) & 1), Z = 2 * z + (d >> 2);
+      g += *reinterpret_cast<const f32x4*>(dy + (((bat * 2 * nz + Z) * 2 * ny + Y) * 2 * nx + X) * ldy + c);
     }
-    dsrc[i] = s;
-  } else if (i < n1 + n2) {
-    const int64_t j = i - n1;
-    const int c = (int)(j % C2);
-    const int64_t p = j / C2;
-    dskip[j] = dcat[p * Ct + C1 + c];
+  } else {
+    g = *reinterpret_cast<const f32x4*>(dy + p * ldy + c);
+    if constexpr (SRC == GradPool) {
+      const int yy = xy / nx, x = xy - yy * nx;
+      const int64_t q = ((bat * (nz / 2) + z / 2) * (ny / 2) + yy / 2) * (nx / 2) + x / 2;
+      g += 0.125f * *reinterpret_cast<const f32x4*>(dc + q * C + c);
+    }
   }
-}
-
-// dfine[p][c] += dcoarse[p/2][c] / 8
-__global__ void k_pool_back_add(const float* __restrict__ dc, float* __restrict__ df, int C, int nx,
-                                int ny, int nz, int64_t nb) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nf = (int64_t)nx * ny * nz;
-  if (i >= nb * nf * C) return;
-  const int c = (int)(i % C);
-  const int64_t p = (i / C) % nf, bat = i / (C * nf);
-  const int x = (int)(p % nx), y = (int)((p / nx) % ny), z = (int)(p / ((int64_t)nx * ny));
-  const int64_t q = ((int64_t)(z / 2) * (ny / 2) + y / 2) * (nx / 2) + x / 2;
-  df[i] += 0.125f * dc[(bat * (nf / 8) + q) * C + c];
+  if (y) {
+    const bf16x4 v = *reinterpret_cast<const bf16x4*>(y + p * C + c);
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (!((float)v[k] > 0.f)) g[k] = 0.f;
+  }
+  bf16x4 o;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    if (c + k >= C) g[k] = 0.f;
+    o[k] = (bf16)g[k];
+  }
+  const int64_t at = (p << (sh + 2)) + c;
+  *reinterpret_cast<f32x4*>(dzf + at) = g;
+  *reinterpret_cast<bf16x4*>(dzb + at) = o;
 }
 
 // n voxels of 8 channels; VEC: a is 16-byte aligned
@@ -905,13 +909,12 @@ void unet_reserve(UNet& n, int B, int nx, int ny, int nz, bool training) {
     add((void**)&n.f48, 4 * n0 * 48);
     add((void**)&n.fa, 4 * n0 * 16);
     add((void**)&n.fb, 4 * n0 * 4);
-    add((void**)&n.de1, 4 * n0 * 16);
-    add((void**)&n.de2, 4 * n1 * 32);
+    add((void**)&n.f96, 4 * n1 * 96);
     add((void**)&n.dzf, 4 * n0 * 16);
     add((void**)&n.dzb, 2 * n0 * 16);
     add((void**)&n.dwp, 4 * dw_part_size(n, B, nx, ny, nz));
   } else {
-    n.dout = n.f48 = n.fa = n.fb = n.de1 = n.de2 = n.dzf = n.dwp = nullptr;
+    n.dout = n.f48 = n.fa = n.fb = n.f96 = n.dzf = n.dwp = nullptr;
     n.dzb = nullptr;
   }
   void* base = nullptr;
@@ -1116,7 +1119,7 @@ static void conv_dw(UNet& n, int li, const float* dzf, int ldz, Src s1, Src s2, 
   else if (no % 2 == 0 && ni == 1) dw_go<2, 1, false>(a, slots, 1, no / 2, s);
   else if (no % 2 == 0 && ni % 2 == 0) dw_go<2, 2, false>(a, slots, ni / 2, no / 2, s);
   else G2G_CHECK(false, -1, "no weight-gradient kernel for this layer width");
-  hipLaunchKernelGGL(k_dw_reduce, dim3(nblk(a.pstride, 64)), dim3(UB), 0, s, n.dwp, slots * (l.ntap == 1 ? 3 : 1),
+  hipLaunchKernelGGL(k_dw_reduce, dim3(nblk(a.pstride, 64)), dim3(64 * DWR), 0, s, n.dwp, slots * (l.ntap == 1 ? 3 : 1),
                      a.pstride, n.grads + l.poff);
 }
 
@@ -1156,13 +1159,16 @@ void unet_forward(UNet& n, hipStream_t s, const float* x, float* y) {
   G2G_HIP(hipGetLastError());
 }
 
-// one layer of the backward pass: dz = dy*(y>0), weight gradient, data gradient into dx
+// one layer of the backward pass: dz = g*(y>0), weight gradient, data gradient into dx
+template <GradSource SRC = GradPlain>
 static void layer_back(UNet& n, int li, const float* dy, int ldy, const bf16* y, Src s1, Src s2, int nx,
-                       int ny, int nz, float* dx, hipStream_t s) {
+                       int ny, int nz, float* dx, hipStream_t s, const float* dc = nullptr) {
   const UNetLayer& l = n.L[li];
-  const int64_t nv = (int64_t)n.B * nx * ny * nz;
-  hipLaunchKernelGGL(k_relu_back, dim3(nblk(nv * l.coutT)), dim3(UB), 0, s, dy, ldy, l.relu ? y : nullptr,
-                     l.cout, l.coutT, n.dzf, n.dzb, nv);
+  int sh = 0;
+  while ((4 << sh) < l.coutT) sh++;
+  G2G_CHECK((4 << sh) == l.coutT && (!l.relu || l.cout == l.coutT), -3, "layer widths are powers of two");
+  hipLaunchKernelGGL(k_relu_back<SRC>, dim3(nblk((int64_t)(nx * ny) << sh), nz, n.B), dim3(UB), 0, s, dy, ldy, dc,
+                     l.relu ? y : nullptr, l.cout, sh, n.dzf, n.dzb, nx, ny);
   conv_dw(n, li, n.dzf, l.coutT, s1, s2, nx, ny, nz, s);
   if (dx) conv_dx(n, li, n.dzb, nx, ny, nz, dx, s);
 }
@@ -1172,27 +1178,20 @@ void unet_backward(UNet& n, hipStream_t s) {
   const int X0 = n.nx, Y0 = n.ny, Z0 = n.nz, X1 = X0 / 2, Y1 = Y0 / 2, Z1 = Z0 / 2, X2 = X1 / 2,
             Y2 = Y1 / 2, Z2 = Z1 / 2;
   const int64_t v0 = (int64_t)X0 * Y0 * Z0, v1 = v0 / 8, v2 = v0 / 64;
-  const int64_t B = n.B;
   const Src none = src(nullptr, 0, 0, 0);
   bf16** A = n.act;
   layer_back(n, 10, n.dout, 8, nullptr, src(A[9], 16, 0, v0 * 16), none, X0, Y0, Z0, n.fa, s);
   layer_back(n, 9, n.fa, 16, A[9], src(A[8], 16, 0, v0 * 16), none, X0, Y0, Z0, n.fa, s);
   layer_back(n, 8, n.fa, 16, A[8], src(A[7], 32, 1, v1 * 32), src(A[1], 16, 0, v0 * 16), X0, Y0, Z0, n.f48,
              s);
-  hipLaunchKernelGGL(k_split_cat, dim3(nblk(B * v1 * 32 + B * v0 * 16)), dim3(UB), 0, s, n.f48, 32, 16, n.fb,
-                     n.de1, X0, Y0, Z0, B);
-  layer_back(n, 7, n.fb, 32, A[7], src(A[6], 32, 0, v1 * 32), none, X1, Y1, Z1, n.fb, s);
-  layer_back(n, 6, n.fb, 32, A[6], src(A[5], 64, 1, v2 * 64), src(A[3], 32, 0, v1 * 32), X1, Y1, Z1, n.f48,
+  layer_back<GradUpsample>(n, 7, n.f48, 48, A[7], src(A[6], 32, 0, v1 * 32), none, X1, Y1, Z1, n.fb, s);
+  layer_back(n, 6, n.fb, 32, A[6], src(A[5], 64, 1, v2 * 64), src(A[3], 32, 0, v1 * 32), X1, Y1, Z1, n.f96,
              s);
-  hipLaunchKernelGGL(k_split_cat, dim3(nblk(B * v2 * 64 + B * v1 * 32)), dim3(UB), 0, s, n.f48, 64, 32, n.fb,
-                     n.de2, X1, Y1, Z1, B);
-  layer_back(n, 5, n.fb, 64, A[5], src(A[4], 64, 0, v2 * 64), none, X2, Y2, Z2, n.fb, s);
+  layer_back<GradUpsample>(n, 5, n.f96, 96, A[5], src(A[4], 64, 0, v2 * 64), none, X2, Y2, Z2, n.fb, s);
   layer_back(n, 4, n.fb, 64, A[4], src(n.p2, 32, 0, v2 * 32), none, X2, Y2, Z2, n.fb, s);
-  hipLaunchKernelGGL(k_pool_back_add, dim3(nblk(B * v1 * 32)), dim3(UB), 0, s, n.fb, n.de2, 32, X1, Y1, Z1, B);
-  layer_back(n, 3, n.de2, 32, A[3], src(A[2], 32, 0, v1 * 32), none, X1, Y1, Z1, n.fb, s);
+  layer_back<GradPool>(n, 3, n.f96 + 64, 96, A[3], src(A[2], 32, 0, v1 * 32), none, X1, Y1, Z1, n.fb, s, n.fb);
   layer_back(n, 2, n.fb, 32, A[2], src(n.p1, 16, 0, v1 * 16), none, X1, Y1, Z1, n.fb, s);
-  hipLaunchKernelGGL(k_pool_back_add, dim3(nblk(B * v0 * 16)), dim3(UB), 0, s, n.fb, n.de1, 16, X0, Y0, Z0, B);
-  layer_back(n, 1, n.de1, 16, A[1], src(A[0], 16, 0, v0 * 16), none, X0, Y0, Z0, n.fa, s);
+  layer_back<GradPool>(n, 1, n.f48 + 32, 48, A[1], src(A[0], 16, 0, v0 * 16), none, X0, Y0, Z0, n.fa, s, n.fb);
   layer_back(n, 0, n.fa, 16, A[0], src(n.in, 8, 0, v0 * 8), none, X0, Y0, Z0, nullptr, s);
   G2G_HIP(hipGetLastError());
 }

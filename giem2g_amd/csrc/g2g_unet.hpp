@@ -35,8 +35,8 @@ struct UNet {
   size_t ws_bytes = 0;
   bf16 *in = nullptr, *act[11] = {}, *p1 = nullptr, *p2 = nullptr;
   float* out = nullptr;
-  float *dout = nullptr, *f48 = nullptr, *fa = nullptr, *fb = nullptr, *de1 = nullptr,
-        *de2 = nullptr, *dzf = nullptr, *dwp = nullptr;
+  float *dout = nullptr, *f48 = nullptr, *fa = nullptr, *fb = nullptr, *f96 = nullptr,
+        *dzf = nullptr, *dwp = nullptr;
   bf16* dzb = nullptr;
   double* dscal = nullptr;  // loss accumulator / residual scale
 };

@@ -220,3 +220,33 @@ def test_weight_gradient_sums(B, Z, Y, X):
     b9 = g[offs[9] + 16 * 27 * 16:offs[10]]
     assert np.all(np.abs(b9[:6] - D9.sum(0)) <= bar * np.abs(D9).sum(0)) and not np.any(b9[6:])
     net.close()
+
+
+@pytest.mark.parametrize("B,Z,Y,X", [(3, 12, 4, 8), (1, 8, 12, 20), (2, 4, 28, 4)])
+def test_gradient_through_the_levels(B, Z, Y, X):
+    """Layers whose output's gradient comes from a concatenation (the sum of
+    the upsampled voxel's eight children) or from a concatenation and a pooling,
+    on volumes of different sides: every layer's gradients against the oracle
+    (the 5e-2 bar above) and the same bits twice."""
+    torch = _torch()
+    from giem2g_amd import learned
+    from oracle import unet_ref as U
+    print("case", B, Z, Y, X, flush=True)
+    rng = np.random.default_rng(X)
+    p = _params(5)
+    x = rng.standard_normal((B, Z, Y, X, 8)).astype(np.float32)
+    dy = rng.standard_normal((B, Z, Y, X, 6)).astype(np.float32)
+    net = learned.UNet(params=p)
+    net.forward(torch.from_numpy(x).cuda(), keep=True)
+    g = net.backward(torch.from_numpy(dy).cuda())
+    assert np.array_equal(net.backward(torch.from_numpy(dy).cuda()), g)
+    gref = np.zeros(p.size)
+    for b in range(B):
+        _, cache = U.forward(p.astype(np.float64), x[b].astype(np.float64), round_bf16=True)
+        gref += U.backward(p, cache, dy[b].astype(np.float64), round_bf16=True)
+    off = 0
+    for li, (W, bb) in enumerate(U.split(gref)):
+        for ref in (W.ravel(), bb):
+            assert rel(g[off:off + ref.size].astype(np.float64), ref) < 5e-2, ("layer", li)
+            off += ref.size
+    net.close()
