@@ -144,15 +144,18 @@ __device__ inline void tap_window(int* kw, int K, bool on) {
 }
 
 // One block per offset b = lx + Nx*ly.  Output wts[c][K][b] (IE order) and
-// the offset's window of taps win[b].
+// the offset's window of taps win[b].  A thread keeps the weights of its taps K =
+// threadIdx.x + 256 u in registers and the twiddles stay in global memory:
+// with the transforms' 49 KB of LDS two blocks share a CU (with weights and
+// twiddles in LDS, 89 KB, one did: one wave per SIMD).  128x128 offsets: 3.61 ->
+// 2.19 ms; twiddles in LDS 2.30, registers for three blocks 2.26.
 __global__ __launch_bounds__(256) void k_weights(double* __restrict__ wts, int2* __restrict__ win,
                                                  const zd* __restrict__ f1,
                                                  const zd* __restrict__ twg,
                                                  const double* __restrict__ lms, WParams P) {
   constexpr int NRW = 3, LS = VBN + 1;
   __shared__ zd buf[NRW * LS];
-  __shared__ zd tw[VBN];
-  __shared__ double wt[6][NTAPS];
+  double wt[6][2];
   __shared__ double red[8];
   const int b = blockIdx.x, lx = b % P.Nx, ly = b / P.Nx;
   const double x = lx * P.dx + P.dx / 2.0, y = ly * P.dy + P.dy / 2.0;
@@ -161,7 +164,6 @@ __global__ __launch_bounds__(256) void k_weights(double* __restrict__ wts, int2*
   const double alpha = P.dx / rho, beta = P.dy / rho, phi = atan2(y, x);
   const double cphi = cos(phi), sphi = sin(phi);
   const double s = log(rho) - P.log_rmin;
-  for (int i = threadIdx.x; i < VBN; i += 256) tw[i] = twg[i];
   for (int half = 0; half < 2; half++) {
     __syncthreads();
     for (int i = threadIdx.x; i < VBN; i += 256) {
@@ -175,33 +177,38 @@ __global__ __launch_bounds__(256) void k_weights(double* __restrict__ wts, int2*
       for (int c = 0; c < NRW; c++) buf[c * LS + i] = mkz(sg * R[half * 3 + c], 0.0);
     }
     __syncthreads();
-    lds_fft<zd, VBN, NRW, LS, 256, +1>(buf, tw);
+    lds_fft<zd, VBN, NRW, LS, 256, +1>(buf, twg);
     for (int i = threadIdx.x; i < NRW * VBN; i += 256) {
       const int c = i / VBN, J = i - c * VBN;
       const zd h = cdiv(buf[c * LS + J], f1[J]);
       buf[c * LS + J] = (J & 1) ? -h : h;
     }
     __syncthreads();
-    lds_fft<zd, VBN, NRW, LS, 256, -1>(buf, tw);
-    for (int i = threadIdx.x; i < NRW * NTAPS; i += 256) {
-      const int c = i / NTAPS, K = i - c * NTAPS, J = K + NFIRST;
-      double h = buf[c * LS + J].x / (double)VBN;
-      if (J & 1) h = -h;
-      const int col = half * 3 + c;  // reference output order D0,DXX,DXY,DX,DYY,DY
-      h = h / P.dx / P.dy * rp[col];
-      const int ie = col == 0 ? IE_D0 : col == 1 ? IE_DXX : col == 2 ? IE_DXY
-                   : col == 3 ? IE_DX : col == 4 ? IE_DYY : IE_DY;
-      wt[ie][K] = h;
+    lds_fft<zd, VBN, NRW, LS, 256, -1>(buf, twg);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int K = threadIdx.x + 256 * u, J = K + NFIRST;
+      // reference output order D0,DXX,DXY,DX,DYY,DY
+      auto tap = [&](int c) {
+        if (K >= NTAPS) return 0.0;
+        double h = buf[c * LS + J].x / (double)VBN;
+        if (J & 1) h = -h;
+        return h / P.dx / P.dy * rp[half * 3 + c];
+      };
+      if (half == 0) {
+        wt[IE_D0][u] = tap(0);
+        wt[IE_DXX][u] = tap(1);
+        wt[IE_DXY][u] = tap(2);
+      } else {
+        wt[IE_DX][u] = tap(0);
+        wt[IE_DYY][u] = tap(1);
+        wt[IE_DY][u] = tap(2);
+      }
     }
   }
-  __syncthreads();
   // COMPUTE_WEIGHTS W0 logic (calc_ie_tensor_module.F90:327-351)
   double W0[6];
-  auto colmax = [&](int c) {
-    double m = 0;
-    for (int K = threadIdx.x; K < NTAPS; K += 256) m = fmax(m, fabs(wt[c][K]));
-    return block_max(m, red);
-  };
+  auto colmax = [&](int c) { return block_max(fmax(fabs(wt[c][0]), fabs(wt[c][1])), red); };
   W0[IE_DXX] = colmax(IE_DXX);
   if (lx != 0 && ly != 0) {
     double m = fmax(fmax(colmax(IE_DXY), colmax(IE_DYY)), fmax(colmax(IE_DX), colmax(IE_DY)));
@@ -222,9 +229,12 @@ __global__ __launch_bounds__(256) void k_weights(double* __restrict__ wts, int2*
   __shared__ int kw[2];
   if (threadIdx.x < 2) kw[threadIdx.x] = threadIdx.x == 0 ? NTAPS : 0;
   __syncthreads();
-  for (int K = threadIdx.x; K < NTAPS; K += 256) {
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int K = threadIdx.x + 256 * u;
+    if (K >= NTAPS) break;
     double w[6];
-    for (int c = 0; c < 6; c++) w[c] = wt[c][K];
+    for (int c = 0; c < 6; c++) w[c] = wt[c][u];
     if (lx == 0) {  // :330-342
       w[IE_DXY] = 0;
       w[IE_DX] = 0;
@@ -940,15 +950,15 @@ struct RcWParams {
 // One block per offset point p = ix*2Ny + iy of one receiver.  Output
 // wts[c][K][p] in IE order, masked (1e-12 of the largest weight of the
 // offset, calc_rc_tensor_module.F90:202-212) and lambda-scaled (:214-219);
-// zero on the ix = Nx and iy = Ny offsets.
+// zero on the ix = Nx and iy = Ny offsets.  LDS and registers as in k_weights
+// (65536 offsets: 12.1 -> 7.1 ms).
 __global__ __launch_bounds__(256) void k_rc_weights(double* __restrict__ wts, int2* __restrict__ win,
                                                     const zd* __restrict__ f1,
                                                     const zd* __restrict__ twg,
                                                     const double* __restrict__ lms, RcWParams P) {
   constexpr int NRW = 3, LS = VBN + 1;
   __shared__ zd buf[NRW * LS];
-  __shared__ zd tw[VBN];
-  __shared__ double wt[6][NTAPS];
+  double wt[6][2];
   __shared__ double red[8];
   const int Ny2 = 2 * P.Ny;
   const int64_t NP = (int64_t)4 * P.Nx * P.Ny;
@@ -964,7 +974,6 @@ __global__ __launch_bounds__(256) void k_rc_weights(double* __restrict__ wts, in
   const double alpha = P.dx / rho, beta = P.dy / rho, phi = atan2(y, x);
   const double cphi = cos(phi), sphi = sin(phi);
   const double s = log(rho) - P.log_rmin;
-  for (int i = threadIdx.x; i < VBN; i += 256) tw[i] = twg[i];
   for (int half = 0; half < 2; half++) {
     __syncthreads();
     for (int i = threadIdx.x; i < VBN; i += 256) {
@@ -978,46 +987,57 @@ __global__ __launch_bounds__(256) void k_rc_weights(double* __restrict__ wts, in
       for (int c = 0; c < NRW; c++) buf[c * LS + i] = mkz(sg * R[half * 3 + c], 0.0);
     }
     __syncthreads();
-    lds_fft<zd, VBN, NRW, LS, 256, +1>(buf, tw);
+    lds_fft<zd, VBN, NRW, LS, 256, +1>(buf, twg);
     for (int i = threadIdx.x; i < NRW * VBN; i += 256) {
       const int c = i / VBN, J = i - c * VBN;
       const zd h = cdiv(buf[c * LS + J], f1[J]);
       buf[c * LS + J] = (J & 1) ? -h : h;
     }
     __syncthreads();
-    lds_fft<zd, VBN, NRW, LS, 256, -1>(buf, tw);
-    for (int i = threadIdx.x; i < NRW * NTAPS; i += 256) {
-      const int c = i / NTAPS, K = i - c * NTAPS, J = K + NFIRST;
-      double h = buf[c * LS + J].x / (double)VBN;
-      if (J & 1) h = -h;
-      const int col = half * 3 + c;  // reference output order D0,DXX,DXY,DX,DYY,DY
-      // scalings of VolumeBesselTransforms.F90:222-228
-      if (col == 0) h = h * rho;
-      else if (col == 1 || col == 2 || col == 4) h = h / rho;
-      const int ie = col == 0 ? IE_D0 : col == 1 ? IE_DXX : col == 2 ? IE_DXY
-                   : col == 3 ? IE_DX : col == 4 ? IE_DYY : IE_DY;
-      wt[ie][K] = h;
+    lds_fft<zd, VBN, NRW, LS, 256, -1>(buf, twg);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int K = threadIdx.x + 256 * u, J = K + NFIRST;
+      auto tap = [&](int c) {
+        if (K >= NTAPS) return 0.0;
+        double h = buf[c * LS + J].x / (double)VBN;
+        return (J & 1) ? -h : h;
+      };
+      // reference output order D0,DXX,DXY,DX,DYY,DY; scalings of
+      // VolumeBesselTransforms.F90:222-228
+      if (half == 0) {
+        wt[IE_D0][u] = tap(0) * rho;
+        wt[IE_DXX][u] = tap(1) / rho;
+        wt[IE_DXY][u] = tap(2) / rho;
+      } else {
+        wt[IE_DX][u] = tap(0);
+        wt[IE_DYY][u] = tap(1) / rho;
+        wt[IE_DY][u] = tap(2);
+      }
     }
   }
-  __syncthreads();
   double m = 0;
-  for (int i = threadIdx.x; i < 6 * NTAPS; i += 256) m = fmax(m, fabs(wt[i / NTAPS][i % NTAPS]));
+#pragma unroll
+  for (int c = 0; c < 6; c++) m = fmax(m, fmax(fabs(wt[c][0]), fabs(wt[c][1])));
   const double W0 = block_max(m, red);
   __shared__ int kw[2];
   if (threadIdx.x < 2) kw[threadIdx.x] = threadIdx.x == 0 ? NTAPS : 0;
   __syncthreads();
-  for (int K = threadIdx.x; K < NTAPS; K += 256) {
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int K = threadIdx.x + 256 * u;
+    if (K >= NTAPS) break;
     double Wm = 0;
-    for (int c = 0; c < 6; c++) Wm = fmax(Wm, fabs(wt[c][K] / W0));
+    for (int c = 0; c < 6; c++) Wm = fmax(Wm, fabs(wt[c][u] / W0));
     const bool on = Wm > 1e-12;
     const double lm = lms[K];
     double o[6];
-    o[IE_DXX] = wt[IE_DXX][K] / lm;
-    o[IE_DYY] = wt[IE_DYY][K] / lm;
-    o[IE_DXY] = wt[IE_DXY][K] / lm;
-    o[IE_DX] = wt[IE_DX][K] * lm;
-    o[IE_DY] = wt[IE_DY][K] * lm;
-    o[IE_D0] = wt[IE_D0][K] * lm;
+    o[IE_DXX] = wt[IE_DXX][u] / lm;
+    o[IE_DYY] = wt[IE_DYY][u] / lm;
+    o[IE_DXY] = wt[IE_DXY][u] / lm;
+    o[IE_DX] = wt[IE_DX][u] * lm;
+    o[IE_DY] = wt[IE_DY][u] * lm;
+    o[IE_D0] = wt[IE_D0][u] * lm;
     for (int c = 0; c < 6; c++) wts[((int64_t)c * NTAPS + K) * NP + p] = on ? o[c] : 0.0;
     tap_window(kw, K, on);
   }
