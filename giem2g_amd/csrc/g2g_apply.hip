@@ -2711,18 +2711,23 @@ __global__ void k_dsig(const zd* __restrict__ csiga, const zd* __restrict__ csig
   dsig[i] = csiga[i] - csigb[z];
 }
 
-void rc_init(RcOperator& rc, Operator& op, int Nr, const double* xs, const double* ys, const double* depth) {
-  G2G_CHECK(Nr >= 1 && Nr <= 64, -3, "Nr must be in [1,64]");
+void rc_check_corners(const Operator& op, int Nr, const double* xs, const double* ys) {
+  // the weights need a nonzero distance to the source cell corner
+  // (VBTransformWeightsAllSingleInt takes log(rho))
   for (int r = 0; r < Nr; r++) {
-    G2G_CHECK(std::isfinite(xs[r]) && std::isfinite(ys[r]) && std::isfinite(depth[r]) && depth[r] >= 0, -3,
-              "receiver shifts must be finite and depths non-negative");
-    // the weights need a nonzero distance to the source cell corner
-    // (VBTransformWeightsAllSingleInt takes log(rho))
     const double fx = xs[r] / op.dx - 0.5, fy = ys[r] / op.dy - 0.5;
     const bool cx = std::fabs(fx - std::nearbyint(fx)) < 1e-12 && std::fabs(std::nearbyint(fx)) < op.Nx;
     const bool cy = std::fabs(fy - std::nearbyint(fy)) < 1e-12 && std::fabs(std::nearbyint(fy)) < op.Ny;
     G2G_CHECK(!(cx && cy), -3, "receiver on a cell corner: the filter weights are singular there");
   }
+}
+
+void rc_init(RcOperator& rc, Operator& op, int Nr, const double* xs, const double* ys, const double* depth) {
+  G2G_CHECK(Nr >= 1 && Nr <= 64, -3, "Nr must be in [1,64]");
+  for (int r = 0; r < Nr; r++)
+    G2G_CHECK(std::isfinite(xs[r]) && std::isfinite(ys[r]) && std::isfinite(depth[r]) && depth[r] >= 0, -3,
+              "receiver shifts must be finite and depths non-negative");
+  rc_check_corners(op, Nr, xs, ys);
   rc.op = &op;
   rc.Nr = Nr;
   rc.xs.assign(xs, xs + Nr);

@@ -276,6 +276,7 @@ struct RcOperator {
   zd *Xf = nullptr, *S = nullptr, *So = nullptr, *Xi = nullptr;  // FFT work buffers
   int NR = 0, nchunk_f = 0, nchunk_i = 0;
   bool have_wts = false, have_tensor = false, spectral = false, have_sigma = false;
+  double wts_dx = 0, wts_dy = 0;  // the cell sizes the kept weights were made for
   int tensor_version = -1, sigma_version = -1;  // background version each was made for
   double t_tensor = 0, t_fft = 0, t_apply = 0;
   int64_t applies = 0;
@@ -358,6 +359,8 @@ void op_free_tensor_scratch(Operator& op);
 void rc_init(RcOperator& rc, Operator& op, int Nr, const double* xs, const double* ys,
              const double* depth);                                     // g2g_apply.hip
 void rc_fini(RcOperator& rc);                                          // g2g_apply.hip
+// refuses receivers on a corner of the operator's cells (their filter weights are singular)
+void rc_check_corners(const Operator& op, int Nr, const double* xs, const double* ys);  // g2g_apply.hip
 void rc_prepare_receivers(RcOperator& rc);                             // g2g_tensor.hip
 void rc_build_tensor(RcOperator& rc);                                  // g2g_tensor.hip
 void rc_tensor_fft(RcOperator& rc);                                    // g2g_tensor.hip

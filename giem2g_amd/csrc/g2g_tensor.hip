@@ -1222,6 +1222,11 @@ void rc_build_tensor(RcOperator& rc) {
   Operator& op = *rc.op;
   G2G_CHECK(op.have_bkg, -4, "background not set");
   G2G_CHECK(op.Nl <= 64 && op.Nz <= MAX_NZ, -3, "tensor build supports Nl <= 64 and Nz <= 256");
+  // weights of other cell sizes (the operator's geometry has changed since) are made anew
+  if (rc.wts_dx != op.dx || rc.wts_dy != op.dy) {
+    rc_check_corners(op, rc.Nr, rc.xs.data(), rc.ys.data());
+    rc.have_wts = false;
+  }
   rc_prepare_receivers(rc);
   const int Nz = op.Nz, Nr = rc.Nr;
   const int64_t NP = rc.NP, BS = rc.BS, WS = (int64_t)6 * NTAPS * NP + NP;  // weights per receiver, then the points' windows of taps
@@ -1296,6 +1301,8 @@ void rc_build_tensor(RcOperator& rc) {
   G2G_HIP(hipEventElapsedTime(&ms, op.ev[0], op.ev[1]));
   rc.t_tensor = ms * 1e-3;
   rc.have_wts = rc.have_wts || cache;
+  rc.wts_dx = op.dx;
+  rc.wts_dy = op.dy;
   rc.have_tensor = true;
   rc.spectral = false;
   rc.tensor_version = op.bkg_version;

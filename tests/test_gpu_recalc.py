@@ -192,3 +192,48 @@ def test_receiver_errors():
         op.close()  # the receiver operator still holds it
     rc.close()
     op.close()
+
+
+def test_new_cell_sizes_on_a_kept_receiver_operator(oracle):
+    """set_geometry with other cell sizes: the next build of an existing
+    receiver operator makes its filter weights anew.  Real-space tensor and
+    spectrum with the same bits as a fresh receiver operator's and within 1e-10
+    of the oracle (the bar above); back at the first sizes the first tensor
+    again; and a receiver that the new sizes put on a cell corner is refused
+    as at creation."""
+    from giem2g_amd import lib as L, models, operator as gop
+    m = models.small(8, 10, 3, seed=21, freq=0.9)
+    xs, ys, depth = RECV[3]
+    op, rc = make_ops(m, xs, ys, depth)
+    rc.calc_kernel()
+    first = rc.get_tensor()
+    for dx, dy in ((m.dx, 1.5 * m.dy), (0.75 * m.dx, 1.5 * m.dy)):
+        op.set_geometry(dx, dy, m.z)
+        op.set_background(m.csigb(), m.thick, m.omega)
+        fresh = gop.ReceiverOperator(op, xs, ys, depth)
+        rc.calc_kernel()
+        fresh.calc_kernel()
+        om = oracle.Model(m.csigb(), m.thick, m.omega, m.Nx, m.Ny, m.Nz, dx, dy, m.z)
+        e = rel(rc.get_tensor(), oracle.Receivers(om, xs, ys, depth).tensor_realspace())
+        print("  dx %g dy %g: tensor %.2e" % (dx, dy, e), flush=True)
+        assert e < 1e-10
+        assert np.array_equal(rc.get_tensor(), fresh.get_tensor())
+        rc.calc_fft_of_kernel()
+        fresh.calc_fft_of_kernel()
+        assert np.array_equal(rc.get_tensor(), fresh.get_tensor())
+        fresh.close()
+    op.set_geometry(m.dx, m.dy, m.z)
+    op.set_background(m.csigb(), m.thick, m.omega)
+    rc.calc_kernel()
+    assert np.array_equal(rc.get_tensor(), first)
+    rc.close()
+    # shifts (50, 75): inside a cell of 100 x 100, on the corner of one of 100 x 150
+    rc = gop.ReceiverOperator(op, [50.0], [75.0], [0.0])
+    rc.build()
+    op.set_geometry(100.0, 150.0, m.z)
+    with pytest.raises(L.G2GError, match="corner"):
+        rc.calc_kernel()
+    op.set_geometry(m.dx, m.dy, m.z)
+    rc.build()
+    rc.close()
+    op.close()
