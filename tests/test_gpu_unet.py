@@ -250,3 +250,61 @@ def test_gradient_through_the_levels(B, Z, Y, X):
             assert rel(g[off:off + ref.size].astype(np.float64), ref) < 5e-2, ("layer", li)
             off += ref.size
     net.close()
+
+
+@pytest.mark.parametrize("B,Z,Y,X,q", [(1, 4, 4, 20, (0, 0, 19)), (2, 12, 20, 12, (11, 19, 0)), (1, 8, 4, 36, (4, 2, 17)),
+                                       (1, 4, 28, 16, (3, 27, 15))])
+def test_infinite_activation_in_the_gradient(B, Z, Y, X, q):
+    """One infinite input voxel through a network of positive weights: every
+    layer's input is positive and infinite near that voxel, the output
+    gradient is positive and finite.  A product of an infinite activation
+    with a nonzero gradient is infinite, and voxels outside the volume (in
+    tiles with remainders) have none: no entry of the gradient is NaN, the
+    first layer's infinite entries are those whose tap reaches the voxel from
+    inside the volume, and the rest are the sums of a run whose voxel is
+    finite, to the bar of the sums above."""
+    torch = _torch()
+    from giem2g_amd import learned
+    print("case", B, Z, Y, X, q, flush=True)
+    rng = np.random.default_rng(X)
+    parts = []
+    for ci, co, t in learned.ARCH:
+        parts += [rng.uniform(0.5, 1.5, co * t * ci) / (t * ci), np.full(co, 0.01)]
+    net = learned.UNet(params=np.concatenate(parts).astype(np.float32))
+    x = torch.from_numpy(rng.uniform(0.5, 1.0, (B, Z, Y, X, 8)).astype(np.float32)).cuda()
+    dy = torch.from_numpy(rng.uniform(0.5, 1.0, (B, Z, Y, X, 6)).astype(np.float32)).cuda()
+    ch, bat = 5, B - 1
+    net.forward(x, keep=True)
+    gf = net.backward(dy).astype(np.float64)
+    x[(bat,) + q + (ch,)] = float("inf")
+    y = net.forward(x, keep=True)
+    assert not torch.isnan(y).any()
+    g = net.backward(dy).astype(np.float64)
+    assert not np.isnan(g).any() and np.all(g >= 0)
+    n = B * Z * Y * X
+    bar = 2 * (n / 32 + 64) * 2.0 ** -24
+    off = 0
+    for li, (ci, co, t) in enumerate(learned.ARCH):
+        w, wf = g[off:off + co * t * ci].reshape(co, t, ci), gf[off:off + co * t * ci].reshape(co, t, ci)
+        off += co * t * ci
+        b, bf = g[off:off + co], gf[off:off + co]
+        off += co
+        assert np.all(np.abs(b - bf) <= bar * bf), ("bias", li)
+        if li:
+            assert np.isinf(w).any(), li
+            continue
+        for k in range(27):
+            p = [q[0] - (k // 9 - 1), q[1] - ((k // 3) % 3 - 1), q[2] - (k % 3 - 1)]
+            inside = all(0 <= a < s for a, s in zip(p, (Z, Y, X)))
+            assert np.all(np.isinf(w[:, k, ch]) == inside), (k, inside)
+        fin = np.isfinite(w)
+        fin[:, :, ch] = False
+        assert np.all(np.delete(fin, ch, 2))
+        assert np.all(np.abs(w[fin] - wf[fin]) <= bar * wf[fin])
+    # back on finite data, the same bits as before
+    x[(bat,) + q + (ch,)] = 0.75
+    net.forward(x, keep=True)
+    g1 = net.backward(dy)
+    net.forward(x, keep=True)
+    assert np.array_equal(net.backward(dy), g1) and np.isfinite(g1).all()
+    net.close()
