@@ -2728,6 +2728,7 @@ void rc_init(RcOperator& rc, Operator& op, int Nr, const double* xs, const doubl
     G2G_CHECK(std::isfinite(xs[r]) && std::isfinite(ys[r]) && std::isfinite(depth[r]) && depth[r] >= 0, -3,
               "receiver shifts must be finite and depths non-negative");
   rc_check_corners(op, Nr, xs, ys);
+  for (auto& e : rc.ev) G2G_HIP(hipEventCreate(&e));
   rc.op = &op;
   rc.Nr = Nr;
   rc.xs.assign(xs, xs + Nr);
@@ -2759,6 +2760,10 @@ void rc_fini(RcOperator& rc) {
   if (rc.wts) (void)hipFree(rc.wts);
   rc.wts = nullptr;
   rc.par.release();
+  for (auto& e : rc.ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
 }
 
 // FinalizeRCOperator (:168-196): the conductivity of the current frequency

@@ -248,7 +248,7 @@ struct Operator {
   Arena ws[2];
   size_t tabs_bytes = 0;
   DevTables par, spar;  // tables of the tensor build, of the conductivity
-  hipEvent_t ev[8] = {};  // (0, 1 and 2 also time the tensor builds)
+  hipEvent_t ev[8] = {};  // (0, 1 and 2 also time the IE tensor's builds)
 
   int64_t ncell() const { return (int64_t)Nx * Ny * Nz; }
   int64_t nvec() const { return 3 * ncell(); }
@@ -281,6 +281,9 @@ struct RcOperator {
   double t_tensor = 0, t_fft = 0, t_apply = 0;
   int64_t applies = 0;
   size_t bytes = 0;
+  // time the builds (not the operator's: its other receiver operators may be
+  // built by other host threads meanwhile)
+  hipEvent_t ev[2] = {};
 };
 
 // GetLayerSingle (data_types_module.F90:75-103): background layer of depth z

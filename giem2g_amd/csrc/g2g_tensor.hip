@@ -1232,7 +1232,7 @@ void rc_build_tensor(RcOperator& rc) {
   const int64_t NP = rc.NP, BS = rc.BS, WS = (int64_t)6 * NTAPS * NP + NP;  // weights per receiver, then the points' windows of taps
   const double rmin = std::sqrt(op.dx * op.dx + op.dy * op.dy) / 2.0;  // :67
   const BuildTables bt = build_tables(op, rc.par, rmin);
-  G2G_HIP(hipEventRecord(op.ev[0], op.stream));
+  G2G_HIP(hipEventRecord(rc.ev[0], op.stream));
   // The weights do not depend on frequency: all receivers' weights are kept
   // when they fit in 8 GB, else one receiver's are recomputed per build.
   const bool cache = (double)Nr * WS * sizeof(double) <= 8.0 * (1 << 30);
@@ -1295,10 +1295,10 @@ void rc_build_tensor(RcOperator& rc) {
                        (const int2*)(W + 6 * NTAPS * NP), 0, scale, jobs);
   }
   G2G_HIP(hipGetLastError());
-  G2G_HIP(hipEventRecord(op.ev[1], op.stream));
+  G2G_HIP(hipEventRecord(rc.ev[1], op.stream));
   G2G_HIP(hipStreamSynchronize(op.stream));
   float ms = 0;
-  G2G_HIP(hipEventElapsedTime(&ms, op.ev[0], op.ev[1]));
+  G2G_HIP(hipEventElapsedTime(&ms, rc.ev[0], rc.ev[1]));
   rc.t_tensor = ms * 1e-3;
   rc.have_wts = rc.have_wts || cache;
   rc.wts_dx = op.dx;
@@ -1316,7 +1316,7 @@ void rc_tensor_fft(RcOperator& rc) {
   const int Nx2 = 2 * op.Nx, Ny2 = 2 * op.Ny;
   const zd *twx = op.d64.twx, *twy = op.d64.twy;
   const FftPlan &py = op.py, &px = op.px;
-  G2G_HIP(hipEventRecord(op.ev[0], op.stream));
+  G2G_HIP(hipEventRecord(rc.ev[0], op.stream));
   len_dispatch(Ny2, [&](auto LC) {
     constexpr int LL = decltype(LC)::value;
     constexpr int NE = ne_for<LL>();
@@ -1330,10 +1330,10 @@ void rc_tensor_fft(RcOperator& rc) {
                        dim3(256), 0, op.stream, rc.G, twx, Ny2, rc.BS, px);
   });
   G2G_HIP(hipGetLastError());
-  G2G_HIP(hipEventRecord(op.ev[1], op.stream));
+  G2G_HIP(hipEventRecord(rc.ev[1], op.stream));
   G2G_HIP(hipStreamSynchronize(op.stream));
   float ms = 0;
-  G2G_HIP(hipEventElapsedTime(&ms, op.ev[0], op.ev[1]));
+  G2G_HIP(hipEventElapsedTime(&ms, rc.ev[0], rc.ev[1]));
   rc.t_fft = ms * 1e-3;
   rc.spectral = true;
 }

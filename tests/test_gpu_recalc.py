@@ -237,3 +237,39 @@ def test_new_cell_sizes_on_a_kept_receiver_operator(oracle):
     rc.build()
     rc.close()
     op.close()
+
+
+def test_receiver_operators_built_from_two_threads():
+    """Two receiver operators of one IE operator, built again and again by two
+    host threads at once: every build ends without an error and with the bits
+    of a build alone."""
+    import threading
+    from giem2g_amd import models, operator as gop
+    m = models.small(16, 12, 4, seed=8, freq=0.9)
+    op, rc0 = make_ops(m, *RECV[3])
+    rcs = [rc0, gop.ReceiverOperator(op, *RECV[1])]
+    alone = []
+    for rc in rcs:
+        rc.build()
+        alone.append(rc.get_tensor())
+    errors = []
+
+    def work(rc, ref):
+        try:
+            for _ in range(60):
+                rc.build()
+            if not np.array_equal(rc.get_tensor(), ref):
+                errors.append("tensor differs")
+        except Exception as e:
+            errors.append(e)
+
+    th = [threading.Thread(target=work, args=a) for a in zip(rcs, alone)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not errors, errors
+    for rc in rcs:
+        assert rc.stats()["t_tensor"] > 0 and rc.stats()["t_tensor_fft"] > 0
+        rc.close()
+    op.close()
