@@ -2760,6 +2760,7 @@ void rc_fini(RcOperator& rc) {
   if (rc.wts) (void)hipFree(rc.wts);
   rc.wts = nullptr;
   rc.par.release();
+  rc.spar.release();
   for (auto& e : rc.ev) {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
@@ -2770,10 +2771,10 @@ void rc_fini(RcOperator& rc) {
 void rc_set_sigma(RcOperator& rc, const zd* d_csiga) {
   Operator& op = *rc.op;
   G2G_CHECK(op.have_bkg, -4, "background not set");
-  rc.par.h.clear();
-  const size_t o0 = rc.par.add(op.csigb.data(), op.Nz);
-  rc.par.send();
-  const zd* d_csigb = rc.par.at<zd>(o0);
+  rc.spar.h.clear();
+  const size_t o0 = rc.spar.add(op.csigb.data(), op.Nz);
+  rc.spar.send();
+  const zd* d_csigb = rc.spar.at<zd>(o0);
   const int64_t n = op.ncell();
   hipLaunchKernelGGL(k_dsig, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, op.stream, d_csiga, d_csigb,
                      rc.dsig, (int64_t)op.Nx * op.Ny, op.Nz);

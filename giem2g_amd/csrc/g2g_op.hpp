@@ -180,7 +180,8 @@ template <typename R> struct OpBuffers {
 // keeps: add() each, then one copy.  (A buffer, a copy and a free of their own
 // for every table, and transform twiddles made anew, took the next frequency
 // at 128x128x32 0.2 ms of 2.5.)  The kernels that read the tables of one
-// send() must have ended before the next.
+// send() must have ended before the next, so calls that may run at the same time
+// (a build, a new conductivity) have a DevTables each.
 struct DevTables {
   char* d = nullptr;
   size_t cap = 0;
@@ -271,7 +272,7 @@ struct RcOperator {
   zd* G = nullptr;        // tensor, NP*BS
   double* wts = nullptr;  // masked, lambda-scaled weights [r][6][501][NP] (frequency independent)
   zd* tabs = nullptr;     // per-tap kernel tables of one receiver [501][13][Nz]
-  DevTables par;          // tables of the tensor build, of the conductivity
+  DevTables par, spar;    // tables of the tensor build, of the conductivity
   zd* dsig = nullptr;     // sigma_a - sigma_b per cell
   zd *Xf = nullptr, *S = nullptr, *So = nullptr, *Xi = nullptr;  // FFT work buffers
   int NR = 0, nchunk_f = 0, nchunk_i = 0;

@@ -273,3 +273,38 @@ def test_receiver_operators_built_from_two_threads():
         assert rc.stats()["t_tensor"] > 0 and rc.stats()["t_tensor_fft"] > 0
         rc.close()
     op.close()
+
+
+def test_receiver_build_and_conductivity_from_two_threads():
+    """One thread sets a receiver operator's conductivity while another builds
+    its tensor: each has device tables of its own, so both end with the bits of
+    the same calls one after the other."""
+    import threading
+    from giem2g_amd import models
+    m = models.small(16, 12, 4, seed=9, freq=0.9)
+    op, rc = make_ops(m, *RECV[3])
+    rc.build()
+    rc.set_sigma(m.csiga())
+    G = rc.get_tensor()
+    E = rand_vec(3 * m.ncell, 5)
+    Ea, Ha = rc.recalculate(E)
+    errors = []
+
+    def work(f):
+        try:
+            for _ in range(60):
+                f()
+        except Exception as e:
+            errors.append(e)
+
+    th = [threading.Thread(target=work, args=(f,)) for f in (rc.build, lambda: rc.set_sigma(m.csiga()))]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not errors, errors
+    assert np.array_equal(rc.get_tensor(), G)
+    Eb, Hb = rc.recalculate(E)
+    assert np.array_equal(Ea, Eb) and np.array_equal(Ha, Hb)
+    rc.close()
+    op.close()
