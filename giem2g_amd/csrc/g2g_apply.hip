@@ -2503,16 +2503,31 @@ void op_noalloc_setup(int device) {
   scratch_dev[device] = p;
 }
 
-template <typename R> int op_noalloc_batch_max(const Operator& op, const OpBuffers<R>& b, size_t* need1) {
-  const size_t es = sizeof(cx_t<R>);
-  const size_t nX = (size_t)b.nchunk * b.NR * op.Ny * 2 * op.Nx;
-  const size_t nS = (size_t)4 * op.Nx * op.Ny * 3 * op.Nz;
-  if (need1) *need1 = es * (nX + nS);
+// elements of X and of one spectrum slot in the array
+template <typename R> static size_t noalloc_x(const Operator& op, const OpBuffers<R>& b) {
+  return (size_t)b.nchunk * b.NR * op.Ny * 2 * op.Nx;
+}
+static size_t noalloc_s(const Operator& op) { return (size_t)12 * op.Nx * op.Ny * op.Nz; }
+template <typename R> static int noalloc_fit(const Operator& op, const OpBuffers<R>& b) {
   const int kmax = std::min(op_batch_max(op), sizeof(R) == 8 ? 4 : 8);
   int k = 0;
   for (int kk : {1, 2, 4, 8})
-    if (kk <= kmax && es * (nX + nS * kk) <= NOALLOC_SCRATCH_BYTES) k = kk;
+    if (kk <= kmax && sizeof(cx_t<R>) * (noalloc_x(op, b) + noalloc_s(op) * kk) <= NOALLOC_SCRATCH_BYTES) k = kk;
   return k;
+}
+// The form of the passes in the array: b's own, or 2N-point passes where more
+// vectors fit with these.  (Factor-plan rows of more than 512 points in
+// complex64: half-length tiles of X hold eight rows, 2N-point ones four, so X
+// may be padded with less.  With b's form alone 388x408x11 does not fit.)
+template <typename R> static OpBuffers<R> noalloc_form(const Operator& op, const OpBuffers<R>& b) {
+  OpBuffers<R> f = b;
+  if (b.half && !(is_pow2(op.Nx) && is_pow2(op.Ny))) {
+    f.half = false;
+    f.NR = nr_rt<R>(2 * op.Nx);
+    f.nchunk = (3 * op.Nz + f.NR - 1) / f.NR;
+    if (noalloc_fit(op, f) == noalloc_fit(op, b)) f = b;
+  }
+  return f;
 }
 
 template <typename R>
@@ -2523,14 +2538,17 @@ void op_apply_batch_noalloc(Operator& op, OpBuffers<R>& b, int nrhs, const cx_t<
   G2G_CHECK(b.X != nullptr, -4,
             "complex64 operator not made yet: make it with a complex64 apply or batch before the "
             "allocation-free apply");
-  size_t need1 = 0;
-  const int kcap = op_noalloc_batch_max<R>(op, b, &need1);
+  // the operator's buffers with X and the spectrum slots moved into scratch;
+  // the single-vector path's spectrum S is the first slot
+  OpBuffers<R> bl = noalloc_form(op, b);
+  const int kcap = noalloc_fit(op, bl);
+  const size_t nX = noalloc_x(op, bl), nS = noalloc_s(op);
   if (kcap < 1) {
     char msg[200];
     std::snprintf(msg, sizeof msg,
                   "grid too large for the allocation-free apply: one vector needs %zu bytes of scratch, "
                   "the library holds %zu",
-                  need1, (size_t)NOALLOC_SCRATCH_BYTES);
+                  sizeof(T2) * (nX + nS), (size_t)NOALLOC_SCRATCH_BYTES);
     throw Error(-3, msg);
   }
   G2G_CHECK(op.have_tensor && op.have_sigma, -4, "operator not ready: tensor or conductivity missing");
@@ -2539,13 +2557,8 @@ void op_apply_batch_noalloc(Operator& op, OpBuffers<R>& b, int nrhs, const cx_t<
   G2G_HIP(hipGetDevice(&dev));
   G2G_CHECK(dev >= 0 && dev < MAX_DEVICES && scratch_dev[dev] != nullptr, -4,
             "no operator was created on the current device");
-  // the operator's buffers with X and the spectrum slots moved into scratch;
-  // the single-vector path's spectrum S is the first slot
-  OpBuffers<R> bl = b;
   T2* base = static_cast<T2*>(scratch_dev[dev]);
-  const size_t nX = (size_t)b.nchunk * b.NR * op.Ny * 2 * op.Nx;
-  const size_t nS = (size_t)4 * op.Nx * op.Ny * 3 * op.Nz, all = NOALLOC_SCRATCH_BYTES / sizeof(T2);
-  bl.x_fixed = (int)std::min<size_t>(8, (all - nS * kcap) / nX);
+  bl.x_fixed = (int)std::min<size_t>(8, (NOALLOC_SCRATCH_BYTES / sizeof(T2) - nS * kcap) / nX);
   bl.X = base;
   bl.SB = base + nX * bl.x_fixed;
   bl.S = bl.SB;
@@ -2567,8 +2580,6 @@ void op_apply_batch_noalloc(Operator& op, OpBuffers<R>& b, int nrhs, const cx_t<
     r0 += k;
   }
 }
-template int op_noalloc_batch_max<double>(const Operator&, const OpBuffers<double>&, size_t*);
-template int op_noalloc_batch_max<float>(const Operator&, const OpBuffers<float>&, size_t*);
 template void op_apply_batch_noalloc<double>(Operator&, OpBuffers<double>&, int, const zd*, zd*, hipStream_t);
 template void op_apply_batch_noalloc<float>(Operator&, OpBuffers<float>&, int, const zf*, zf*, hipStream_t);
 

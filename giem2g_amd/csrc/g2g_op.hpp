@@ -335,9 +335,6 @@ void op_apply_batch(Operator& op, OpBuffers<R>& b, int nrhs, const cx_t<R>* vin,
 // on one GPU share the array and race.
 constexpr size_t NOALLOC_SCRATCH_BYTES = size_t(256) << 20;
 void op_noalloc_setup(int device);
-// vectors per tensor read the array allows (0 when one vector does not fit;
-// *need1 = bytes one vector needs)
-template <typename R> int op_noalloc_batch_max(const Operator& op, const OpBuffers<R>& b, size_t* need1);
 template <typename R>
 void op_apply_batch_noalloc(Operator& op, OpBuffers<R>& b, int nrhs, const cx_t<R>* vin, cx_t<R>* vout,
                             hipStream_t s);

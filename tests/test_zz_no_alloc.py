@@ -93,3 +93,18 @@ def test_noalloc_rejects_what_it_cannot_serve():
     with pytest.raises(Exception, match="too large for the allocation-free apply"):
         big.apply_batch_dev_noalloc(v, torch.empty_like(v))
     big.close()
+
+
+def test_noalloc_complex64_lengths_of_1024_points():
+    """complex64 rows of more than 512 points that are not powers of two: the
+    half-length passes pad their rows to a multiple of 8, the whole ones to a
+    multiple of 4, and a grid whose vector fits the array only with the latter
+    is taken (388x408x11), as is one that fits either way (312x340x7)."""
+    torch = _torch()
+    for Nx, Ny, Nz, nrhs in ((388, 408, 11, 1), (312, 340, 7, 2)):
+        print("noalloc", Nx, Ny, Nz, flush=True)
+        _, op = make_op(Nx, Ny, Nz, 9)
+        one = rand_rows(torch, 1, op.nvec, 8, torch.complex64)
+        op.apply_dev_f32(one[0], torch.empty_like(one[0]))
+        compare(torch, op, nrhs, torch.complex64, 6)
+        op.close()
