@@ -2269,14 +2269,16 @@ template <typename R> static int pass_vectors(const Operator& op, const OpBuffer
   return (int)std::max<size_t>(1, std::min<size_t>(k, BATCH_PASS_BYTES / one));
 }
 // Whether the k vectors can share launches: equal distances, and no output
-// over another vector's input (the vectors' passes keep their order then).
+// over another vector's input or output (the vectors' passes keep their order then).
 template <typename T2> static bool in_step(int k, const T2* const* vins, T2* const* vouts, int64_t nv) {
   for (int i = 0; i < k; i++) {
     if (i && ((const char*)vins[i] - (const char*)vins[0] != i * ((const char*)vins[1] - (const char*)vins[0]) ||
               (char*)vouts[i] - (char*)vouts[0] != i * ((char*)vouts[1] - (char*)vouts[0])))
       return false;
     for (int j = 0; j < k; j++)
-      if (i != j && vouts[i] < vins[j] + nv && vins[j] < vouts[i] + nv) return false;
+      if (i != j && ((vouts[i] < vins[j] + nv && vins[j] < vouts[i] + nv) ||
+                     (vouts[i] < vouts[j] + nv && vouts[j] < vouts[i] + nv)))
+        return false;
   }
   return k < 2 || (((const char*)vins[1] - (const char*)vins[0]) % (int64_t)sizeof(T2) == 0 &&
                    ((char*)vouts[1] - (char*)vouts[0]) % (int64_t)sizeof(T2) == 0);

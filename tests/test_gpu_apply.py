@@ -617,3 +617,28 @@ def test_fewest_layers(oracle, Nx, Ny, Nz):
     op.sync()
     assert rel(o32.cpu().numpy().astype(np.complex128), ref) < 2e-6
     op.close()
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+def test_pair_outputs_that_overlap(dt):
+    """Pairs whose vectors may not share launches of the passes: both products
+    to one output (the second stays), and the second to the first's input."""
+    torch = _torch()
+    from giem2g_amd import models, operator as gop
+    m = models.small(32, 30, 9, seed=4, freq=0.7, dz=25.0)
+    op = gop.operator_for(m)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    V = torch.complex(*torch.randn(2, 2, op.nvec, dtype=torch.float64, device="cuda", generator=g))
+    V = V.to(torch.complex128 if dt == "c128" else torch.complex64).contiguous()
+    ref, out = torch.empty_like(V), torch.empty_like(V[0])
+    op.apply_pair_dev(V[0], V[1], ref[0], ref[1])
+    for k in range(50):
+        op.apply_pair_dev(V[0], V[1], out, out)
+        op.sync()
+        assert torch.equal(torch.view_as_real(out), torch.view_as_real(ref[1])), k
+    W = V.clone()
+    op.apply_pair_dev(W[0], W[1], out, W[0])
+    op.sync()
+    assert torch.equal(torch.view_as_real(out), torch.view_as_real(ref[0]))
+    assert torch.equal(torch.view_as_real(W[0]), torch.view_as_real(ref[1]))
+    op.close()
