@@ -2284,6 +2284,11 @@ template <typename T2> static bool in_step(int k, const T2* const* vins, T2* con
                    ((char*)vouts[1] - (char*)vouts[0]) % (int64_t)sizeof(T2) == 0);
 }
 
+// vectors that one contraction takes.  FP64 takes at most four per tensor read:
+// an eight-vector FP64 kernel held 360 registers per lane (one wave per SIMD)
+// and measured 22% slower per vector than four at 128x128x32
+template <typename R> static int batch_cap(const Operator& op) { return std::min(op_batch_max(op), sizeof(R) == 8 ? 4 : 8); }
+
 // The slots of X for merged passes (and of S, where each vector has its own
 // contraction).  Made once, for the largest batch, so that a captured graph
 // keeps valid addresses; false when they cannot be made (stream under
@@ -2298,8 +2303,8 @@ template <typename R> static bool pass_slots(const Operator& op, OpBuffers<R>& b
     return false;
   }
   if (st != hipStreamCaptureStatusNone) return false;
-  const int m = pass_vectors(op, b, 8);
   const bool own = op_batch_max(op) == 1;
+  const int m = pass_vectors(op, b, own ? 8 : batch_cap<R>(op));
   const size_t nX = (size_t)b.nchunk * b.NR * op.Ny * 2 * op.Nx, nS = (size_t)12 * op.Nx * op.Ny * op.Nz;
   T2* p = nullptr;
   if (hipMalloc((void**)&p, sizeof(T2) * m * (nX + (own ? nS : 0))) != hipSuccess) {
@@ -2446,13 +2451,10 @@ void op_apply_batch(Operator& op, OpBuffers<R>& b, int nrhs, const cx_t<R>* vin,
   G2G_CHECK(op.have_tensor && op.have_sigma, -4, "operator not ready: tensor or conductivity missing");
   G2G_CHECK(nrhs >= 1, -3, "batched apply needs at least one vector");
   const int64_t nv = 3 * (int64_t)op.ncell();
-  // FP64 takes at most four per tensor read: an eight-vector FP64 kernel
-  // held 360 registers per lane (one wave per SIMD) and measured 22% slower
-  // per vector than four at 128x128x32
-  // (layer counts with no contraction of several vectors share the FFT passes
+  // layer counts with no contraction of several vectors share the FFT passes
   // where these take several; an output over another vector's input keeps
-  // the vectors one after the other)
-  int kmax = std::min(op_batch_max(op), sizeof(R) == 8 ? 4 : 8);
+  // the vectors one after the other
+  int kmax = batch_cap<R>(op);
   const bool apart = vin == vout || vout + nv * nrhs <= vin || vin + nv * nrhs <= vout;
   const bool passes = kmax == 1 && nrhs > 1 && apart && pass_vectors(op, b, 8) > 1 && pass_slots<R>(op, b, s);
   if (passes) kmax = b.xb_cap;
@@ -2511,7 +2513,7 @@ template <typename R> static size_t noalloc_x(const Operator& op, const OpBuffer
 }
 static size_t noalloc_s(const Operator& op) { return (size_t)12 * op.Nx * op.Ny * op.Nz; }
 template <typename R> static int noalloc_fit(const Operator& op, const OpBuffers<R>& b) {
-  const int kmax = std::min(op_batch_max(op), sizeof(R) == 8 ? 4 : 8);
+  const int kmax = batch_cap<R>(op);
   int k = 0;
   for (int kk : {1, 2, 4, 8})
     if (kk <= kmax && sizeof(cx_t<R>) * (noalloc_x(op, b) + noalloc_s(op) * kk) <= NOALLOC_SCRATCH_BYTES) k = kk;

@@ -642,3 +642,28 @@ def test_pair_outputs_that_overlap(dt):
     assert torch.equal(torch.view_as_real(out), torch.view_as_real(ref[0]))
     assert torch.equal(torch.view_as_real(W[0]), torch.view_as_real(ref[1]))
     op.close()
+
+
+@pytest.mark.parametrize("Nx,Ny,Nz,dt,most", [(16, 16, 33, "c128", 2), (16, 16, 50, "c64", 2), (16, 14, 9, "c128", 4),
+                                              (16, 14, 9, "c64", 8)])
+def test_batch_keeps_no_more_slots_than_it_uses(Nx, Ny, Nz, dt, most):
+    """What the first batch adds to the operator: at most a spectrum and an FFT
+    intermediate (3 Nz rows padded to a multiple of 8) for each of the vectors
+    that one tensor read serves."""
+    torch = _torch()
+    from giem2g_amd import models, operator as gop
+    m = models.small(Nx, Ny, Nz, seed=4, freq=0.7, dz=25.0)
+    op = gop.operator_for(m)
+    es, t = (16, torch.complex128) if dt == "c128" else (8, torch.complex64)
+    v = torch.ones((9, op.nvec), dtype=t, device="cuda")
+    out = torch.empty_like(v)
+    (op.apply_dev if dt == "c128" else op.apply_dev_f32)(v[0], out[0])
+    op.sync()
+    before = op.stats()["device_bytes"]
+    op.apply_batch_dev(v, out)
+    op.sync()
+    grown = op.stats()["device_bytes"] - before
+    one = es * (12 * Nx * Ny * Nz + 2 * Nx * Ny * ((3 * Nz + 7) // 8 * 8))
+    print("  grown %d, one vector %d" % (grown, one), flush=True)
+    assert grown <= most * one
+    op.close()
