@@ -648,45 +648,51 @@ __global__ void k_pool(const bf16* __restrict__ src, bf16* __restrict__ dst, int
 // element and two 64-bit divisions per thread, 240 us of a gradient at 8 x
 // 64x64x16, now 132.
 enum GradSource { GradPlain, GradUpsample, GradPool };
+// The grid's y axis takes the layers z, so the rows beyond its limit (GRID_Y_MAX,
+// long volumes) are a second turn of the loop.
+constexpr int GRID_Y_MAX = 65535;
 template <GradSource SRC>
 __global__ void k_relu_back(const float* __restrict__ dy, int ldy, const float* __restrict__ dc, const bf16* __restrict__ y,
-                            int C, int sh, float* __restrict__ dzf, bf16* __restrict__ dzb, int nx, int ny) {
+                            int C, int sh, float* __restrict__ dzf, bf16* __restrict__ dzb, int nx, int ny, int nz) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int xy = i >> sh, c = (i & ((1 << sh) - 1)) * 4, nz = gridDim.y, z = blockIdx.y;
+  const int xy = i >> sh, c = (i & ((1 << sh) - 1)) * 4;
   if (xy >= nx * ny) return;
-  const int64_t bat = blockIdx.z, p = (bat * nz + z) * nx * ny + xy;
-  f32x4 g;
-  if constexpr (SRC == GradUpsample) {
-    const int yy = xy / nx, x = xy - yy * nx;
-    g = f32x4{0, 0, 0, 0};
-#pragma unroll
-    for (int d = 0; d < 8; d++) {
-      const int X = 2 * x + (d & 1), Y = 2 * yy + ((d >> 1) & 1), Z = 2 * z + (d >> 2);
-      g += *reinterpret_cast<const f32x4*>(dy + (((bat * 2 * nz + Z) * 2 * ny + Y) * 2 * nx + X) * ldy + c);
-    }
-  } else {
-    g = *reinterpret_cast<const f32x4*>(dy + p * ldy + c);
-    if constexpr (SRC == GradPool) {
+  const int64_t bat = blockIdx.z;
+  for (int z = blockIdx.y; z < nz; z += gridDim.y) {
+    const int64_t p = (bat * nz + z) * nx * ny + xy;
+    f32x4 g;
+    if constexpr (SRC == GradUpsample) {
       const int yy = xy / nx, x = xy - yy * nx;
-      const int64_t q = ((bat * (nz / 2) + z / 2) * (ny / 2) + yy / 2) * (nx / 2) + x / 2;
-      g += 0.125f * *reinterpret_cast<const f32x4*>(dc + q * C + c);
+      g = f32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int d = 0; d < 8; d++) {
+        const int X = 2 * x + (d & 1), Y = 2 * yy + ((d >> 1) & 1), Z = 2 * z + (d >> 2);
+        g += *reinterpret_cast<const f32x4*>(dy + (((bat * 2 * nz + Z) * 2 * ny + Y) * 2 * nx + X) * ldy + c);
+      }
+    } else {
+      g = *reinterpret_cast<const f32x4*>(dy + p * ldy + c);
+      if constexpr (SRC == GradPool) {
+        const int yy = xy / nx, x = xy - yy * nx;
+        const int64_t q = ((bat * (nz / 2) + z / 2) * (ny / 2) + yy / 2) * (nx / 2) + x / 2;
+        g += 0.125f * *reinterpret_cast<const f32x4*>(dc + q * C + c);
+      }
     }
-  }
-  if (y) {
-    const bf16x4 v = *reinterpret_cast<const bf16x4*>(y + p * C + c);
+    if (y) {
+      const bf16x4 v = *reinterpret_cast<const bf16x4*>(y + p * C + c);
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-      if (!((float)v[k] > 0.f)) g[k] = 0.f;
-  }
-  bf16x4 o;
+      for (int k = 0; k < 4; k++)
+        if (!((float)v[k] > 0.f)) g[k] = 0.f;
+    }
+    bf16x4 o;
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    if (c + k >= C) g[k] = 0.f;
-    o[k] = (bf16)g[k];
+    for (int k = 0; k < 4; k++) {
+      if (c + k >= C) g[k] = 0.f;
+      o[k] = (bf16)g[k];
+    }
+    const int64_t at = (p << (sh + 2)) + c;
+    *reinterpret_cast<f32x4*>(dzf + at) = g;
+    *reinterpret_cast<bf16x4*>(dzb + at) = o;
   }
-  const int64_t at = (p << (sh + 2)) + c;
-  *reinterpret_cast<f32x4*>(dzf + at) = g;
-  *reinterpret_cast<bf16x4*>(dzb + at) = o;
 }
 
 // n voxels of 8 channels; VEC: a is 16-byte aligned
@@ -1212,8 +1218,8 @@ static void layer_back(UNet& n, int li, const float* dy, int ldy, const bf16* y,
   int sh = 0;
   while ((4 << sh) < l.coutT) sh++;
   G2G_CHECK((4 << sh) == l.coutT && (!l.relu || l.cout == l.coutT), -3, "layer widths are powers of two");
-  hipLaunchKernelGGL(k_relu_back<SRC>, dim3(nblk((int64_t)(nx * ny) << sh), nz, n.B), dim3(UB), 0, s, dy, ldy, dc,
-                     l.relu ? y : nullptr, l.cout, sh, n.dzf, n.dzb, nx, ny);
+  hipLaunchKernelGGL(k_relu_back<SRC>, dim3(nblk((int64_t)(nx * ny) << sh), std::min(nz, GRID_Y_MAX), n.B), dim3(UB), 0,
+                     s, dy, ldy, dc, l.relu ? y : nullptr, l.cout, sh, n.dzf, n.dzb, nx, ny, nz);
   conv_dw(n, li, n.dzf, l.coutT, s1, s2, nx, ny, nz, s);
   if (dx) conv_dx(n, li, n.dzb, nx, ny, nz, dx, s);
 }

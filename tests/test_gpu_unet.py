@@ -308,3 +308,31 @@ def test_infinite_activation_in_the_gradient(B, Z, Y, X, q):
     net.forward(x, keep=True)
     assert np.array_equal(net.backward(dy), g1) and np.isfinite(g1).all()
     net.close()
+
+
+def test_gradient_of_a_long_volume():
+    """More layers than a launch grid's y axis takes (65535).  The output
+    gradient is zero but for the last 8 layers.  It reaches fewer than 30 layers
+    back and the activations there 30 further, so every layer's gradient is
+    that of the last 96 layers alone.  Both are FP32 sums of the same products
+    (at most 16 x 50 nonzero ones) in another order: 800 x 2^-24."""
+    torch = _torch()
+    from giem2g_amd import learned
+    from oracle import unet_ref as U
+    Z, K = 65540, 96
+    rng = np.random.default_rng(4)
+    net = learned.UNet(params=_params(2))
+    x = torch.from_numpy(rng.standard_normal((1, Z, 4, 4, 8)).astype(np.float32)).cuda()
+    dy = torch.zeros((1, Z, 4, 4, 6), device="cuda")
+    dy[:, -8:] = torch.from_numpy(rng.standard_normal((1, 8, 4, 4, 6)).astype(np.float32)).cuda()
+    net.forward(x, keep=True)
+    g = net.backward(dy).astype(np.float64)
+    net.forward(x[:, -K:].contiguous(), keep=True)
+    ref = net.backward(dy[:, -K:].contiguous()).astype(np.float64)
+    off = 0
+    for li, (W, bb) in enumerate(U.split(ref)):
+        for r in (W.ravel(), bb):
+            e = rel(g[off:off + r.size], r)
+            assert e < 800 * 2.0 ** -24, (li, e)
+            off += r.size
+    net.close()
