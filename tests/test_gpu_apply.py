@@ -667,3 +667,82 @@ def test_batch_keeps_no_more_slots_than_it_uses(Nx, Ny, Nz, dt, most):
     print("  grown %d, one vector %d" % (grown, one), flush=True)
     assert grown <= most * one
     op.close()
+
+
+@pytest.mark.parametrize("Nx,Ny,Nz,dt,nrhs", [(128, 128, 32, "c64", 8), (96, 96, 70, "c64", 7), (96, 96, 70, "c128", 5),
+                                              (112, 96, 70, "c64", 9), (280, 276, 6, "c64", 9)])
+def test_batch_in_groups_of_passes(Nx, Ny, Nz, dt, nrhs):
+    """Grids of which fewer vectors fit one launch of the FFT passes than a
+    batch has (X and spectrum of one vector above an eighth of 512 MiB), with
+    and without a contraction of several vectors, ragged last groups and a last
+    group of one vector: every row against a one-vector apply (FP64 1e-14,
+    complex64 2e-6), in place with the same bits, and the allocation-free
+    apply, where it holds one, within the same bars."""
+    torch = _torch()
+    from giem2g_amd import lib as L, models, operator as gop
+    print("groups", Nx, Ny, Nz, dt, nrhs, flush=True)
+    es, t, tol = (16, torch.complex128, 1e-14) if dt == "c128" else (8, torch.complex64, 2e-6)
+    assert nrhs * es * (12 * Nx * Ny * Nz + 6 * Nx * Ny * Nz) > 512 << 20
+    m = models.small(Nx, Ny, Nz, seed=Nx + Nz, freq=0.7, dz=25.0)
+    op = gop.operator_for(m)
+    g = torch.Generator(device="cuda").manual_seed(Nx + nrhs)
+    vin = torch.complex(*torch.randn(2, nrhs, op.nvec, dtype=torch.float64, device="cuda", generator=g)).to(t).contiguous()
+    vout, one = torch.empty_like(vin), torch.empty_like(vin[0])
+    op.apply_batch_dev(vin, vout)
+    apply = op.apply_dev if dt == "c128" else op.apply_dev_f32
+
+    def diff(a):
+        return float((a - one).abs().pow(2).sum().sqrt() / one.abs().pow(2).sum().sqrt())
+    na = torch.empty_like(vin)
+    try:
+        op.apply_batch_dev_noalloc(vin, na)
+    except L.G2GError as e:
+        assert "too large" in str(e)
+        na = None
+    for r in range(nrhs):
+        apply(vin[r], one)
+        op.sync()
+        assert diff(vout[r]) < tol, r
+        assert na is None or diff(na[r]) < tol, r
+    op.apply_batch_dev(vin, vin)
+    op.sync()
+    assert torch.equal(torch.view_as_real(vin), torch.view_as_real(vout))
+    op.close()
+
+
+@pytest.mark.parametrize("Nx,Ny,Nz", [(16, 14, 6), (10, 16, 66), (16, 14, 9), (14, 16, 40)])
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+def test_batch_outputs_over_inputs(Nx, Ny, Nz, dt):
+    """Batches whose outputs lie over other vectors' inputs do not share
+    launches of the passes.  Each output over the input before it: the rows of
+    an apply to another place, bit for bit.  Each output over the input after
+    it, where a contraction takes one vector (below 8 and above 64 layers): the
+    products of products, one after the other."""
+    torch = _torch()
+    from giem2g_amd import models, operator as gop
+    print("over", Nx, Ny, Nz, dt, flush=True)
+    n = 5
+    m = models.small(Nx, Ny, Nz, seed=Nx + Nz, freq=0.7, dz=25.0)
+    op = gop.operator_for(m)
+    t = torch.complex128 if dt == "c128" else torch.complex64
+    g = torch.Generator(device="cuda").manual_seed(Nz)
+    V = torch.complex(*torch.randn(2, n, op.nvec, dtype=torch.float64, device="cuda", generator=g)).to(t).contiguous()
+    ref = torch.empty_like(V)
+    op.apply_batch_dev(V, ref)
+    buf = torch.empty((n + 1, op.nvec), dtype=t, device="cuda")
+    buf[1:] = V
+    op.apply_batch_dev(buf[1:], buf[:n])
+    op.sync()
+    assert torch.equal(torch.view_as_real(buf[:n]), torch.view_as_real(ref))
+    if Nz < 8 or Nz > 64:
+        apply = op.apply_dev if dt == "c128" else op.apply_dev_f32
+        buf[:n] = V
+        op.apply_batch_dev(buf[:n], buf[1:])
+        ref[0] = V[0]
+        out = torch.empty_like(V[0])
+        for r in range(n):
+            apply(ref[0], out)
+            op.sync()
+            assert torch.equal(torch.view_as_real(buf[r + 1]), torch.view_as_real(out)), r
+            ref[0] = out
+    op.close()
