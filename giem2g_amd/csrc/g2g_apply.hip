@@ -501,7 +501,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, 
 template <typename R, int L, bool RT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rt_waves<R, L, RT>()))) void k_inv_x_h(const cx_t<R>* __restrict__ X,
                                                 const cx_t<R>* __restrict__ vin,
-                                              const cx_t<R>* __restrict__ asiga,
+                                                const cx_t<R>* __restrict__ asiga,
                                                 const R* __restrict__ sq,
                                                 const R* __restrict__ dzn,
                                                 cx_t<R>* __restrict__ vout,

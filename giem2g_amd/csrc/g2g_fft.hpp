@@ -235,12 +235,13 @@ constexpr int prime_tiles(int tot, int lc, int waves) {
 // + x_{R-q} and differences d_q (q = 1 .. H = (R-1)/2, after the twiddles) take
 // the inputs' places in LDS; then [cos 2 pi qk/R] t and [sin] d for k = 0 .. H are
 // real matrix products with eight butterflies (16 real columns) per tile, and
-// the outputs k and R - k are their sum and difference.  H^2 products per
-// butterfly where a sum over all inputs for every output takes 4 R^2 (both
-// directions at 148x172x27, primes 37 and 43: FP64 706 -> 360 us, complex64 880
-// -> 289 us; eight vectors at 194x194x19, prime 97: 13.8 -> 5.9 ms a batch).  (The rows
-// in batches of four tiles per wave, for fewer registers, made the complex64
-// passes 1.4-2.4 times as long.)
+// the outputs k and R - k are their sum and difference.  4 H (H + 1), about R^2,
+// real products per butterfly (with k padded to tiles of 16 rows) where a sum
+// over all inputs for every output takes 4 R^2 (both directions at 148x172x27,
+// primes 37 and 43: FP64 706 -> 360 us, complex64 880 -> 289 us; eight vectors
+// at 194x194x19, prime 97: 13.8 -> 5.9 ms a batch).  (The rows in batches of
+// four tiles per wave, for fewer registers, made the complex64 passes 1.4-2.4
+// times as long.)
 template <typename T2, int LC, int NR, int NT, int DIR>
 __device__ inline void stockham_stage_prime(T2* buf, const T2* tw, int L, int LS, int R, int Ns) {
   using RR = decltype(T2::x);

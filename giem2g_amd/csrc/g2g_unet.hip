@@ -67,28 +67,18 @@ struct ConvArgs {
   int cout2;
 };
 
-// bias, ReLU and store of four consecutive output channels of one voxel
+// bias, ReLU and store of four consecutive output channels of one voxel (all
+// outputs stored here have a multiple of four channels, conv_launch)
 __device__ inline void conv_store(const ConvArgs& a, f32x4 c, int co0, int64_t p, int bat) {
   if (co0 >= a.cout) return;
-  float o[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    o[q] = c[q] + ((a.bias && co0 + q < a.cout) ? a.bias[co0 + q] : 0.f);
-    if (a.relu) o[q] = fmaxf(o[q], 0.f);
+    if (a.bias) c[q] += a.bias[co0 + q];
+    if (a.relu) c[q] = fmaxf(c[q], 0.f);
   }
-  if (a.ybf) {
-    const bf16x4 b = {(bf16)o[0], (bf16)o[1], (bf16)o[2], (bf16)o[3]};
-    *reinterpret_cast<bf16x4*>(a.ybf + bat * a.ybstride + p * a.ldy + co0) = b;
-  } else {
-    float* y = a.yf + bat * a.ybstride + p * a.ldy + co0;
-    if ((a.ldy & 3) == 0 && co0 + 3 < a.cout) {
-      *reinterpret_cast<f32x4*>(y) = f32x4{o[0], o[1], o[2], o[3]};
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (co0 + q < a.cout) y[q] = o[q];
-    }
-  }
+  const int64_t at = bat * a.ybstride + p * a.ldy + co0;
+  if (a.ybf) *reinterpret_cast<bf16x4*>(a.ybf + at) = bf16x4{(bf16)c[0], (bf16)c[1], (bf16)c[2], (bf16)c[3]};
+  else *reinterpret_cast<f32x4*>(a.yf + at) = c;
 }
 
 // A convolution tile of (1 << lx, 1 << ly, 1 << lz) voxels: tile counts, the
@@ -129,31 +119,6 @@ __global__ __launch_bounds__(UB) void k_conv1x1(ConvArgs a) {
   }
 }
 
-// 3x3x3 convolution, CIN input channels, CT x 16 output channels, a tile of
-// 64 G voxels (4 waves of 16 G voxels x all output channels).
-// The tile with its one-voxel rim is copied to LDS once, zero outside the
-// volume, concatenated and upsampled on the way, in planes of 8 channels
-// ([chunk][voxel], 16 bytes each): the 16 lanes of a matrix column then read
-// 16 neighbouring voxels without bank conflicts, and a tap is an offset added
-// to the lane's own voxel (a 4-byte table entry per k-step and lane quarter)
-// instead of the three bounds checks, the address and the global gather that
-// each fragment took when every wave read its input from memory: that kernel
-// ran at 0.10-0.17 of the matrix rate with the vector unit busy on addresses.
-// Every fragment read from LDS feeds the CT output tiles.  LDS bandwidth
-// bounds it (16 bytes a lane per CT products).  Measured at 256x256x32, all
-// layers of one forward pass: 1508 -> 555 us (251 GFLOP, 0.17 -> 0.45
-// PFLOP/s; 48 -> 16 channels 0.60 PFLOP/s); the whole pass 1541 -> 595 us
-// with the input conversion and the 1x1 output layer done on the way.  The sums run over k in the same order and instruction
-// as before, so the results are the same bit for bit.
-// Weights: fragment order [co tile][k-step][lane][8], one contiguous 1 KB
-// load per k-step and tile.
-constexpr int conv_g(int cin) { return cin >= 64 ? 2 : 4; }
-
-// An upsampled source (its first UPC channels) is kept in LDS at half
-// resolution: a quarter to an eighth of the bytes, so that three to five
-// blocks share a CU instead of one or two (48 channels 270 -> 143 us, 96
-// channels 173 -> 81 us).  Its offset of a tap depends on
-// the parity of the voxel's coordinates (eight table entries per k-step).
 // FP32 input rounded to bf16 on the way
 __device__ inline bf16x8 to_bf16x8(const float* x) {
   const f32x4 a = *reinterpret_cast<const f32x4*>(x), b = *reinterpret_cast<const f32x4*>(x + 4);
@@ -182,6 +147,32 @@ __device__ inline void conv_stage(bf16x8* xs, const ConvBox& b, const T* x, int 
   }
 }
 
+constexpr int conv_g(int cin) { return cin >= 64 ? 2 : 4; }
+
+// 3x3x3 convolution, CIN input channels, CT x 16 output channels, a tile of
+// 64 G voxels (4 waves of 16 G voxels x all output channels).
+// The tile with its one-voxel rim is copied to LDS once, zero outside the
+// volume, concatenated and upsampled on the way, in planes of 8 channels
+// ([chunk][voxel], 16 bytes each): the 16 lanes of a matrix column then read
+// 16 neighbouring voxels without bank conflicts, and a tap is an offset added
+// to the lane's own voxel (a 4-byte table entry per k-step and lane quarter)
+// instead of the three bounds checks, the address and the global gather that
+// each fragment took when every wave read its input from memory: that kernel
+// ran at 0.10-0.17 of the matrix rate with the vector unit busy on addresses.
+// Every fragment read from LDS feeds the CT output tiles.  LDS bandwidth
+// bounds it (16 bytes a lane per CT products).  Measured at 256x256x32, all
+// layers of one forward pass: 1508 -> 555 us (251 GFLOP, 0.17 -> 0.45
+// PFLOP/s; 48 -> 16 channels 0.60 PFLOP/s); the whole pass 1541 -> 595 us
+// with the input conversion and the 1x1 output layer done on the way.  The
+// sums run over k in the same order and instruction as before, so the results
+// are the same bit for bit.
+// Weights: fragment order [co tile][k-step][lane][8], one contiguous 1 KB
+// load per k-step and tile.
+// An upsampled source (its first UPC channels) is kept in LDS at half
+// resolution: a quarter to an eighth of the bytes, so that three to five
+// blocks share a CU instead of one or two (48 channels 270 -> 143 us, 96
+// channels 173 -> 81 us).  Its offset of a tap depends on the parity of the
+// voxel's coordinates (eight table entries per k-step).
 template <int CIN, int CT, int UPC>
 __global__ __launch_bounds__(UB) void k_conv3(ConvArgs a, ConvTile t) {
   constexpr int G = conv_g(CIN), NKS = (27 * CIN + 31) / 32, NU = UPC / 8, NF = CIN / 8 - NU;
@@ -1056,6 +1047,7 @@ template <int CIN, int CT, int UPC> static void conv3_go(const ConvArgs& a, int 
 
 // the network's widths (forward, and the data gradient's transposed ones)
 static void conv_launch(const ConvArgs& a, int coutP, int B, hipStream_t s) {
+  G2G_CHECK(a.cout % 4 == 0 && a.ldy % 4 == 0, -1, "convolution outputs of a multiple of four channels");
   const int64_t nvox = (int64_t)a.nx * a.ny * a.nz;
   if (a.ntap == 1) {
     G2G_CHECK(a.kp == 32 && a.s2.C == 0 && a.s1.up == 0, -1, "1x1 convolution of more than 32 channels");
