@@ -71,14 +71,18 @@ struct ConvArgs {
 // outputs stored here have a multiple of four channels, conv_launch)
 __device__ inline void conv_store(const ConvArgs& a, f32x4 c, int co0, int64_t p, int bat) {
   if (co0 >= a.cout) return;
+  float o[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    if (a.bias) c[q] += a.bias[co0 + q];
-    if (a.relu) c[q] = fmaxf(c[q], 0.f);
+    o[q] = c[q] + ((a.bias && co0 + q < a.cout) ? a.bias[co0 + q] : 0.f);
+    if (a.relu) o[q] = fmaxf(o[q], 0.f);
   }
-  const int64_t at = bat * a.ybstride + p * a.ldy + co0;
-  if (a.ybf) *reinterpret_cast<bf16x4*>(a.ybf + at) = bf16x4{(bf16)c[0], (bf16)c[1], (bf16)c[2], (bf16)c[3]};
-  else *reinterpret_cast<f32x4*>(a.yf + at) = c;
+  if (a.ybf) {
+    const bf16x4 b = {(bf16)o[0], (bf16)o[1], (bf16)o[2], (bf16)o[3]};
+    *reinterpret_cast<bf16x4*>(a.ybf + bat * a.ybstride + p * a.ldy + co0) = b;
+  } else {
+    *reinterpret_cast<f32x4*>(a.yf + bat * a.ybstride + p * a.ldy + co0) = f32x4{o[0], o[1], o[2], o[3]};
+  }
 }
 
 // A convolution tile of (1 << lx, 1 << ly, 1 << lz) voxels: tile counts, the
