@@ -511,9 +511,10 @@ __global__ __launch_bounds__(64) void k_lambda(zd* __restrict__ tabs,
 // C[o][coff + e] = scale * sum_seg sum_K A_seg[K][o] * B_seg[K][e] for every
 // offset o and entry e (A real weights, B complex tables): FP64 matrix
 // products (offsets x taps) (taps x 2 entries) on v_mfma_f64_16x16x4, all
-// jobs (tensor components) of a build in one launch.  Bound by the FP64
-// matrix rate.  Three things keep it below the (offsets x 501 x entries) of
-// the plain sum:
+// jobs (tensor components) of a build in one launch.  A large FP64 product
+// reaches 71 TFLOP/s on this card; the tiles here, with a barrier per 8 taps,
+// 42 to 59.  Three things keep the work below the (offsets x 501 x entries)
+// of the plain sum:
 //   - the taps: a block sums the window in which one of its offsets has a
 //     weight (the 1e-12 mask of the weights leaves 210 to 370 of 501 taps);
 //   - the x-y mirror (TRI): on a square grid with dx = dy the block at
@@ -523,8 +524,9 @@ __global__ __launch_bounds__(64) void k_lambda(zd* __restrict__ tabs,
 //     chunks of 8 taps, so that the loads of a chunk run beside the matrix
 //     products of the one before.
 // Measured (128x128x32): six launches on the vector unit, every tap and offset,
-// 4830 us (35 TFLOP/s) -> 980 us (46 TFLOP/s of the sums that are left); with
-// two receivers, thirty launches 5930 us (27 TFLOP/s) -> 1400 us (59 TFLOP/s).
+// 4830 us (35 TFLOP/s) -> 980 to 1080 us (46 to 42 TFLOP/s of the sums that are
+// left); with two receivers, thirty launches 5930 us (27 TFLOP/s) -> 1400 us
+// (59 TFLOP/s).
 struct WJob {
   int coff, coff2, Ne, nseg;  // coff or coff2 < 0: not stored there
   const double *A0, *A1;  // [K][lda]
@@ -678,8 +680,8 @@ template <int L> constexpr int ne_for() { return L <= 64 ? 32 : (L <= 128 ? 16 :
 // MIR (the half tensor of op_build_tensor): yy and yz are xx and xz with the
 // axes exchanged, so only xx, xy, zz and xz are read and transformed, and the
 // second pass stores xx and xz of (kx,ky) also as yy and yz of (ky,kx): 0.72
-// of the bytes.  HBM bound (128x128x32: 1180 -> 790 us for the two passes,
-// 4.0 TB/s).
+// of the bytes.  HBM bound (128x128x32: 1180 -> 790 to 830 us for the two passes,
+// 4.0 to 3.8 TB/s).
 template <int L, int AXIS, bool RT, bool MIR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT ? 2 : 1))) void k_tfft(zd* __restrict__ G, const zd* __restrict__ twg,
                                               int Nx, int Ny, int Nz, int64_t BS, FftPlan plan) {

@@ -165,8 +165,8 @@ constexpr int conv_g(int cin) { return cin >= 64 ? 2 : 4; }
 // ran at 0.10-0.17 of the matrix rate with the vector unit busy on addresses.
 // Every fragment read from LDS feeds the CT output tiles.  LDS bandwidth
 // bounds it (16 bytes a lane per CT products).  Measured at 256x256x32, all
-// layers of one forward pass: 1508 -> 555 us (251 GFLOP, 0.17 -> 0.45
-// PFLOP/s; 48 -> 16 channels 0.60 PFLOP/s); the whole pass 1541 -> 595 us
+// layers of one forward pass: 1508 -> 585 us (251 GFLOP, 0.17 -> 0.43
+// PFLOP/s; 48 -> 16 channels 0.60 PFLOP/s); the whole pass 1541 -> 597 us
 // with the input conversion and the 1x1 output layer done on the way.  The
 // sums run over k in the same order and instruction as before, so the results
 // are the same bit for bit.
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(UB) void k_conv3(ConvArgs a, ConvTile t) {
 // their way to LDS).  Strides of an odd number of 16-byte units spread the 16 channels of a
 // read over the banks.  The transposition and the LDS reads bound it (matrix
 // cores about a fifth busy).  Measured at 8 x 64x64x16, all layers: 7910 us on
-// the FP32 vector unit with atomics -> 560 us; error of the sums against FP64
+// the FP32 vector unit with atomics -> 520 us; error of the sums against FP64
 // 4.4e-7 -> 0.6e-7.
 struct DwArgs {
   const float* dz;

@@ -171,8 +171,15 @@ int giem2g_op_apply_pair_dev(void *ie_op, int precision, const void *in0_dev, co
  * read serves up to 8 complex64 or 4 complex128 vectors at Nz 8 to 32 and
  * 2 at Nz 33 to 64 (the matrix-core contraction with one 16-column operand
  * per two vectors; a layer count that is not a multiple of 16 is padded with
- * zero layers inside the kernel); Nz below 8 applies the vectors one by one.  No reference counterpart (the
- * reference applies the operator to one vector at a time). */
+ * zero layers inside the kernel); below 8 and above 64 layers every vector
+ * reads the tensor.  Vectors also share launches of the FFT passes where their
+ * FFT intermediates and spectra fit in 512 MiB; the first batch or pair makes
+ * the memory for that (at most 512 MiB for each precision), which the operator
+ * keeps until it is destroyed.  When it cannot be had (device memory full, a
+ * stream under capture) the passes take the vectors one by one.  An output may
+ * be its own input; one that lies over another vector's input makes the passes
+ * take the vectors one after the other, in order.  No reference counterpart
+ * (the reference applies the operator to one vector at a time). */
 int giem2g_op_apply_batch_dev(void *ie_op, int precision, int nrhs, const void *in_dev, void *out_dev);
 /* Allocation-free variant of giem2g_op_apply_batch_dev, with the same
  * arguments and products.  No counterpart in the reference: it is for callers
